@@ -308,9 +308,8 @@ def stack_result(args, ctx):
                                "addresses and values, 604 MB walked per token at 36 layers), one HIP graph per token, %s layout, %s"
                                % (layers, n_q, ctx, layers, "head-major" if args.layout == 1 else "position-major",
                                   "one launch per layer" if args.stack_mode == 2 else
-                                  "ONE resident launch for all layers (llmi_hip_mha_decode_append_stack): the next layer's K/V tiles "
-                                  "stream while this layer's results are merged, and a layer reads its query / K row / V row only after "
-                                  "every head of the layer before has published its output" if args.stack_mode == 5 else
+                                  "ONE resident launch for all layers (llmi_hip_mha_decode_append_stack); every layer has buffers of its own "
+                                  "here, so no layer's inputs depend on another layer's output and the layers run as one stream" if args.stack_mode == 5 else
                                   "three launches per layer: packed QKV GEMV (hidden %d), attention, output projection + "
                                   "residual" % hidden if args.stack_mode == 3 else
                                   "two launches per layer: packed QKV GEMV (hidden %d), attention whose idle workgroups do the "
@@ -545,7 +544,8 @@ def run_calibrate_hbm(args):
 
 
 def run_stack_timeline(args, ctx):
-    """Where a layer's time goes inside the resident launch (llmi_hip_mha_decode_append_stack): needs a build of the
+    """Where a layer's time goes inside the resident launch of layers that depend on each other
+    (llmi_hip_mha_decode_append_stack): needs a build of the
     library with the phase stamps compiled in,
 
         python -m llminfer_amd.build --define LLMI_STACK_STAMPS=1 --only mha_stack.hip --output /tmp/libllmi_stamps.so
@@ -570,9 +570,11 @@ def run_stack_timeline(args, ctx):
         return x.to(torch.bfloat16)
 
     k, v = rnd(L * N_KV * msl, D).reshape(-1), rnd(L * N_KV * msl, D).reshape(-1)
-    q, kn, vn = rnd(L * n_q, D, norm=False).reshape(-1), rnd(L * N_KV, D, norm=False).reshape(-1), rnd(L * N_KV, D, norm=False).reshape(-1)
+    # (a chain: every layer's query is the output of the layer before, so the launch has to honour the order between them)
+    rows = rnd((L + 1) * n_q, D, norm=False).reshape(-1)
+    q, out = rows, rows[dim:]
+    kn, vn = rnd(L * N_KV, D, norm=False).reshape(-1), rnd(L * N_KV, D, norm=False).reshape(-1)
     w = (1 + 0.02 * torch.randn(L * 2 * D, generator=gen, device=dev)).to(torch.bfloat16)
-    out = torch.zeros(L * dim, dtype=torch.bfloat16, device=dev)
     sin_d, cos_d = ops.sincos_table(D, msl, dev)
     ws = torch.zeros(max(ops.workspace_bytes(n_q, D, msl), 6 << 20) // 4, dtype=torch.float32, device=dev)
     side = ops.workspace_side(ws)

@@ -232,7 +232,11 @@ typedef struct llmi_mha_stack_args {
  * needs: the fused split path with 2..64 splits and a host-side position, a query group of at most 4 heads, a grid no
  * larger than the device's compute unit count, and a workspace sized by llmi_hip_mha_workspace_bytes (the plan's need
  * plus 4.3 KiB for the tags). Anything else runs as layer_count launches of llmi_hip_mha_decode_append.
- * llmi_hip_mha_stack_launches tells which: 1 or layer_count (or a negative status for invalid arguments). */
+ * llmi_hip_mha_stack_launches tells which: 1 or layer_count (or a negative status for invalid arguments).
+ * In the one-launch form, layers that cannot see each other's writes do not wait for each other: if no address range that
+ * the call writes (outputs, tap, the layers' caches, workspace; each from the first layer's first byte to the last layer's last
+ * one) overlaps one it reads or another one it writes, and every layer has output rows of its own, the layers run as one
+ * stream (same bits, less than half the time). The order described above holds wherever it can be observed. */
 int llmi_hip_mha_decode_append_stack(const llmi_mha_stack_args* args);
 int llmi_hip_mha_stack_launches(const llmi_mha_stack_args* args);
 

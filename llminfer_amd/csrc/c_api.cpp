@@ -482,6 +482,43 @@ int llmi_hip_mha_decode_append_oproj(const llmi_attn_oproj_args* args) {
                        static_cast<hipStream_t>(m.stream));
 }
 
+// Whether the layers of a call can be told apart in time: true unless something one of them reads or writes overlaps
+// something another one writes (outputs, the tap, the caches' layers, the workspace). Judged by address ranges, each buffer
+// from its first layer's first byte to its last layer's last one, so interleaved buffers count as overlapping.
+static bool layers_are_independent(const llmi_mha_stack_args& st) {
+    struct Range {
+        uintptr_t lo, hi;
+    };
+    const llmi_mha_append_args& ap = st.first;
+    const llmi_mha_args& m = ap.mha;
+    const int64_t L = st.layer_count, dim = (int64_t)m.head_num * m.head_dim;
+    auto range = [&](const void* base, int64_t stride, int64_t elems, int64_t size) {
+        const int64_t last = (L - 1) * stride;
+        const uintptr_t b = reinterpret_cast<uintptr_t>(base);
+        return Range{b + (uintptr_t)((last < 0 ? last : 0) * size), b + (uintptr_t)(((last > 0 ? last : 0) + elems) * size)};
+    };
+    const int64_t layer_elems = (int64_t)m.max_seq_len * m.kv_dim;
+    const uint16_t* k = static_cast<const uint16_t*>(m.key_cache) + (int64_t)m.layer_id * layer_elems;
+    const uint16_t* v = static_cast<const uint16_t*>(m.value_cache) + (int64_t)m.layer_id * layer_elems;
+    const Range writes[] = {range(m.output, st.output_stride, dim, 2), range(k, layer_elems, layer_elems, 2),
+                            range(v, layer_elems, layer_elems, 2),
+                            {reinterpret_cast<uintptr_t>(m.workspace), reinterpret_cast<uintptr_t>(m.workspace) + m.workspace_bytes},
+                            m.output_f32 ? range(m.output_f32, st.output_stride, dim, 4) : Range{0, 0}};
+    const int64_t table = (int64_t)(m.pos + 1) * (m.head_dim / 2);
+    const Range reads[] = {range(m.query, st.query_stride, dim, 2), range(ap.key_new, st.key_new_stride, m.kv_dim, 2),
+                           range(ap.value_new, st.value_new_stride, m.kv_dim, 2),
+                           range(ap.norm_weight, st.norm_weight_stride, 2 * m.head_dim, 2), range(ap.sin_cache, 0, table, 4),
+                           range(ap.cos_cache, 0, table, 4)};
+    auto apart = [](const Range& a, const Range& b) { return a.hi <= b.lo || b.hi <= a.lo; };
+    for (const Range& w : writes)
+        for (const Range& r : reads)
+            if (!apart(w, r)) return false;
+    for (const Range& w : writes)
+        for (const Range& x : writes)
+            if (&w != &x && !apart(w, x)) return false;
+    return L == 1 || st.output_stride >= dim || st.output_stride <= -dim;  // (each layer writes rows of its own)
+}
+
 // Validates a multi-layer call and decides between the one-launch form (*one_launch = true, plan = layer 0's) and
 // one launch per layer.
 static int plan_stack(const llmi_mha_stack_args* args, llmi_mha_plan* plan, bool* one_launch) {
@@ -526,7 +563,7 @@ int llmi_hip_mha_decode_append_stack(const llmi_mha_stack_args* args) {
     llmi_mha_plan plan;
     bool one = false;
     if (int rc = plan_stack(args, &plan, &one)) return rc;
-    if (one) return launch_mha_stack(*args, plan);
+    if (one) return launch_mha_stack(*args, plan, layers_are_independent(*args));
     for (int32_t l = 0; l < args->layer_count; ++l) {
         llmi_mha_append_args a = args->first;
         a.mha.layer_id += l;

@@ -222,12 +222,29 @@ static int fill_kernel_args(const llmi_mha_args& args, const llmi_mha_plan& plan
 
 size_t stack_workspace_extra(int head_num) { return 256 + stack_done_bytes(head_num); }
 
-int launch_mha_stack(const llmi_mha_stack_args& st, const llmi_mha_plan& plan) {
+int launch_mha_stack(const llmi_mha_stack_args& st, const llmi_mha_plan& plan_in, bool independent) {
     const llmi_mha_args& m = st.first.mha;
+    llmi_mha_plan plan = plan_in;
     StackArgs sa{};
+    if (independent && st.layer_count > 1) {
+        // As many layers' partial rows and records in the workspace as fit: a layer is merged two layers and more behind the
+        // stream. (Plain layout: what by-side saves is latency, which is hidden.) A workspace sized by
+        // llmi_hip_mha_workspace_bytes has room for twice the splits of the longest context, by side: for three regions at least.
+        const size_t region = (fused_workspace(m.head_num, m.head_dim, plan.num_splits, false).bytes() + 255) & ~(size_t)255;
+        const size_t tags = stack_workspace_extra(m.head_num);
+        size_t fit = m.workspace_bytes > tags ? (m.workspace_bytes - tags) / region : 0;
+        if (fit > (size_t)stack_max_regions(m.head_num)) fit = stack_max_regions(m.head_num);
+        if (fit > (size_t)st.layer_count) fit = st.layer_count;
+        if (fit >= 3 && plan.num_splits >= m.kv_mul) {  // (a workgroup merges at most one head per layer)
+            plan.workspace_side = 0;
+            sa.regions = (int32_t)fit;
+            sa.region_bytes = (int64_t)region;
+        }
+    }
     char* fused_end = nullptr;
     if (int rc = fill_kernel_args(m, plan, &st.first, nullptr, st.layer_count, &sa.a, &fused_end)) return rc;
     if (!fused_end) return LLMI_ERR_INVALID_ARG;  // (the caller has checked: fused split path)
+    if (sa.regions > 0) fused_end = static_cast<char*>(m.workspace) + sa.regions * sa.region_bytes;
     sa.layers = st.layer_count;
     sa.q_stride = st.query_stride;
     sa.knew_stride = st.key_new_stride;

@@ -62,10 +62,17 @@ struct StackArgs {
     int64_t q_stride, knew_stride, vnew_stride, normw_stride, out_stride;  // elements between consecutive layers
     int64_t cache_stride;  // elements between consecutive layers' K (and V) caches
     uint32_t* done;        // in the workspace: the heads' "done" tags, stack_done_bytes() bytes
+    // > 0: the layers do not depend on each other (mha_layers_kernel). Layer l keeps its partial rows and, behind them, its
+    // records in region l % regions of the workspace, region_bytes apart from a.ws on; done[region * 64 + head] then says
+    // which layer of the region has been merged.
+    int32_t regions;
+    int64_t region_bytes;
 };
 // Groups of 1, 2 or 4 query heads (padded), four wavefronts per workgroup; false otherwise.
 bool launch_stack(const StackArgs& sa, int n_kv, int group_pad, int waves, hipStream_t stream);
 size_t stack_done_bytes(int head_num);
+// Most regions the done tags have room for (0: none for this many heads).
+int stack_max_regions(int head_num);
 hipError_t poll_timeouts_stack(unsigned int* n);
 
 // Launchers of the kernels instantiated for a (padded) group of G query heads per KV head; each lives in its own

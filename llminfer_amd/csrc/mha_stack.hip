@@ -19,6 +19,10 @@
 //   * within a layer everything is the split kernel's: online softmax over 16-position tiles on the matrix cores,
 //     the merge of a workgroup's wavefronts through LDS, partial results and arrival records handed to the
 //     workgroup of the head's last split, which merges them (log-sum-exp) and writes the bf16 output.
+// That chain (mha_stack_kernel) costs 6.8 us per layer, six dependent trips through memory, with HBM idle two thirds of the
+// time. It is needed only where a layer can see another layer's writes. Where the caller's buffers say that none can (no
+// layer's inputs overlap anything a layer writes, see layers_are_independent in c_api.cpp), the layers may run in any order
+// and mha_layers_kernel below runs them as one stream with nothing between a layer and the next.
 // Every wait is bounded (llmi_hip_set_poll_limit): a wait that gives up is counted and poisons the outputs of its
 // layer and the following ones with NaN instead of hanging the device; every wavefront reaches the end of the kernel.
 // Needs every workgroup of the grid resident at once (the host checks the grid against the compute unit count).
@@ -80,6 +84,84 @@ namespace {
 constexpr int kDoneCopies = LLMI_STACK_DONE_COPIES;
 static_assert(kDoneCopies >= 1 && kDoneCopies <= 64, "one lane of the merging wavefront writes each copy");
 constexpr int kDoneLineWords = 64;  // 256 bytes: room for 64 heads' tags per copy (128 heads: two lines per copy)
+
+// One tile of 16 positions into a wavefront's running softmax: q.K^T, online softmax, P^T.V on the matrix cores (the
+// probabilities as hi + lo bf16), for groups of at most four query heads. row0: the lane's first position in the split.
+__device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4], int row0, int nrows, float scale_log2e,
+                                          float& m_run, float& l_run, f32x4 (&o)[8]) {
+    f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, r.k[j]), __builtin_bit_cast(bf16x8, qb[j]), c, 0, 0, 0);
+    float s[4];
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        s[e] = (row0 + e < nrows) ? c[e] * scale_log2e : -INFINITY;
+        tmax = fmaxf(tmax, s[e]);
+    }
+    tmax = rows_max(tmax);
+    const float m_new = fmaxf(m_run, tmax);
+    const float alpha = fast_exp2(m_run - m_new);
+    float p[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = fast_exp2(s[e] - m_new);
+    l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+    m_run = m_new;
+    const uint32_t p01 = pack_bf16(p[0], p[1]);
+    const uint32_t p23 = pack_bf16(p[2], p[3]);
+    const uint32_t q01 = pack_bf16(p[0] - bf16_lo(p01), p[1] - bf16_hi(p01));
+    const uint32_t q23 = pack_bf16(p[2] - bf16_lo(p23), p[3] - bf16_hi(p23));
+    if (__any(alpha != 1.0f)) {
+        static_for<0, 4>([&](auto rr) {
+            const float ar = row_bcast<rr.value>(alpha);  // (G <= 4: only DPP row 0 holds heads)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o[j][rr.value] *= ar;
+        });
+    }
+    const i16x4 pa = __builtin_bit_cast(i16x4, u32x2{p01, p23});
+    const i16x4 pb = __builtin_bit_cast(i16x4, u32x2{q01, q23});
+    i16x4 vb4[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+        const uint32_t b01 = __builtin_amdgcn_perm(r.v[1][j >> 1], r.v[0][j >> 1], sel);
+        const uint32_t b23 = __builtin_amdgcn_perm(r.v[3][j >> 1], r.v[2][j >> 1], sel);
+        vb4[j] = __builtin_bit_cast(i16x4, u32x2{b01, b23});
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, vb4[j], o[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pb, vb4[j], o[j], 0, 0, 0);
+}
+
+// A wavefront's running softmax of the new token alone: score q.k, weight 1, output = the V row. new_rows: its K row
+// (normalised and rotated, operand layout) and V row in LDS, 16-byte chunks.
+__device__ __forceinline__ void start_from_new_row(const u32x4* new_rows, const u32x4 (&qb)[4], int kg, int n16, float scale_log2e,
+                                                   u32x4 (&kf)[4], u32x4& vf, float& m_run, float& l_run, f32x4 (&o)[8]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kf[j] = new_rows[j * 4 + kg];
+    vf = new_rows[16 + n16];
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t qw = qb[j][c], kw = kf[j][c];  // (bit_cast straight from a vector element reads element 0)
+            dot = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, qw), __builtin_bit_cast(bf16x2, kw), dot, false);
+        }
+    dot = rows_sum(dot);
+    m_run = dot * scale_log2e;
+    l_run = kg == 0 ? 1.0f : 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t vw = vf[j >> 1];
+        const float vj = (j & 1) ? bf16_hi(vw) : bf16_lo(vw);
+        o[j] = f32x4{vj, vj, vj, vj};
+    }
+}
+
 
 template <int G, int NW, int NSTAGE, bool BYSIDE>
 __global__ __launch_bounds__(NW * 64, 2) void mha_stack_kernel(StackArgs sa) {
@@ -285,35 +367,9 @@ __global__ __launch_bounds__(NW * 64, 2) void mha_stack_kernel(StackArgs sa) {
                 const u32x4 qv = rows4[hq_local * 16 + j * 4 + kg];
                 qb[j] = live ? qv : u32x4{0u, 0u, 0u, 0u};
             }
-            if (holds_new_row) {
-                // The new token: its K row (normalised + rotated above) and V row go to the cache slot of this layer, and
-                // the running softmax starts from that one position -- score q.k, weight 1, output = the V row.
-                typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-                u32x4 kf[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) kf[j] = sh4[64 + j * 4 + kg];
-                const u32x4 vf = sh4[64 + 16 + n16];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) new_k[j] = kf[j];
-                new_v = vf;  // (filed in the cache behind the tiles: the stores' acknowledgement must not sit in front of a tile's wait)
-                float dot = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const uint32_t qw = qb[j][c], kw = kf[j][c];
-                        dot = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, qw), __builtin_bit_cast(bf16x2, kw), dot, false);
-                    }
-                dot = rows_sum(dot);
-                m_run = dot * a.scale_log2e;
-                l_run = kg == 0 ? 1.0f : 0.0f;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint32_t vw = vf[j >> 1];
-                    const float vj = (j & 1) ? bf16_hi(vw) : bf16_lo(vw);
-                    o[j] = f32x4{vj, vj, vj, vj};
-                }
-            }
+            // The new token's row starts the running softmax; it is filed in this layer's cache slot behind the tiles (the
+            // stores' acknowledgement must not sit in front of a tile's wait).
+            if (holds_new_row) start_from_new_row(sh4 + 64, qb, kg, n16, a.scale_log2e, new_k, new_v, m_run, l_run, o);
         }
 
         // ---- (3) this layer's tiles ----
@@ -325,52 +381,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mha_stack_kernel(StackArgs sa) {
             rd_stage = (rd_stage + 1 == NSTAGE) ? 0 : rd_stage + 1;
             --in_flight;
             issue_within(layer);
-            // q.K^T, online softmax, P^T.V on the matrix cores (the probabilities as hi + lo bf16)
-            f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, r.k[j]), __builtin_bit_cast(bf16x8, qb[j]), c, 0, 0, 0);
-            const int row0 = (wave + i * NW) * kTile + 4 * kg;
-            float s[4];
-            float tmax = -INFINITY;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                s[e] = (row0 + e < nrows) ? c[e] * a.scale_log2e : -INFINITY;
-                tmax = fmaxf(tmax, s[e]);
-            }
-            tmax = rows_max(tmax);
-            const float m_new = fmaxf(m_run, tmax);
-            const float alpha = fast_exp2(m_run - m_new);
-            float p[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) p[e] = fast_exp2(s[e] - m_new);
-            l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
-            m_run = m_new;
-            const uint32_t p01 = pack_bf16(p[0], p[1]);
-            const uint32_t p23 = pack_bf16(p[2], p[3]);
-            const uint32_t q01 = pack_bf16(p[0] - bf16_lo(p01), p[1] - bf16_hi(p01));
-            const uint32_t q23 = pack_bf16(p[2] - bf16_lo(p23), p[3] - bf16_hi(p23));
-            if (__any(alpha != 1.0f)) {
-                static_for<0, 4>([&](auto rr) {
-                    const float ar = row_bcast<rr.value>(alpha);  // (G <= 4: only DPP row 0 holds heads)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) o[j][rr.value] *= ar;
-                });
-            }
-            const i16x4 pa = __builtin_bit_cast(i16x4, u32x2{p01, p23});
-            const i16x4 pb = __builtin_bit_cast(i16x4, u32x2{q01, q23});
-            i16x4 vb4[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-                const uint32_t b01 = __builtin_amdgcn_perm(r.v[1][j >> 1], r.v[0][j >> 1], sel);
-                const uint32_t b23 = __builtin_amdgcn_perm(r.v[3][j >> 1], r.v[2][j >> 1], sel);
-                vb4[j] = __builtin_bit_cast(i16x4, u32x2{b01, b23});
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, vb4[j], o[j], 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pb, vb4[j], o[j], 0, 0, 0);
+            fold_tile(r, qb, (wave + i * NW) * kTile + 4 * kg, nrows, a.scale_log2e, m_run, l_run, o);
         }
 
         if (holds_new_row) {
@@ -582,6 +593,410 @@ __global__ __launch_bounds__(NW * 64, 2) void mha_stack_kernel(StackArgs sa) {
     }
 }
 
+// ---- layers that cannot see each other's writes ----
+// The same results as mha_stack_kernel and as one launch per layer, bit for bit (the same tiles per split and wavefront, the
+// same folds in the same order), with nothing in front of a layer: what bounds it is the K/V stream. The grid is the same,
+// one workgroup per (KV head, split) and compute unit, resident, walking the layers; its eight wavefronts have roles, and meet
+// at one workgroup barrier per layer:
+//   0-3  stream: tiles through a ring of kNStage LDS slots, one sequence over all layers, and fold them; four slots hold two
+//        layers' tiles ahead at 4096 positions. They do nothing else: no wavefront that streams ever waits for a store;
+//   4, 5 fold the four wavefronts' results of the layer before (one thread per head and 16-byte column) and store the split's
+//        partial rows, while 0-3 are in the next layer; the records follow a layer later, when the rows' acknowledgement has
+//        long arrived;
+//   6    brings in a later layer's small operands, normalises and rotates the query group once for the workgroup (the
+//        streaming wavefronts read operand fragments) and files the new token's rows in the cache;
+//   7    merges a head's splits, a step per layer and nothing waited for in between: asks for the records two layers behind,
+//        turns them into weights and asks for the partial rows three layers behind, sums them up four layers behind. A head's
+//        merging workgroup moves on from layer to layer (merge_split), so that each takes part every num_splits / group layers.
+// With the stream running a trip to memory takes 2 us and more, about as long as a layer's stream per workgroup (2.4 us at 4096
+// positions): waiting for one anywhere in a layer costs the stream (records right behind their rows + 12 us, a merge in
+// one piece + 10 us of 89 us over 36 layers).
+// A layer's partial rows and records live in region layer % regions of the workspace; region reuse waits for the heads' done
+// tags of the layer that had it before (set by 7 once the rows have been read back; normally long there).
+// Layer j's tags are set while layer j + kMergeLag streams, so with more regions than that no wait is for anything later than
+// its own layer and there is no cycle; with fewer (three or four) 7 takes its steps one after the other two layers behind.
+// 32 Q / 8 KV heads, 36 layers at 4096 + 1 positions: 243 us as a chain (mha_stack_kernel) -> 107 us = 5.6 TB/s; at 300 positions
+// 190 -> 54 us. The stream alone, with neither partial rows stored nor merges, is 89 us (6.8 TB/s): half a megabyte of stores per
+// layer costs 10 us and reading it back 8, whatever their cache policy and however many layers' stores go out together --
+// writes between a saturating stream of reads. Two, three or four ring slots: level.
+constexpr int kLayersStage = 4;   // ring slots per streaming wavefront
+constexpr int kLayersWaves = 8;
+constexpr int kStreamWaves = 4;   // wavefronts per split, as in the per-layer launches
+constexpr int kRecordLag = 2;     // layers behind the stream at which a merge asks for the records ...
+constexpr int kMergeLag = 4;      // ... and finishes
+
+// The workgroup (its split) that merges head h of the group in a layer.
+__device__ __forceinline__ int merge_split(int layer, int h, int group, int S) {
+    return S - 1 - (int)((uint32_t)(layer * group + h) % (uint32_t)S);
+}
+
+template <int G>
+__global__ __launch_bounds__(kLayersWaves * 64, 2) void mha_layers_kernel(StackArgs sa) {
+    static_assert(G <= 4, "two wavefronts fold a workgroup's G * 32 columns");
+    const KernelArgs& a = sa.a;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n16 = lane & 15;
+    const int kg = lane >> 4;
+    const int kvh = blockIdx.x;
+    const int split = blockIdx.y;
+    const int S = a.num_splits, L = sa.layers;
+    const int seq_len = a.seq_len, cached_len = seq_len - 1;
+    const int run = a.tiles_run, longer = a.tiles_longer;
+    const int ntiles = run + (split < longer ? 1 : 0);
+    const int begin = (split * run + min(split, longer)) * kTile;
+    const int nrows = min(ntiles * kTile, cached_len - begin);
+    const bool holds_new_row = split == S - 1;
+
+    // LDS: the rings; three layers' small operands (3 KiB each: q_norm | k_norm | sin | cos, new K row | new V row, the
+    // query rows); two layers' results of the streaming wavefronts; the weights of a merge.
+    constexpr int kStageBytes = 8192;
+    constexpr int kRingBytes = kStreamWaves * kLayersStage * kStageBytes;
+    constexpr int kOperandBytes = 3 * 1024, kOperandSets = 3;
+    constexpr int kFoldRows = kStreamWaves * G * kHeadDim * (int)sizeof(float);
+    constexpr int kFoldBytes = kFoldRows + 2 * kStreamWaves * G * (int)sizeof(float);
+    constexpr int kSmemBytes = kRingBytes + kOperandSets * kOperandBytes + 2 * kFoldBytes + 64 * (int)sizeof(float);
+    static_assert(kSmemBytes <= 160 * 1024, "LDS of one compute unit");
+    static_assert(kFoldBytes % 16 == 0, "16-byte accesses");
+    __shared__ __attribute__((aligned(1024))) char smem[kSmemBytes];
+    char* operands = smem + kRingBytes;
+    char* folds = operands + kOperandSets * kOperandBytes;
+    float* s_w = reinterpret_cast<float*>(folds + 2 * kFoldBytes);
+    auto fold_o = [&](int set, int w, int h) { return reinterpret_cast<float*>(folds + set * kFoldBytes) + (w * G + h) * kHeadDim; };
+    auto fold_m = [&](int set, int w, int h) { return reinterpret_cast<float*>(folds + set * kFoldBytes + kFoldRows) + w * G + h; };
+    auto fold_l = [&](int set, int w, int h) { return fold_m(set, kStreamWaves + w, h); };
+    // This wavefront's LDS accesses are done, then all wavefronts meet. (Requests to memory stay in flight.)
+    auto meet = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto layer_tag = [&](int layer) { return 0x80000000u | ((a.tag + (uint32_t)layer) & 0x7fffffffu); };
+    // (a record: tag, max, tag, sum; behind the region's partial rows)
+    auto record_offset = [&](int region, int hq, int sp) {
+        return (uint32_t)region * (uint32_t)sa.region_bytes + (uint32_t)(a.n_q * S) * (kHeadDim * 4u) + (uint32_t)(hq * S + sp) * 16u;
+    };
+    const __amdgpu_buffer_rsrc_t part_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(a.ws, 0, (int)(sa.regions * sa.region_bytes), 0x00020000);
+
+    if (wave < kStreamWaves) {
+        const int64_t split_off = (int64_t)kvh * a.head_stride + (int64_t)begin * a.row_stride;
+        const uint32_t rs = (uint32_t)a.row_stride * 2u;
+        const uint32_t last_off = (uint32_t)(nrows - 1) * rs;
+        const uint32_t k_row = (uint32_t)kg * rs;
+        const uint32_t k_col0 = (uint32_t)(n16 ^ kg) * 16u;
+        const uint32_t k_col1 = (uint32_t)(n16 ^ (4 + kg)) * 16u;
+        const uint32_t k_rd = (uint32_t)((n16 >> 2) * 1024 + (n16 & 3) * 256);
+        const uint32_t k_rd0 = k_rd + (uint32_t)((kg ^ (n16 & 7)) * 16);
+        const uint32_t k_rd1 = k_rd + (uint32_t)(((4 + kg) ^ (n16 & 7)) * 16);
+        const uint32_t v_col = (uint32_t)n16 * 16u;
+        char* my_ring = smem + wave * kLayersStage * kStageBytes;
+        const uint32_t my_ring_lds = (uint32_t)(uintptr_t)my_ring;
+        const int n_my = wave < ntiles ? (ntiles - wave + kStreamWaves - 1) / kStreamWaves : 0;
+        int iss_layer = 0, iss_i = 0, iss_stage = 0, in_flight = 0, rd_stage = 0;
+        auto issue_next = [&]() {
+            if (n_my == 0 || iss_layer >= L) return;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's previous contents have reached the VGPRs
+            const char* kb = reinterpret_cast<const char*>(a.k + (int64_t)iss_layer * sa.cache_stride + split_off);
+            const char* vb = reinterpret_cast<const char*>(a.v + (int64_t)iss_layer * sa.cache_stride + split_off);
+            const uint32_t base = (uint32_t)(wave + iss_i * kStreamWaves) * (kTile * rs);
+            const uint32_t slot = my_ring_lds + (uint32_t)iss_stage * kStageBytes;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t ko = min(base + k_row + (uint32_t)(4 * i) * rs, last_off) + ((i & 1) ? k_col1 : k_col0);
+                dma16(kb, ko, slot + i * 1024);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t vo = min(base + k_row + (uint32_t)(4 * i) * rs, last_off) + v_col;
+                dma16(vb, vo, slot + 4096 + i * 1024);
+            }
+            ++in_flight;
+            iss_stage = (iss_stage + 1 == kLayersStage) ? 0 : iss_stage + 1;
+            if (++iss_i == n_my) {
+                iss_i = 0;
+                ++iss_layer;
+            }
+        };
+        for (int s0 = 0; s0 < kLayersStage; ++s0) issue_next();
+        meet();  // layer 0's query is in LDS
+        int op_set = 0;
+        for (int layer = 0; layer < L; ++layer) {
+            const u32x4* ops4 = reinterpret_cast<const u32x4*>(operands + op_set * kOperandBytes);
+            op_set = op_set + 1 == kOperandSets ? 0 : op_set + 1;
+            const int hq_local = min(n16, a.group - 1);
+            const bool live = n16 < a.group;
+            u32x4 qb[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u32x4 qv = ops4[128 + hq_local * 16 + j * 4 + kg];
+                qb[j] = live ? qv : u32x4{0u, 0u, 0u, 0u};
+            }
+            float m_run = -INFINITY, l_run = 0.0f;
+            f32x4 o[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (holds_new_row && wave == 0) {
+                u32x4 kf[4], vf;
+                start_from_new_row(ops4 + 64, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o);
+            }
+            for (int i = 0; i < n_my; ++i) {
+                TileRegs r;
+                wait_tiles_in_flight(in_flight - 1);
+                const char* kp = my_ring + rd_stage * kStageBytes;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    r.k[j] = *reinterpret_cast<const u32x4*>(kp + ((j & 1) ? k_rd1 : k_rd0) + (j >> 1) * 128);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    r.v[e] = *reinterpret_cast<const u32x4*>(kp + 4096 + kg * 1024 + e * 256 + n16 * 16);
+                rd_stage = (rd_stage + 1 == kLayersStage) ? 0 : rd_stage + 1;
+                --in_flight;
+                issue_next();
+                fold_tile(r, qb, (wave + i * kStreamWaves) * kTile + 4 * kg, nrows, a.scale_log2e, m_run, l_run, o);
+            }
+            l_run = rows_sum(l_run);
+            const int set = layer & 1;
+            if (kg == 0) {
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    if (r4 < G) {
+                        float* dst = fold_o(set, wave, r4) + n16 * 8;
+                        *reinterpret_cast<f32x4*>(dst) = f32x4{o[0][r4], o[1][r4], o[2][r4], o[3][r4]};
+                        *reinterpret_cast<f32x4*>(dst + 4) = f32x4{o[4][r4], o[5][r4], o[6][r4], o[7][r4]};
+                    }
+                }
+                if (n16 < G) {
+                    *fold_m(set, wave, n16) = m_run;
+                    *fold_l(set, wave, n16) = l_run;
+                }
+            }
+            meet();
+        }
+    } else if (wave < 6) {
+        const int u = (wave - kStreamWaves) * 64 + lane;
+        const int h = min(u >> 5, a.group - 1), c4 = u & 31;
+        const bool active = u < a.group * (kHeadDim / 4);
+        const int hq = kvh * a.group + h;
+        const uint32_t po = (uint32_t)(((int64_t)hq * S + split) * kHeadDim + c4 * 4) * (uint32_t)sizeof(float);
+        // Region reuse: every `step` layers the tags of the `step` layers that had the next regions, one lane per layer and
+        // head, asked for a layer ahead.
+        const int step = max(1, min(8, sa.regions - kMergeLag - 2));
+        int next_check = sa.regions;
+        auto ask_done = [&](int layer) {
+            const int k = min(lane >> 2, step - 1);
+            return __hip_atomic_load(sa.done + ((layer + k) % sa.regions) * kDoneLineWords + kvh * a.group + min(lane & 3, a.group - 1),
+                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        auto wanted = [&](int layer) { return layer_tag(layer - sa.regions + min(lane >> 2, step - 1)); };
+        uint32_t seen = 0;
+        bool poisoned = false;  // a wait gave up: this split's results of the layer and the following ones are NaN
+        int region = 0, prev_region = 0;
+        float prev_m = 0.0f, prev_l = 0.0f;
+        // The records of a layer's partial rows, once those are acknowledged. (The 32 columns of a head are stored by one half
+        // of one wavefront.)
+        auto publish = [&](int layer) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            // (one 16-byte store: either half carries the tag, so it does not matter if they arrive one after the other)
+            if (active && c4 == 0)
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    u32x4{layer_tag(layer), __builtin_bit_cast(uint32_t, prev_m), layer_tag(layer), __builtin_bit_cast(uint32_t, prev_l)},
+                    part_rsrc, record_offset(prev_region, hq, split), 0, kCacheDevice);
+        };
+        meet();
+        for (int layer = 0; layer < L; ++layer) {
+            meet();
+            const int set = layer & 1;
+            float mw[kStreamWaves], lw[kStreamWaves];
+            f32x4 ow[kStreamWaves];
+#pragma unroll
+            for (int w = 0; w < kStreamWaves; ++w) {
+                mw[w] = *fold_m(set, w, h);
+                lw[w] = *fold_l(set, w, h);
+                ow[w] = *reinterpret_cast<const f32x4*>(fold_o(set, w, h) + c4 * 4);
+            }
+            if (layer > 0) publish(layer - 1);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            float mx = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < kStreamWaves; ++w) mx = fmaxf(mx, mw[w]);
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            float lsum = 0.0f;
+#pragma unroll
+            for (int w = 0; w < kStreamWaves; ++w) {
+                const float f = (mw[w] == -INFINITY) ? 0.0f : fast_exp2(mw[w] - mx);
+                acc += ow[w] * f;
+                lsum += lw[w] * f;
+            }
+            if (layer == next_check && !poisoned) {
+                bool free = a.max_polls > 0 && __all(seen == wanted(layer));
+                for (int spin = 1; spin < a.max_polls && !free; ++spin) free = __all(ask_done(layer) == wanted(layer));
+                if (__builtin_expect(!free, 0)) {
+                    poisoned = true;
+                    if (lane == 0) atomicAdd(&g_poll_timeouts, 1u);
+                }
+                next_check += step;
+            }
+            if (active)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), part_rsrc,
+                                                       po + (uint32_t)region * (uint32_t)sa.region_bytes, 0, kCacheDevice);
+            prev_m = mx;
+            prev_l = poisoned ? __builtin_nanf("") : lsum;
+            prev_region = region;
+            region = region + 1 == sa.regions ? 0 : region + 1;
+            if (layer + 1 == next_check) seen = ask_done(layer + 1);
+        }
+        publish(L - 1);
+    } else if (wave == 6) {
+        const int c16 = lane & 15, which = lane >> 4;
+        auto fetch = [&](int layer, int set) {
+            const uint32_t st = (uint32_t)(uintptr_t)(operands + set * kOperandBytes);
+            const float* sin_row = a.sin_cache + (int64_t)(seq_len - 1) * 64;
+            const float* cos_row = a.cos_cache + (int64_t)(seq_len - 1) * 64;
+            const uint64_t w_base = reinterpret_cast<uint64_t>(a.norm_w + (int64_t)layer * sa.normw_stride) + (uint64_t)(which & 1) * 256u;
+            const uint64_t t_base = reinterpret_cast<uint64_t>(which == 2 ? sin_row : cos_row);
+            dma16_gather(reinterpret_cast<const void*>((which < 2 ? w_base : t_base) + (uint64_t)c16 * 16u), st);
+            if (holds_new_row) {
+                const uint16_t* kn = a.k_new + (int64_t)layer * sa.knew_stride;
+                const uint16_t* vn = a.v_new + (int64_t)layer * sa.vnew_stride;
+                const uint64_t p1 = reinterpret_cast<uint64_t>((which & 1) == 0 ? kn : vn) + (uint64_t)(kvh * kHeadDim * 2 + c16 * 16);
+                dma16_gather(reinterpret_cast<const void*>(p1), st + 1024);
+            }
+            const int head = min(which, a.group - 1);
+            dma16_gather(a.q + (int64_t)layer * sa.q_stride + (int64_t)(kvh * a.group + head) * kHeadDim + c16 * 8, st + 2048);
+        };
+        // Layer p's operands are asked for a barrier ahead of their use here and handed over a barrier ahead of the layer.
+        fetch(0, 0);
+        int set = 0;
+        for (int p = 0; p < L; ++p) {
+            char* ops = operands + set * kOperandBytes;
+            set = set + 1 == kOperandSets ? 0 : set + 1;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (p + 1 < L) fetch(p + 1, set);
+            norm_rope_rows_lds(ops + 2048, ops, ops + 512, ops + 768, kg, n16, a.eps);
+            if (holds_new_row) {
+                norm_rope_rows_lds(ops + 1024, ops + 256, ops + 512, ops + 768, 0, n16, a.eps);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                const u32x4* rows = reinterpret_cast<const u32x4*>(ops + 1024);
+                const int64_t row_off = (int64_t)p * sa.cache_stride + (int64_t)(seq_len - 1) * a.row_stride + kvh * a.slot_head_stride;
+                uint16_t* dst = const_cast<uint16_t*>(which == 0 ? a.k : a.v) + row_off;
+                if (which < 2) *reinterpret_cast<u32x4*>(dst + c16 * 8) = rows[which * 16 + c16];
+            }
+            meet();
+        }
+        meet();
+    } else {
+        const int c4 = lane & 31, part = lane >> 5;
+        constexpr int kBatch = 16;
+        // What a merge carries from step to step: the records, then the rows and what their weights need.
+        u32x4 rec = {0u, 0u, 0u, 0u};
+        f32x4 v[kBatch];
+        float den = 0.0f;
+        bool arrived = false;
+        auto head_of = [&](int layer) {  // the head of the group this workgroup merges in the layer, or -1
+            if (layer < 0 || layer >= L) return -1;
+            int found = -1;
+            for (int h = 0; h < a.group; ++h) found = merge_split(layer, h, a.group, S) == split ? h : found;
+            return found;
+        };
+        auto load_record = [&](int layer, int hq) {
+            return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 part_rsrc, record_offset(layer % sa.regions, hq, min(lane, S - 1)), 0, kCacheDevice));
+        };
+        auto load_partial = [&](int layer, int hq, int sp) {
+            const uint32_t base = (uint32_t)(layer % sa.regions) * (uint32_t)sa.region_bytes + (uint32_t)hq * (uint32_t)S * (kHeadDim * 4u);
+            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 part_rsrc, base + (uint32_t)c4 * 16u + (uint32_t)min(sp, S - 1) * (kHeadDim * 4u), 0, kCacheDevice));
+        };
+        auto ask_records = [&](int layer) {
+            const int h = head_of(layer);
+            if (h < 0) return;
+            asm volatile("" ::: "memory");
+            rec = load_record(layer, kvh * a.group + h);
+        };
+        auto ask_rows = [&](int layer) {
+            const int h = head_of(layer);
+            if (h < 0) return;
+            const int hq = kvh * a.group + h;
+            const uint32_t tag = layer_tag(layer);
+            arrived = a.max_polls > 0 && __all(rec[0] == tag && rec[2] == tag);
+            for (int spin = 1; spin < a.max_polls && !arrived; ++spin) {
+                asm volatile("" ::: "memory");  // (a poll is a load of its own ...)
+                rec = load_record(layer, hq);
+                arrived = __all(rec[0] == tag && rec[2] == tag);
+            }
+            asm volatile("" ::: "memory");  // (... and the rows are asked for behind the last one)
+            if (__builtin_expect(!arrived, 0) && lane == 0) atomicAdd(&g_poll_timeouts, 1u);
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) v[j] = load_partial(layer, hq, part + 2 * j);
+            const uint32_t m_bits = rec[1], l_bits = rec[3];
+            const float m_reg = lane < S ? __builtin_bit_cast(float, m_bits) : -INFINITY;
+            const float l_reg = lane < S ? __builtin_bit_cast(float, l_bits) : 0.0f;
+            const float mx = wave_max(m_reg);
+            const float f = (m_reg == -INFINITY) ? 0.0f : fast_exp2(m_reg - mx);
+            if (lane < S) {
+                s_w[lane] = f;
+                // A record is cleared only where a replay of this launch (same tags) would find it again: in a region that
+                // one layer has to itself. Elsewhere the region's other layers leave another layer's tag there.
+                if (layer < sa.regions && layer + sa.regions >= L)
+                    __builtin_amdgcn_raw_buffer_store_b128(u32x4{0u, 0u, 0u, 0u}, part_rsrc, record_offset(layer, hq, lane), 0, kCacheDevice);
+            }
+            den = wave_sum(lane < S ? l_reg * f : 0.0f);
+        };
+        auto finish = [&](int layer) {
+            const int h = head_of(layer);
+            if (h < 0) return;
+            const int hq = kvh * a.group + h;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                const int sp = part + 2 * j;
+                sum += v[j] * (sp < S ? s_w[sp] : 0.0f);
+            }
+            for (int s0 = part + 2 * kBatch; s0 < S; s0 += 2 * kBatch) {
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) v[j] = load_partial(layer, hq, s0 + 2 * j);
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) {
+                    const int sp = s0 + 2 * j;
+                    sum += v[j] * (sp < S ? s_w[sp] : 0.0f);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] = halves_sum(sum[e]);
+            // The rows have been read and the records are cleared (asked for a step ago): the region is free for this head.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (lane == 0)
+                __hip_atomic_store(sa.done + (layer % sa.regions) * kDoneLineWords + hq, layer_tag(layer), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (part == 0) {
+                const f32x4 r = sum * (arrived ? 1.0f / den : __builtin_nanf(""));
+                const int64_t off = (int64_t)layer * sa.out_stride + (int64_t)hq * kHeadDim + c4 * 4;
+                *reinterpret_cast<uint2*>(a.out + off) = make_uint2(pack_bf16(r[0], r[1]), pack_bf16(r[2], r[3]));
+                if (a.out_f32) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) a.out_f32[off + e] = r[e];  // (only 4-byte alignment is promised)
+                }
+            }
+        };
+        const bool in_steps = sa.regions > kMergeLag;
+        meet();
+        for (int layer = 0; layer < L + kMergeLag; ++layer) {
+            if (layer < L) meet();
+            if (in_steps) {
+                finish(layer - kMergeLag);
+                ask_rows(layer - kRecordLag - 1);
+                ask_records(layer - kRecordLag);
+            } else {
+                ask_records(layer - kRecordLag);
+                ask_rows(layer - kRecordLag);
+                finish(layer - kRecordLag);
+            }
+        }
+    }
+}
+
 template <int G>
 bool launch_stack_g(const StackArgs& sa, int n_kv, hipStream_t stream) {
 #ifndef LLMI_STACK_WAVES
@@ -589,6 +1004,10 @@ bool launch_stack_g(const StackArgs& sa, int n_kv, hipStream_t stream) {
 #endif
     constexpr int NW = LLMI_STACK_WAVES, NSTAGE = 8 / NW;  // the rings hold eight tiles per workgroup either way
     const dim3 grid(n_kv, sa.a.num_splits), block(NW * 64);
+    if (sa.regions > 0) {
+        hipLaunchKernelGGL((mha_layers_kernel<G>), grid, dim3(kLayersWaves * 64), 0, stream, sa);
+        return true;
+    }
     if (sa.a.by_side) hipLaunchKernelGGL((mha_stack_kernel<G, NW, NSTAGE, true>), grid, block, 0, stream, sa);
     else hipLaunchKernelGGL((mha_stack_kernel<G, NW, NSTAGE, false>), grid, block, 0, stream, sa);
     return true;
@@ -605,6 +1024,8 @@ bool launch_stack(const StackArgs& sa, int n_kv, int group_pad, int waves, hipSt
         default: return false;
     }
 }
+
+int stack_max_regions(int head_num) { return head_num <= kDoneLineWords ? kDoneCopies : 0; }
 
 size_t stack_done_bytes(int head_num) {
     return (size_t)kDoneCopies * (size_t)((head_num + kDoneLineWords - 1) / kDoneLineWords) * kDoneLineWords * sizeof(uint32_t);
