@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -111,10 +112,11 @@ int test_far_home() { return g_test_far_home.load(std::memory_order_relaxed); }
 // many workgroups; with fewer, the workgroup of the last split merges them all. Measured, 32 Q / 8 KV heads, spread
 // against not: 16 splits 5.08 : 4.98 us at 1024 positions, 5.87 : 5.77 at 2048; 8 splits 4.51 : 4.41 at 256; 32 splits
 // 5.03 : 5.14 at 1024, 5.71 : 5.80 at 2048, 6.86 : 7.08 at 4096, 7.88 : 8.10 at 6000; 64 Q heads, 16 splits 5.55 : 5.68 at
-// 1024, 7.63 : 7.81 at 4096, 32 splits at 32768 24.4 : 25.3. LLMI_HIP_SPREAD_MIN_SPLITS moves the boundary.
+// 1024, 7.63 : 7.81 at 4096, 32 splits at 32768 24.4 : 25.3. Groups of 16 (four wavefronts): always, as soon as there is a
+// split for every head. LLMI_HIP_SPREAD_MIN_SPLITS moves the boundary.
 int spread_merge_min_splits(int group_pad) {
     static const int v = env_int("LLMI_HIP_SPREAD_MIN_SPLITS", 1, 1 << 20, 0);
-    return v ? v : group_pad >= 8 ? 16 : 32;
+    return v ? v : group_pad >= 16 ? 1 : group_pad >= 8 ? 16 : 32;
 }
 
 // Where the splits' runs start a multiple of 512 KiB apart, the workgroups of a KV head, walking in step, keep hitting
@@ -153,6 +155,37 @@ int dyn_stagger(int kv_layout, int64_t max_run_bytes) {
 }
 
 int check_launch() { return record_hip_error(hipGetLastError(), "kernel launch"); }
+
+// Longest context (cached positions) that runs as a single pass at a wave count. Groups of 8 query heads run 8 waves per
+// workgroup, which carry a single pass a little further (64 query / 8 KV heads: single pass 5.14 us against 5.64 us split at
+// 208 positions; at 256, where 16 splits have a tile each, 5.51 against 5.34).
+// Groups of more than 8 heads stay with it until there is a split per head to merge them (32 Q / 2 KV heads, single pass : 14 or
+// 17 splits: 6.1 : 9.5 us at 220 positions, 6.8 : 5.9 at 260, where the 17 can take a head each).
+static int single_pass_limit(int kv_mul, int group_pad, bool eight_waves) {
+    if (env_tuning().single_pass_max >= 0) return env_tuning().single_pass_max;
+    if (group_pad > 8) return kTile * kv_mul - 1 > kSinglePassMaxLen ? kTile * kv_mul - 1 : kSinglePassMaxLen;
+    return group_pad == 8 && eight_waves ? 240 : kSinglePassMaxLen;
+}
+
+// Split counts below the full grid's: half of the workgroups, a quarter of them.
+// (Never fewer than heads in a group of more than 8: see single_pass_limit.)
+static int fewest_splits(int kv_mul) { return kv_mul > 8 ? kv_mul : 2; }
+static int half_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv, fewest_splits(kv_mul)); }
+static int quarter_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv / 2, fewest_splits(kv_mul)); }
+
+void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, int* single, int* quarter, int* half) {
+    *single = *quarter = *half = 0;
+    if (args.num_splits != 0 || args.force_path != LLMI_PATH_AUTO || env_tuning().num_splits) return;
+    const int n_kv = args.kv_dim / args.head_dim;
+    // (the launch has the split path's waves: four, eight for groups of 8 heads. At four a single pass still is the faster one
+    // up to the same length as at the eight that a launch planned for it would have: 4.34 : 4.51 us at 176 positions,
+    // 4.96 : 4.67 at 220)
+    *single = single_pass_limit(args.kv_mul, plan.group_pad, plan.waves_per_group >= 8) / kTile;
+    // (no more than the launch has workgroups for)
+    const int q = quarter_splits(n_kv, args.kv_mul), h = half_splits(n_kv, args.kv_mul);
+    *quarter = q < plan.num_splits ? q : plan.num_splits;
+    *half = h < plan.num_splits ? h : plan.num_splits;
+}
 
 static int validate_mha(const llmi_mha_args* a) {
     if (!a) return LLMI_ERR_NULL_POINTER;
@@ -194,11 +227,7 @@ static int make_plan(const llmi_mha_args* a, llmi_mha_plan* p, int wave_cap = kM
     const size_t per_split_fused = (size_t)a->head_num * (a->head_dim * sizeof(float) + 2 * sizeof(unsigned long long));
 
     const int single_waves_max = (max_waves < wave_cap ? max_waves : wave_cap);  // 8 where the kernel variant allows
-    // Groups of 8 query heads run 8 waves per workgroup, which carry a single pass a little further
-    // (64 query / 8 KV heads: single pass 5.14 us against 5.64 us split at 208 positions; at 256, where
-    // 16 splits have a tile each, 5.51 against 5.34).
-    int single_pass_max = (group_pad == 8 && wave_cap >= 8) ? 240 : kSinglePassMaxLen;
-    if (env_tuning().single_pass_max >= 0) single_pass_max = env_tuning().single_pass_max;
+    const int single_pass_max = single_pass_limit(a->kv_mul, group_pad, wave_cap >= 8);
     int path = a->force_path;
     if (path == LLMI_PATH_AUTO) {
         if (a->num_splits == 1) path = LLMI_PATH_SINGLE_PASS;
@@ -235,12 +264,9 @@ static int make_plan(const llmi_mha_args* a, llmi_mha_plan* p, int wave_cap = kM
             // traffic and lengthen the combine (64 splits: +1 us everywhere).
             // And no more splits than the caller's workspace can hold.
             int target = kTargetGroups / n_kv;
-            if (target < 2) target = 2;
+            if (target < fewest_splits(a->kv_mul)) target = fewest_splits(a->kv_mul);
             if (target > kMaxSplits) target = kMaxSplits;
-            int half = kMinGroups / n_kv;
-            if (half < 2) half = 2;
-            int quarter = half / 2;
-            if (quarter < 2) quarter = 2;
+            const int half = half_splits(n_kv, a->kv_mul), quarter = quarter_splits(n_kv, a->kv_mul);
             // One workgroup per CU pays as soon as half as many splits would hold more than four tiles each (more than
             // one per wavefront at four wavefronts). Measured with the merge of a KV head's query heads spread over
             // several workgroups (which needs 32 splits to pay at groups of four, see spread_merge_min_splits), 32 Q / 8 KV

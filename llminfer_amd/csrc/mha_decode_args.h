@@ -50,7 +50,12 @@ struct KernelArgs {
     // partial outputs / records; XCDs 4-7 use the other one.
     bool by_side;
     unsigned long long ppar[2], rpar[2];
-    bool spread_merge;  // fused combine: the heads of a KV head are merged by different workgroups (the host's choice, by split count)
+    int32_t spread_min;  // fused combine: fewest splits at which the heads of a KV head are merged by different workgroups
+    // Position read on the device (DYN kernels), the dispatcher's rule for the tiles found: up to dyn_single tiles one split,
+    // below dyn_half tiles dyn_quarter splits, up to 4 * dyn_half tiles dyn_half splits, beyond that num_splits (a forced plan
+    // has zeros: num_splits at every length); dyn_magic: 2^32 / count, rounded up, for the three counts in that order.
+    int32_t dyn_single, dyn_quarter, dyn_half;
+    uint32_t dyn_magic[3];
     int32_t far_home;  // testing aid: 1 = every split but the merging one, 2 = every second one uses the other side's home
 };
 

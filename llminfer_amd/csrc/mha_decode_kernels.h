@@ -70,9 +70,17 @@ namespace {
 template <int G, int NW>
 constexpr int kWavesPerEu = (G >= 16 && NW != 2) ? 1 : LLMI_MIN_WAVES_PER_EU;
 
+// Splits above which the wavefronts of a merging workgroup share a head's splits. (At 64 it is level: 6.50 -> 6.35 us with four
+// wavefronts, 6.43 -> 6.86 with eight, 4001 positions. And the multi-layer kernels, which stand for launches of up to 64
+// splits, add them up in one wavefront's order.)
+#ifndef LLMI_WIDE_MERGE_MIN
+#define LLMI_WIDE_MERGE_MIN 64
+#endif
+constexpr int kWideMergeMin = LLMI_WIDE_MERGE_MIN;
+
 template <int G, int NW, int NSTAGE, bool APPEND, bool DYN, bool STAGGER, bool OPROJ, bool BYSIDE>
 __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState& proj) {
-    constexpr bool kSpreadMerge = LLMI_SPREAD_MERGE && !OPROJ && G <= NW;
+    constexpr bool kSpreadMerge = LLMI_SPREAD_MERGE && !OPROJ;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: loop control stays on the SALU
     const int n16 = lane & 15;  // MFMA column / DPP-row lane
@@ -90,25 +98,50 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     // has work whenever there are at least S tiles and the last split -- the one that merges,
     // and in the append variant the one that holds the new token -- never has the longest run.
     // With a position read from device memory the grid was sized for the largest position:
-    // the same rule is applied to the tiles there are, and splits beyond the tile count leave
-    // at once.
+    // the same rules are applied to the tiles there are -- a single pass, a quarter or half of the
+    // splits or all of them, as the host would have planned --, and the splits that are not needed leave at once.
+    // 32 Q / 8 KV heads, append variant in a captured 36-layer step sized for 8192 positions, us per layer, all splits as far as
+    // there are tiles : the rule: 5.54 : 4.07 at 60 positions, 5.53 : 5.25 at 170, 5.65 : 5.41 at 300, 5.69 : 5.47 at 600.
     // Append variant: the new token's row never comes from the cache (its K and V are in registers
     // and go straight into the running softmax of one wave), so the tiles cover positions 0 .. pos-1.
     int seq_len = a.seq_len, n_active = a.num_splits;
-    if constexpr (DYN) {
-        seq_len = max(0, min(*a.pos_dev, a.seq_len - 1)) + 1;
-        n_active = min(a.num_splits, max(1, (seq_len - (APPEND ? 1 : 0) + kTile - 1) / kTile));
-        if (split >= n_active) return;
-    }
-    const int cached_len = seq_len - (APPEND ? 1 : 0);  // positions streamed from the cache
     // (the host never asks for more splits than tiles; 0 tiles: 1 split). The division is done on
     // the host when the position is known there: it is 33 instructions in front of the first load.
     int run = a.tiles_run, longer = a.tiles_longer;  // splits 0 .. longer-1 take run + 1 tiles
     if constexpr (DYN) {
-        const int total_tiles = (cached_len + kTile - 1) / kTile;
-        run = total_tiles / n_active;
-        longer = total_tiles % n_active;
+        // Everything on the way to the first request depends on the position, which takes a trip to memory of its own: the
+        // arguments the prologue needs are therefore all asked for in one go in front of it (left to itself the compiler
+        // asks for some where they are used, a trip each), and the division by the split count is a multiplication by
+        // the host's reciprocal. With the rule
+        // but without these two 5.84 us per layer at 1100 positions and 9.44 at 8000, with them 5.72 and 9.26 (5.58 and 9.18 with
+        // the position known to the host).
+        asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.row_stride), "s"(a.head_stride), "s"(a.group), "s"(a.num_splits),
+                     "s"(a.dyn_single), "s"(a.dyn_half), "s"(a.dyn_quarter), "s"(a.dyn_magic[0]), "s"(a.dyn_magic[1]), "s"(a.dyn_magic[2]));
+        if constexpr (APPEND) asm volatile("" ::"s"(a.norm_w), "s"(a.sin_cache), "s"(a.cos_cache), "s"(a.k_new), "s"(a.v_new));
+        seq_len = max(0, min(*a.pos_dev, a.seq_len - 1)) + 1;
+        const int tiles = (seq_len - (APPEND ? 1 : 0) + kTile - 1) / kTile;
+        const bool few = tiles < a.dyn_half, medium = tiles <= 4 * a.dyn_half;
+        n_active = few ? a.dyn_quarter : medium ? a.dyn_half : a.num_splits;
+        const uint32_t magic = few ? a.dyn_magic[0] : medium ? a.dyn_magic[1] : a.dyn_magic[2];
+        run = (int)(((uint64_t)(uint32_t)tiles * magic) >> 32);
+        longer = tiles - run * n_active;
+        if (longer < 0) {  // (the rounded-up reciprocal is one too high at most, and only beyond 2^24 tiles)
+            --run;
+            longer += n_active;
+        }
+        if (tiles < n_active) {  // a tile each
+            n_active = tiles;
+            run = 1;
+            longer = 0;
+        }
+        if (tiles <= a.dyn_single || n_active <= 1) {
+            n_active = 1;
+            run = tiles;
+            longer = 0;
+        }
+        if (split >= n_active) return;
     }
+    const int cached_len = seq_len - (APPEND ? 1 : 0);  // positions streamed from the cache
     const int ntiles = run + (split < longer ? 1 : 0);
     const int begin = (split * run + min(split, longer)) * kTile;
     const int nrows = min(ntiles * kTile, cached_len - begin);  // > 0 unless nothing is cached yet
@@ -378,11 +411,12 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     // path of whoever waits for this split (the empty asm statements keep the compiler from moving the work there).
     const bool fused = a.records != nullptr && n_active > 1;
     const int my_xs = package_side<BYSIDE>();  // wave-uniform: the side of the package this workgroup runs on
-    // Who merges a query head's splits (log-sum-exp): where one wavefront merges a head (G <= NW) and there are at
-    // least as many splits as heads in the group, head h's splits are merged by wavefront 0 of the workgroup of split
-    // SA-1-h, so that the heads' read-backs (16 KiB each at 32 splits) run on different compute units at the same
-    // time instead of queueing at one; otherwise the workgroup of the last split merges every head.
-    const bool spread = kSpreadMerge && a.spread_merge && n_active >= a.group;
+    // Who merges a query head's splits (log-sum-exp): with enough splits, and at least as many as heads in the group,
+    // head h's splits are merged by the workgroup of split SA-1-h, so that the heads' read-backs (16 KiB each at 32
+    // splits) run on different compute units at the same time instead of queueing at one; otherwise the workgroup of
+    // the last split merges every head. For groups of 16 (four wavefronts per workgroup) the latter means four heads'
+    // polls in turn and a shared read-back: 32 Q / 2 KV heads 10.9 -> 5.9 us at 500 positions, 27.3 -> 12.2 at 40001.
+    const bool spread = kSpreadMerge && n_active >= a.spread_min && n_active >= a.group;
     const int merge_head = spread && n_active - 1 - split < a.group ? n_active - 1 - split : -1;
     const bool merges_any = spread ? merge_head >= 0 : split == n_active - 1;
     // (testing aid: pretend this split ran on the other side; never a merging one, whose own rows it reads itself)
@@ -531,11 +565,16 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
 
     if constexpr (OPROJ) proj.worker = split != n_active - 1;
     // One thread per (head, 16-byte column): weights e^(m_w - M) of the waves, weighted sum.
-    for (int u = threadIdx.x; u < n_units; u += NW * 64) {
+    constexpr int kUnits = (G * (kHeadDim / 4) + NW * 64 - 1) / (NW * 64);  // columns per thread
+    float unit_m[kUnits], unit_l[kUnits];
+#pragma unroll
+    for (int i = 0; i < kUnits; ++i) {
+        const int u = (int)threadIdx.x + i * NW * 64;
+        if (u >= n_units) break;
         const int h = u >> 5;
         const int c4 = u & 31;
         MergeUnit unit = first_unit;  // (worked out while the first tiles were on their way)
-        if (u != (int)threadIdx.x) unit = merge_unit(u);
+        if (i > 0) unit = merge_unit(u);
         // (all of a unit's LDS reads are requested before the first is used: one round trip, not two)
         float mw[NW], lw[NW];
         f32x4 ow[NW];
@@ -557,6 +596,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             acc += ow[w] * f;
             lsum += lw[w] * f;
         }
+        unit_m[i] = mx;
+        unit_l[i] = lsum;
         const int hq = unit.hq;
         if (n_active == 1) {
             const f32x4 r = acc * (1.0f / lsum);  // (one division, like the fused combine's)
@@ -575,23 +616,6 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 // anyone flushing or invalidating a cache.
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), part_rsrc,
                                                        (uint32_t)(po * (int64_t)sizeof(float)), 0, 16);
-                if (spread ? h != merge_head : split != n_active - 1) {
-                    // Publish the head's record as soon as this wavefront's stores are acknowledged:
-                    // the 32 columns of a head are stored by one half of one wavefront, so no
-                    // workgroup barrier is needed.
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    if (c4 == 0) {
-                        unsigned long long* rec = a.records + unit.rec;
-                        const unsigned long long tag = a.tag;
-                        const unsigned long long m_bits = __builtin_bit_cast(uint32_t, mx);
-                        const unsigned long long l_bits = __builtin_bit_cast(uint32_t, lsum);
-                        __hip_atomic_store(rec, tag | (m_bits << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        __hip_atomic_store(rec + 1, tag | (l_bits << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    }
-                } else if (c4 == 0) {  // the workgroup that merges this head keeps its own pair in LDS
-                    s_fin[2 * h] = mx;
-                    s_fin[2 * h + 1] = lsum;
-                }
             } else {
                 *reinterpret_cast<f32x4*>(a.ws + po) = acc;
                 if (c4 == 0) {
@@ -602,6 +626,31 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         }
     }
     if (!fused) return;
+    // The heads' records, once every column of this wavefront is acknowledged (one wait, however many heads it has).
+#pragma unroll
+    for (int i = 0; i < kUnits; ++i) {
+        const int u = (int)threadIdx.x + i * NW * 64;
+        if (u >= n_units) break;
+        const int h = u >> 5;
+        const int c4 = u & 31;
+        if (spread ? h != merge_head : split != n_active - 1) {
+            // Publish the head's record as soon as this wavefront's stores are acknowledged:
+            // the 32 columns of a head are stored by one half of one wavefront, so no
+            // workgroup barrier is needed.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (c4 == 0) {
+                unsigned long long* rec = a.records + (i > 0 ? merge_unit(u).rec : first_unit.rec);
+                const unsigned long long tag = a.tag;
+                const unsigned long long m_bits = __builtin_bit_cast(uint32_t, unit_m[i]);
+                const unsigned long long l_bits = __builtin_bit_cast(uint32_t, unit_l[i]);
+                __hip_atomic_store(rec, tag | (m_bits << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(rec + 1, tag | (l_bits << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } else if (c4 == 0) {  // the workgroup that merges this head keeps its own pair in LDS
+            s_fin[2 * h] = unit_m[i];
+            s_fin[2 * h + 1] = unit_l[i];
+        }
+    }
 
     // ---- fused combine ----
     // The workgroup of the LAST split of this KV head merges the partials of its
@@ -629,7 +678,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     // lanes' registers. This workgroup's own pair comes straight from LDS: its record would be the
     // last one to become visible. Returns false if a record never came. A record only counts when
     // it carries this call's tag (never zero, which is what a cleared record holds).
-    auto wait_records = [&](int h, auto slots, float* m_reg, float* l_reg, bool* home) -> bool {
+    // (splits first .. first + count - 1: all of them, or a wavefront's share of a wide merge)
+    auto wait_records = [&](int h, int first, int count, auto slots, float* m_reg, float* l_reg, bool* home) -> bool {
         constexpr int kSlots = decltype(slots)::value;  // splits per lane
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) {
@@ -643,7 +693,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         const WsHead wh = ws_head<BYSIDE>(a, kvh * a.group + h);
         const unsigned long long* rec_near[kSlots];
 #pragma unroll
-        for (int j = 0; j < kSlots; ++j) rec_near[j] = a.records + (int64_t)ws_row<9>(wh, min(lane + 64 * j, SA - 1), my_xs) * 2;
+        for (int j = 0; j < kSlots; ++j) rec_near[j] = a.records + (int64_t)ws_row<9>(wh, min(first + lane + 64 * j, SA - 1), my_xs) * 2;
         // One round of polls. BOTH: also look where a split that ran on the other side of the package would have put its
         // record (never needed when the workgroups of a KV head share an XCD, so the first rounds do without).
         auto poll_round = [&](auto both_tag) {
@@ -651,10 +701,11 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             ok = true;
 #pragma unroll
             for (int j = 0; j < kSlots; ++j) {
-                const int sp = lane + 64 * j;
+                const int sp = first + lane + 64 * j;
                 m_reg[j] = -INFINITY;
                 l_reg[j] = 0.0f;
-                if (sp < SA && sp != split) {
+                if (lane + 64 * j >= count) continue;
+                if (sp != split) {
                     const unsigned long long* rec = rec_near[j];
                     unsigned long long r0 = __hip_atomic_load(rec, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     unsigned long long r1 = __hip_atomic_load(rec + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -672,7 +723,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                     ok = ok && here;
                     m_reg[j] = __builtin_bit_cast(float, (uint32_t)(r0 >> 32));
                     l_reg[j] = __builtin_bit_cast(float, (uint32_t)(r1 >> 32));
-                } else if (sp == split) {
+                } else {
                     m_reg[j] = s_fin[2 * h];
                     l_reg[j] = s_fin[2 * h + 1];
                 }
@@ -701,18 +752,19 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     };
     // From the polled (max, sum) pairs: M = max m_s, the weights e^(m_s - M) into the head's row
     // of s_w, the denominator sum l_s * weight; the records are zeroed for the next use.
-    auto make_weights = [&](int h, auto slots, const float* m_reg, const float* l_reg, const bool* home) -> float {
+    auto make_weights = [&](int h, int first, int count, auto slots, const float* m_reg, const float* l_reg, const bool* home,
+                            float& mx) -> float {
         constexpr int kSlots = decltype(slots)::value;
         const WsHead wh = ws_head<BYSIDE>(a, kvh * a.group + h);
-        float mx = -INFINITY;
+        mx = -INFINITY;
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) mx = fmaxf(mx, m_reg[j]);
         mx = wave_max(mx);
         float den = 0.0f;
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) {
-            const int sp = lane + 64 * j;
-            if (sp < SA) {
+            const int sp = first + lane + 64 * j;
+            if (lane + 64 * j < count) {
                 const float f = (m_reg[j] == -INFINITY) ? 0.0f : fast_exp2(m_reg[j] - mx);
                 s_w[h * kMaxSplits + sp] = f;
                 den += l_reg[j] * f;
@@ -729,8 +781,9 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         constexpr int kSlots = decltype(slots)::value;
         float m_reg[kSlots], l_reg[kSlots];
         bool home[kSlots];  // (plain layout on this path: one home)
-        const bool arrived = wait_records(h, slots, m_reg, l_reg, home);
-        den_out = make_weights(h, slots, m_reg, l_reg, home);
+        const bool arrived = wait_records(h, 0, SA, slots, m_reg, l_reg, home);
+        float mx;
+        den_out = make_weights(h, 0, SA, slots, m_reg, l_reg, home, mx);
         return arrived;
     };
     auto poll_head = [&](int h, float& den_out) -> bool {
@@ -740,19 +793,27 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     const __amdgpu_buffer_rsrc_t ws_rsrc = part_rsrc;
     constexpr int kCoherent = kCacheDevice;
 
-    if (G <= NW || a.group <= NW) {  // (G, the group rounded up, decides it at compile time where it can)
+    if (G <= NW || a.group <= NW || spread) {  // (G, the group rounded up, decides it at compile time where it can)
         // One wavefront per head, all the way: poll, then read the head's partials back and write
         // its 128 outputs, without a workgroup barrier (a wave whose records are in need not wait
         // for the others). Lane = (16-byte column, half of the splits); the two halves are added
         // with one lane swap. The partials of the other workgroups were acknowledged before
         // their records were written; they are read with device-coherent 16-byte loads, a
         // lane's loads all in flight at once.
-        if (spread ? wave != 0 : wave >= a.group) return;
+        // With many splits (shapes of few KV heads: 64 to 256) the merging workgroup's wavefronts share them: each polls,
+        // weighs and reads back its own contiguous part, and wavefront 0 adds the parts up. One wavefront would read
+        // 32 rows per round trip, one round after the other: 16 Q / 2 KV heads (128 splits) 12.97 -> 11.68 us at 40001
+        // positions, 8 Q / 1 KV head (256 splits) 11.2 -> 7.7 at 12001, 18.8 -> 15.2 at 120001.
+        const bool wide = NW >= 4 && spread && SA > kWideMergeMin;
+        if (spread ? wave != 0 && !wide : wave >= a.group) return;
         const int h = spread ? merge_head : wave;
+        const int share = wide ? (SA + NW - 1) / NW : SA;  // (at most 64: 256 splits, four wavefronts)
+        const int first = wide ? wave * share : 0;
+        const int count = wide ? max(0, min(share, SA - first)) : SA;
         const int c4 = lane & 31;
         const int part = lane >> 5;
         const int hq = kvh * a.group + h;
-        const float* w = s_w + h * kMaxSplits;
+        const float* w = s_w + h * kMaxSplits + first;
         const WsHead wh = ws_head<BYSIDE>(a, hq);
         // Byte offset of split sp's partial row, in both layouts with the same few instructions: plain, it is
         // B = row * 512; by side, the row's pair of 8 KiB blocks starts at twice B's block start and the home adds 8 KiB
@@ -760,8 +821,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         const uint32_t row0_bytes = (uint32_t)wh.rbase * (kHeadDim * 4u);
         const uint32_t block_mask = BYSIDE ? ~(uint32_t)(kSideBlockBytes - 1) : 0u;
         const uint32_t lane_bytes = (uint32_t)c4 * 16u;
-        auto load_partial = [&](int sp, uint32_t home_bytes) {
-            const int spc = min(sp, SA - 1);  // in range; the weight drops the repeat
+        auto load_partial = [&](int sp, uint32_t home_bytes) {  // (sp counted from `first`)
+            const int spc = first + min(sp, count - 1);  // in range, a row whose record is in; the weight drops the repeat
             const uint32_t B = row0_bytes + (uint32_t)spc * (kHeadDim * 4u);
             return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ws_rsrc, B + (B & block_mask) + home_bytes + lane_bytes, 0, kCoherent));
         };
@@ -772,7 +833,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             constexpr int kBatch = decltype(batch)::value;
             float m_reg[kSlots], l_reg[kSlots];
             bool home[kSlots];
-            const bool arrived = wait_records(h, slots, m_reg, l_reg, home);
+            const bool arrived = wait_records(h, first, count, slots, m_reg, l_reg, home);
             // Which home each split's partial outputs are in: this side's, for all of them, when the workgroups of the KV
             // head share an XCD -- one constant. Otherwise (wave-uniform test) per split, from the polling lanes' flags.
             bool other = false;
@@ -780,7 +841,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             for (int j = 0; j < kSlots; ++j) other = other || home[j] != (my_xs != 0);
             const bool mixed = BYSIDE && __any(other);
             const uint32_t near_bytes = BYSIDE ? (uint32_t)(wh.ppar ^ my_xs) * kSideBlockBytes : 0u;
-            float den = 0.0f;
+            float den = 0.0f, mx = -INFINITY;
             // The read-back, once for the usual case (every split in this side's home: one constant, nothing between the
             // loads) and once for the other one: two copies of the code rather than a test in front of every load.
             auto gather = [&](auto mixed_tag) -> f32x4 {
@@ -789,7 +850,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                     // (the flag of split spc sits in lane spc % 64, slot spc / 64 of the polling layout: the slot's flags
                     // as a 64-bit lane mask, bit spc % 64 of it -- no shuffle, and no indexed array, which the compiler
                     // would put into scratch memory)
-                    const int spc = min(sp, SA - 1);
+                    const int spc = min(sp, max(count - 1, 0));
                     int xs = 0;
 #pragma unroll
                     for (int j = 0; j < kSlots; ++j) {
@@ -802,34 +863,63 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 f32x4 v[kBatch];
 #pragma unroll
                 for (int j = 0; j < kBatch; ++j) v[j] = load_partial(part + 2 * j, home_bytes(part + 2 * j));
-                den = make_weights(h, slots, m_reg, l_reg, home);
+                den = make_weights(h, first, count, slots, m_reg, l_reg, home, mx);
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own weights are in LDS
                 __builtin_amdgcn_wave_barrier();
                 f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int j = 0; j < kBatch; ++j) {
                     const int sp = part + 2 * j;
-                    sum += v[j] * (sp < SA ? w[sp] : 0.0f);
+                    sum += v[j] * (sp < count ? w[sp] : 0.0f);
                 }
-                for (int s0 = part + 2 * kBatch; s0 < SA; s0 += kBatch * 2) {
+                for (int s0 = part + 2 * kBatch; s0 < count; s0 += kBatch * 2) {
 #pragma unroll
                     for (int j = 0; j < kBatch; ++j) v[j] = load_partial(s0 + 2 * j, home_bytes(s0 + 2 * j));
 #pragma unroll
                     for (int j = 0; j < kBatch; ++j) {
                         const int sp = s0 + 2 * j;
-                        sum += v[j] * (sp < SA ? w[sp] : 0.0f);
+                        sum += v[j] * (sp < count ? w[sp] : 0.0f);
                     }
                 }
                 return sum;
             };
-            f32x4 acc;
-            if constexpr (BYSIDE) acc = __builtin_expect(mixed, 0) ? gather(std::true_type{}) : gather(std::false_type{});
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (wide && count == 0) {
+                // (fewer splits than the shares have room for: nothing to read)
+            } else if constexpr (BYSIDE) acc = __builtin_expect(mixed, 0) ? gather(std::true_type{}) : gather(std::false_type{});
             else acc = gather(std::false_type{});
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = halves_sum(acc[e]);
+            bool all_in = arrived;
+            if constexpr (NW >= 4 && !OPROJ) {
+                if (wide) {
+                    // (the epilogue's per-wavefront pairs have been read: their place takes the parts' maxima and sums)
+                    if (part == 0) s_part[wave * 32 + c4] = acc;
+                    if (lane == 0) {
+                        s_m[wave][0] = mx;
+                        s_l[wave][0] = den;
+                        s_ok[wave] = arrived ? 1 : 0;
+                    }
+                    __syncthreads();
+                    if (wave != 0) return;
+                    float top = -INFINITY;
+#pragma unroll
+                    for (int x = 0; x < NW; ++x) top = fmaxf(top, s_m[x][0]);
+                    acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    den = 0.0f;
+#pragma unroll
+                    for (int x = 0; x < NW; ++x) {
+                        const float mw = s_m[x][0];
+                        const float f = (mw == -INFINITY) ? 0.0f : fast_exp2(mw - top);
+                        acc += s_part[x * 32 + c4] * f;
+                        den += s_l[x][0] * f;
+                        all_in = all_in && s_ok[x] != 0;
+                    }
+                }
+            }
             if (part == 0) {
                 // A wait that ran out of patience poisons the output rather than returning a partial sum.
-                const float inv = arrived ? 1.0f / den : __builtin_nanf("");
+                const float inv = all_in ? 1.0f / den : __builtin_nanf("");
                 const f32x4 r = acc * inv;
                 const unsigned long long packed = (unsigned long long)pack_bf16(r[0], r[1]) | ((unsigned long long)pack_bf16(r[2], r[3]) << 32);
                 unsigned long long* op = reinterpret_cast<unsigned long long*>(a.out + (int64_t)hq * kHeadDim + c4 * 4);
@@ -868,9 +958,9 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 }
             }
         };
-        // (the dispatcher's own split counts stay below 64: the rare cases are kept out of the way of the usual ones)
-        if (__builtin_expect(SA > 64, 0)) run(std::integral_constant<int, kMaxSplits / 64>{}, std::integral_constant<int, 16>{});
-        else if (SA <= 16) run(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{});
+        // (a lane polls one split unless a single wavefront has more than 64: a rare case, kept out of the way of the usual ones)
+        if (__builtin_expect(count > 64, 0)) run(std::integral_constant<int, kMaxSplits / 64>{}, std::integral_constant<int, 16>{});
+        else if (count <= 16) run(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{});
         else run(std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
         return;
     }
