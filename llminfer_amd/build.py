@@ -10,6 +10,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libllmi_hip.so")
 HOST_LIB_PATH = os.path.join(HERE, "libllmi_host.so")
 DIAG_LIB_PATH = os.path.join(HERE, "libllmi_diag.so")
+TORCH_OPS_PATH = os.path.join(HERE, "_torch_ops.so")
 
 HIP_SOURCES = ["mha_decode_group4.hip", "mha_decode_group8.hip", "mha_decode_group16.hip", "mha_decode_group2.hip", "mha_decode_group1.hip", "mha_stack.hip",
                "mha_decode.hip", "qk_norm_rope.hip", "gemv.hip", "probes.hip", "c_api.cpp", "pool.cpp"]
@@ -117,8 +118,25 @@ def build_host_library(verbose=False):
     return HOST_LIB_PATH
 
 
+def build_torch_ops(verbose=False):
+    """_torch_ops.so: the native calls of llminfer_amd.ops (a CPython extension against the installed torch; no device code)."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    src = os.path.join(CSRC, "front", "torch_ops.cpp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-I" + os.path.join(ROOT, "include")]
+    for d in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", d]
+    cmd += [src, "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-o", TORCH_OPS_PATH]
+    out = _run(cmd)
+    if verbose and out.strip():
+        print(out)
+    return TORCH_OPS_PATH
+
+
 def build_all(verbose=False):
-    paths = [build_hip_library(verbose), build_diag_library(verbose)]
+    paths = [build_hip_library(verbose), build_diag_library(verbose), build_torch_ops(verbose)]
     host = build_host_library(verbose)
     if host:
         paths.append(host)
