@@ -236,7 +236,10 @@ typedef struct llmi_mha_stack_args {
  * In the one-launch form, layers that cannot see each other's writes do not wait for each other: if no address range that
  * the call writes (outputs, tap, the layers' caches, workspace; each from the first layer's first byte to the last layer's last
  * one) overlaps one it reads or another one it writes, and every layer has output rows of its own, the layers run as one
- * stream (same bits, less than half the time). The order described above holds wherever it can be observed. */
+ * stream (same bits, less than half the time). From 32 KV heads on (layers x KV heads) such layers are also taken a KV head at a time
+ * per workgroup where that is estimated to be faster: groups of up to 8 query heads, single passes and up to 32 splits, any workspace the
+ * per-layer launches accept; only heads that are cut for an even load wait for workgroups started before theirs, under the
+ * same bounded waits (a give-up turns that head's output into NaN). The order described above holds wherever it can be observed. */
 int llmi_hip_mha_decode_append_stack(const llmi_mha_stack_args* args);
 int llmi_hip_mha_stack_launches(const llmi_mha_stack_args* args);
 

@@ -12,7 +12,7 @@ HOST_LIB_PATH = os.path.join(HERE, "libllmi_host.so")
 DIAG_LIB_PATH = os.path.join(HERE, "libllmi_diag.so")
 TORCH_OPS_PATH = os.path.join(HERE, "_torch_ops.so")
 
-HIP_SOURCES = ["mha_decode_group4.hip", "mha_decode_group8.hip", "mha_decode_group16.hip", "mha_decode_group2.hip", "mha_decode_group1.hip", "mha_stack.hip",
+HIP_SOURCES = ["mha_decode_group4.hip", "mha_decode_group8.hip", "mha_decode_group16.hip", "mha_decode_group2.hip", "mha_decode_group1.hip", "mha_stack.hip", "mha_heads.hip",
                "mha_decode.hip", "qk_norm_rope.hip", "gemv.hip", "probes.hip", "c_api.cpp", "pool.cpp"]
 DIAG_SOURCES = ["diag_probes.hip"]
 

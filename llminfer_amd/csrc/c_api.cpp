@@ -545,9 +545,75 @@ static bool layers_are_independent(const llmi_mha_stack_args& st) {
     return L == 1 || st.output_stride >= dim || st.output_stride <= -dim;  // (each layer writes rows of its own)
 }
 
+// Whether the resident launch that walks the layers (mha_stack.hip) takes this shape.
+static bool resident_form(const llmi_mha_args& m, const llmi_mha_plan& plan) {
+    if (plan.path != LLMI_PATH_SPLIT_FUSED || plan.num_splits < 2 || plan.num_splits > 64) return false;
+    if (plan.group_pad > 4 || plan.waves_per_group != 4 || m.head_num > 64) return false;  // (one lane of the polling wavefront per head)
+    if (m.workspace_bytes < plan.workspace_needed + stack_workspace_extra(m.head_num)) return false;
+    // every workgroup must be resident at once: workgroups wait for each other
+    const int cus = compute_units();
+    if (cus <= 0 || (int64_t)(m.kv_dim / m.head_dim) * plan.num_splits > cus) return false;
+    // Lengths at which the per-layer launches stagger their walk stay with them: the resident kernel walks in step, so
+    // it would neither be as fast there nor give the same bits (the order of a split's tiles is the order of its sums).
+    if (!append_walks_in_step(m, plan)) return false;
+    return true;
+}
+
+// Fewest heads (layers x KV heads) that are worth the form that takes them one by one: fewer leave seven eighths of the chip idle.
+constexpr int kFewestHeads = 32;
+
+// Whether a KV head of a layer at a time per workgroup (mha_heads.hip) takes this shape and is the faster form.
+static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan, bool resident, HeadsForm* form) {
+    *form = HeadsForm{};
+    const llmi_mha_args& m = st.first.mha;
+    if (plan.path != LLMI_PATH_SINGLE_PASS && plan.path != LLMI_PATH_SPLIT_FUSED) return false;
+    if (plan.num_splits > 32 || plan.group_pad > 8 || !append_walks_in_step(m, plan)) return false;
+    // The kernel's streaming wavefronts take a split's tiles as the launch's would: as many of them, or a tile each.
+    const int tiles = (m.pos + kTile - 1) / kTile;
+    const int waves = plan.group_pad == 8 || plan.waves_per_group == 8 ? 8 : 4;
+    if (plan.waves_per_group != waves && !(plan.num_splits == 1 && plan.waves_per_group < waves && tiles <= plan.waves_per_group)) return false;
+    const int n_kv = m.kv_dim / m.head_dim;
+    const int cus = compute_units();
+    const int64_t heads = (int64_t)st.layer_count * n_kv;
+    if (cus <= 0 || heads > INT32_MAX / 64) return false;
+    if (heads < kFewestHeads) return false;
+    // What either side takes, in us (fitted to sweeps of 4 to 64 layers, 32 to 20000 positions, groups of 1 to 8; within a tenth
+    // mostly). Here a split costs a workgroup a fixed part (folding, the barrier) and its wavefronts' tiles, all of them share the
+    // memory's rate, and cut heads are handed over at the end: 8 layers at 2048 positions, 2 : 4 : 8 : 16 : 32 splits, 26.9 : 28.8 : 31.8 :
+    // 38.0 : 48.8 (four wavefronts), 27.3 : 28.4 : 31.3 : 38.2 : 62.9 (eight). Both sides near the line, this form : the other one: 36 layers
+    // of 32 Q heads at 4096 96 : 107, 30 at 3000 69 : 75, 24 at 4000 75 : 74, 28 at 2000 50 : 55, 16 at 2000 50 : 33, 10 of 16 Q heads at
+    // 600 16 : 17, 6 of 32 Q heads at 20000 89 : 81; groups of 8 (one launch per layer) 8 at 300 33 : 50, 4 at 6000 26 : 34.
+    const double head_bytes = 4.0 * m.pos * m.head_dim, rate = 6.4e6;
+    const int tiles_per_wave = ceil_div(std::max(ceil_div(tiles, plan.num_splits), 1), waves);
+    const double split_us = waves == 8 ? 0.8 + 1.2 * tiles_per_wave : 0.75 + 0.57 * tiles_per_wave;
+    const int64_t rounds = heads / cus;
+    const int rest = (int)(heads % cus);
+    auto phase = [&](double n_heads, double splits) { return std::max(n_heads * head_bytes / rate, splits * split_us) + 1.0; };
+    double best = 0.0;
+    for (int parts = 1; parts <= std::max(plan.num_splits, 1); parts *= 2) {
+        HeadsForm f{0, parts, parts > 1 ? rest : 0, waves};
+        const int64_t items = heads + (int64_t)f.cut_heads * (parts - 1);
+        f.grid = (int)std::min<int64_t>(items, cus);
+        if (parts > 1 && (rest == 0 || (int64_t)rest * parts > cus || f.grid % parts != 0)) continue;
+        if (heads_workspace(m, f, plan.num_splits) > (m.workspace ? m.workspace_bytes : 0)) continue;
+        double us = 4.0 + (double)rounds * phase(cus, plan.num_splits);
+        if (rest > 0) us += phase(rest, ceil_div(plan.num_splits, parts)) + (parts > 1 ? 3.0 : 0.0);
+        if (form->grid == 0 || us < best) {
+            best = us;
+            *form = f;
+        }
+    }
+    const double layer_us = n_kv * head_bytes / rate;
+    const int regions = resident ? stack_regions(m, plan, st.layer_count) : 0;
+    const double other = !resident     ? ((plan.num_splits > 1 ? 6.0 : 4.3) + layer_us) * st.layer_count
+                         : regions == 0 ? 4.0 + (4.5 + layer_us) * st.layer_count
+                                        : 4.0 + std::max(regions > 4 ? 1.45 : 1.85, layer_us + 0.35) * st.layer_count;
+    return best < 0.97 * other;
+}
+
 // Validates a multi-layer call and decides between the one-launch form (*one_launch = true, plan = layer 0's) and
 // one launch per layer.
-static int plan_stack(const llmi_mha_stack_args* args, llmi_mha_plan* plan, bool* one_launch) {
+static int plan_stack(const llmi_mha_stack_args* args, llmi_mha_plan* plan, bool* one_launch, bool* heads, HeadsForm* form) {
     if (!args) return LLMI_ERR_NULL_POINTER;
     const llmi_mha_append_args& ap = args->first;
     if (!ap.key_new || !ap.value_new || !ap.norm_weight || !ap.sin_cache || !ap.cos_cache) return LLMI_ERR_NULL_POINTER;
@@ -562,33 +628,32 @@ static int plan_stack(const llmi_mha_stack_args* args, llmi_mha_plan* plan, bool
         if (st % 8 != 0) return LLMI_ERR_ALIGNMENT;  // (every layer's rows stay 16-byte aligned)
     if ((int64_t)ap.mha.layer_id + args->layer_count > INT32_MAX) return LLMI_ERR_INVALID_ARG;
     if (int rc = make_plan(&ap.mha, plan, kMaxWaves, 1)) return rc;
-    *one_launch = false;
+    *one_launch = *heads = false;
     const llmi_mha_args& m = ap.mha;
     if (m.pos_device) return LLMI_OK;
-    if (plan->path != LLMI_PATH_SPLIT_FUSED || plan->num_splits < 2 || plan->num_splits > 64) return LLMI_OK;
-    if (plan->group_pad > 4 || plan->waves_per_group != 4 || m.head_num > 64) return LLMI_OK;  // (one lane of the polling wavefront per head)
-    if (m.workspace_bytes < plan->workspace_needed + stack_workspace_extra(m.head_num)) return LLMI_OK;
-    // every workgroup must be resident at once: workgroups wait for each other
-    const int cus = compute_units();
-    if (cus <= 0 || (int64_t)(m.kv_dim / m.head_dim) * plan->num_splits > cus) return LLMI_OK;
-    // Lengths at which the per-layer launches stagger their walk stay with them: the resident kernel walks in step, so
-    // it would neither be as fast there nor give the same bits (the order of a split's tiles is the order of its sums).
-    if (!append_walks_in_step(m, *plan)) return LLMI_OK;
-    *one_launch = true;
+    const bool resident = resident_form(m, *plan);
+    if (plan_heads(*args, *plan, resident, form) && layers_are_independent(*args)) {
+        *heads = true;
+        return LLMI_OK;
+    }
+    *one_launch = resident;
     return LLMI_OK;
 }
 
 int llmi_hip_mha_stack_launches(const llmi_mha_stack_args* args) {
     llmi_mha_plan plan;
-    bool one = false;
-    if (int rc = plan_stack(args, &plan, &one)) return rc;
-    return one ? 1 : args->layer_count;
+    bool one = false, heads = false;
+    HeadsForm form;
+    if (int rc = plan_stack(args, &plan, &one, &heads, &form)) return rc;
+    return one || heads ? 1 : args->layer_count;
 }
 
 int llmi_hip_mha_decode_append_stack(const llmi_mha_stack_args* args) {
     llmi_mha_plan plan;
-    bool one = false;
-    if (int rc = plan_stack(args, &plan, &one)) return rc;
+    bool one = false, heads = false;
+    HeadsForm form;
+    if (int rc = plan_stack(args, &plan, &one, &heads, &form)) return rc;
+    if (heads) return launch_mha_heads(*args, plan, form);
     if (one) return launch_mha_stack(*args, plan, layers_are_independent(*args));
     for (int32_t l = 0; l < args->layer_count; ++l) {
         llmi_mha_append_args a = args->first;

@@ -100,6 +100,17 @@ int launch_mha_decode(const llmi_mha_args& args, const llmi_mha_plan& plan, cons
 // The multi-layer launch (llmi_hip_mha_decode_append_stack in its one-launch form); `plan` is layer 0's.
 // `independent`: no layer reads anything another one writes, so the layers may run in any order.
 int launch_mha_stack(const llmi_mha_stack_args& st, const llmi_mha_plan& plan, bool independent);
+// Layers whose partial rows and records fit the workspace side by side in that launch, 0 if too few for layers that do not wait
+// for each other.
+int stack_regions(const llmi_mha_args& m, const llmi_mha_plan& plan, int layer_count);
+// The same call with a KV head of a layer at a time per workgroup (independent layers only): the last cut_heads of them in
+// `parts` parts each, `grid` workgroups (a multiple of parts), `waves` streaming wavefronts.
+struct HeadsForm {
+    int grid, parts, cut_heads, waves;
+};
+int launch_mha_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan, const HeadsForm& form);
+// Bytes of the workspace the parts hand their results over in.
+size_t heads_workspace(const llmi_mha_args& m, const HeadsForm& form, int num_splits);
 // Bytes the multi-layer launch keeps behind the fused combine's records (its "done" tags, with room to align them).
 size_t stack_workspace_extra(int head_num);
 // What the fused projection holds per wavefront: weight rows, and the widest attention output (elements).

@@ -109,7 +109,7 @@ int static_scratch(void** ptr, size_t* bytes) {
 int read_poll_timeouts(unsigned long long* count) {
     // (every translation unit that instantiates the kernels counts on its own device word)
     hipError_t (*const parts[])(unsigned int*) = {poll_timeouts_group1, poll_timeouts_group2, poll_timeouts_group4,
-                                                  poll_timeouts_group8, poll_timeouts_group16, poll_timeouts_stack};
+                                                  poll_timeouts_group8, poll_timeouts_group16, poll_timeouts_stack, poll_timeouts_heads};
     unsigned long long total = 0;
     for (auto part : parts) {
         unsigned int n = 0;
@@ -227,6 +227,18 @@ static int fill_kernel_args(const llmi_mha_args& args, const llmi_mha_plan& plan
 
 size_t stack_workspace_extra(int head_num) { return 256 + stack_done_bytes(head_num); }
 
+static size_t stack_region_bytes(const llmi_mha_args& m, const llmi_mha_plan& plan) {
+    return (fused_workspace(m.head_num, m.head_dim, plan.num_splits, false).bytes() + 255) & ~(size_t)255;
+}
+
+int stack_regions(const llmi_mha_args& m, const llmi_mha_plan& plan, int layer_count) {
+    const size_t tags = stack_workspace_extra(m.head_num);
+    size_t fit = m.workspace_bytes > tags ? (m.workspace_bytes - tags) / stack_region_bytes(m, plan) : 0;
+    if (fit > (size_t)stack_max_regions(m.head_num)) fit = stack_max_regions(m.head_num);
+    if (fit > (size_t)layer_count) fit = layer_count;
+    return fit >= 3 && plan.num_splits >= m.kv_mul ? (int)fit : 0;  // (a workgroup merges at most one head per layer)
+}
+
 int launch_mha_stack(const llmi_mha_stack_args& st, const llmi_mha_plan& plan_in, bool independent) {
     const llmi_mha_args& m = st.first.mha;
     llmi_mha_plan plan = plan_in;
@@ -235,15 +247,11 @@ int launch_mha_stack(const llmi_mha_stack_args& st, const llmi_mha_plan& plan_in
         // As many layers' partial rows and records in the workspace as fit: a layer is merged two layers and more behind the
         // stream. (Plain layout: what by-side saves is latency, which is hidden.) A workspace sized by
         // llmi_hip_mha_workspace_bytes has room for twice the splits of the longest context, by side: for three regions at least.
-        const size_t region = (fused_workspace(m.head_num, m.head_dim, plan.num_splits, false).bytes() + 255) & ~(size_t)255;
-        const size_t tags = stack_workspace_extra(m.head_num);
-        size_t fit = m.workspace_bytes > tags ? (m.workspace_bytes - tags) / region : 0;
-        if (fit > (size_t)stack_max_regions(m.head_num)) fit = stack_max_regions(m.head_num);
-        if (fit > (size_t)st.layer_count) fit = st.layer_count;
-        if (fit >= 3 && plan.num_splits >= m.kv_mul) {  // (a workgroup merges at most one head per layer)
+        const int fit = stack_regions(m, plan, st.layer_count);
+        if (fit > 0) {
             plan.workspace_side = 0;
-            sa.regions = (int32_t)fit;
-            sa.region_bytes = (int64_t)region;
+            sa.regions = fit;
+            sa.region_bytes = (int64_t)stack_region_bytes(m, plan);
         }
     }
     char* fused_end = nullptr;
@@ -261,6 +269,34 @@ int launch_mha_stack(const llmi_mha_stack_args& st, const llmi_mha_plan& plan_in
     sa.done = reinterpret_cast<uint32_t*>((reinterpret_cast<uintptr_t>(fused_end) + 255u) & ~(uintptr_t)255u);
     if (!launch_stack(sa, m.kv_dim / m.head_dim, plan.group_pad, plan.waves_per_group, static_cast<hipStream_t>(m.stream)))
         return LLMI_ERR_INVALID_ARG;
+    return check_launch();
+}
+
+size_t heads_workspace(const llmi_mha_args& m, const HeadsForm& form, int num_splits) {
+    const size_t pub_splits = (size_t)((form.parts - 1) * num_splits / form.parts);
+    return (size_t)form.cut_heads * m.kv_mul * pub_splits * (m.head_dim * sizeof(float) + 2 * sizeof(unsigned long long));
+}
+
+int launch_mha_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan_in, const HeadsForm& form) {
+    const llmi_mha_args& m = st.first.mha;
+    llmi_mha_plan plan = plan_in;
+    plan.workspace_side = 0;
+    HeadsArgs ha{};
+    char* fused_end = nullptr;
+    if (int rc = fill_kernel_args(m, plan, &st.first, nullptr, 1, &ha.st.a, &fused_end)) return rc;
+    ha.st.layers = st.layer_count;
+    ha.st.q_stride = st.query_stride;
+    ha.st.knew_stride = st.key_new_stride;
+    ha.st.vnew_stride = st.value_new_stride;
+    ha.st.normw_stride = st.norm_weight_stride;
+    ha.st.out_stride = st.output_stride;
+    ha.st.cache_stride = (int64_t)m.max_seq_len * m.kv_dim;
+    ha.n_kv = m.kv_dim / m.head_dim;
+    ha.parts = form.parts;
+    ha.cut_heads = form.cut_heads;
+    ha.pub_splits = (form.parts - 1) * plan.num_splits / form.parts;
+    ha.items = st.layer_count * ha.n_kv + form.cut_heads * (form.parts - 1);
+    launch_heads(ha, form.grid, plan.group_pad, form.waves, static_cast<hipStream_t>(m.stream));
     return check_launch();
 }
 

@@ -73,6 +73,19 @@ struct StackArgs {
     int32_t regions;
     int64_t region_bytes;
 };
+// The multi-layer kernel that takes a KV head of a layer at a time (mha_heads.hip). Items: the parts of the last cut_heads KV
+// heads (`parts` each), then the others whole.
+struct HeadsArgs {
+    StackArgs st;
+    int32_t n_kv;
+    int32_t items;
+    int32_t cut_heads, parts;
+    int32_t pub_splits;  // splits of a cut head that go through the workspace: those of all parts but the last
+};
+// `waves`: wavefronts that stream, 4 or 8 (groups of 8: 8).
+void launch_heads(const HeadsArgs& ha, int grid, int group_pad, int waves, hipStream_t stream);
+hipError_t poll_timeouts_heads(unsigned int* n);
+
 // Groups of 1, 2 or 4 query heads (padded), four wavefronts per workgroup; false otherwise.
 bool launch_stack(const StackArgs& sa, int n_kv, int group_pad, int waves, hipStream_t stream);
 size_t stack_done_bytes(int head_num);

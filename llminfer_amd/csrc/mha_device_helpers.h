@@ -295,6 +295,86 @@ __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, co
     *hi_p = u32x2{pack_bf16(oh[0], oh[1]), pack_bf16(oh[2], oh[3])};
 }
 
+// One tile of 16 positions into a wavefront's running softmax: q.K^T, online softmax, P^T.V on the matrix cores (the
+// probabilities as hi + lo bf16), for groups of G query heads. row0: the lane's first position in the split.
+template <int G>
+__device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4], int row0, int nrows, float scale_log2e,
+                                          float& m_run, float& l_run, f32x4 (&o)[8]) {
+    f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, r.k[j]), __builtin_bit_cast(bf16x8, qb[j]), c, 0, 0, 0);
+    float s[4];
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        s[e] = (row0 + e < nrows) ? c[e] * scale_log2e : -INFINITY;
+        tmax = fmaxf(tmax, s[e]);
+    }
+    tmax = rows_max(tmax);
+    const float m_new = fmaxf(m_run, tmax);
+    const float alpha = fast_exp2(m_run - m_new);
+    float p[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = fast_exp2(s[e] - m_new);
+    l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+    m_run = m_new;
+    const uint32_t p01 = pack_bf16(p[0], p[1]);
+    const uint32_t p23 = pack_bf16(p[2], p[3]);
+    const uint32_t q01 = pack_bf16(p[0] - bf16_lo(p01), p[1] - bf16_hi(p01));
+    const uint32_t q23 = pack_bf16(p[2] - bf16_lo(p23), p[3] - bf16_hi(p23));
+    if (__any(alpha != 1.0f)) {
+        static_for<0, 4>([&](auto rr) {
+            float ar;
+            if constexpr (G <= 4) ar = row_bcast<rr.value>(alpha);  // only row kg = 0 holds heads
+            else ar = row_bcast_per_row<rr.value>(alpha);           // DPP row k takes lane 4*k + r of its own row
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o[j][rr.value] *= ar;
+        });
+    }
+    const i16x4 pa = __builtin_bit_cast(i16x4, u32x2{p01, p23});
+    const i16x4 pb = __builtin_bit_cast(i16x4, u32x2{q01, q23});
+    i16x4 vb4[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+        const uint32_t b01 = __builtin_amdgcn_perm(r.v[1][j >> 1], r.v[0][j >> 1], sel);
+        const uint32_t b23 = __builtin_amdgcn_perm(r.v[3][j >> 1], r.v[2][j >> 1], sel);
+        vb4[j] = __builtin_bit_cast(i16x4, u32x2{b01, b23});
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, vb4[j], o[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pb, vb4[j], o[j], 0, 0, 0);
+}
+
+// A wavefront's running softmax of the new token alone: score q.k, weight 1, output = the V row. new_rows: its K row
+// (normalised and rotated, operand layout) and V row in LDS, 16-byte chunks.
+__device__ __forceinline__ void start_from_new_row(const u32x4* new_rows, const u32x4 (&qb)[4], int kg, int n16, float scale_log2e,
+                                                   u32x4 (&kf)[4], u32x4& vf, float& m_run, float& l_run, f32x4 (&o)[8]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kf[j] = new_rows[j * 4 + kg];
+    vf = new_rows[16 + n16];
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t qw = qb[j][c], kw = kf[j][c];  // (bit_cast straight from a vector element reads element 0)
+            dot = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, qw), __builtin_bit_cast(bf16x2, kw), dot, false);
+        }
+    dot = rows_sum(dot);
+    m_run = dot * scale_log2e;
+    l_run = kg == 0 ? 1.0f : 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t vw = vf[j >> 1];
+        const float vj = (j & 1) ? bf16_hi(vw) : bf16_lo(vw);
+        o[j] = f32x4{vj, vj, vj, vj};
+    }
+}
+
 }  // namespace
 }  // namespace llmi
 
