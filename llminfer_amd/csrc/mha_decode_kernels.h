@@ -115,10 +115,14 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         // the host's reciprocal. With the rule
         // but without these two 5.84 us per layer at 1100 positions and 9.44 at 8000, with them 5.72 and 9.26 (5.58 and 9.18 with
         // the position known to the host).
-        asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.row_stride), "s"(a.head_stride), "s"(a.group), "s"(a.num_splits),
+        asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.row_stride), "s"(a.head_stride), "s"(a.group), "s"(a.num_splits), "s"(a.seq_len),
                      "s"(a.dyn_single), "s"(a.dyn_half), "s"(a.dyn_quarter), "s"(a.dyn_magic[0]), "s"(a.dyn_magic[1]), "s"(a.dyn_magic[2]));
         if constexpr (APPEND) asm volatile("" ::"s"(a.norm_w), "s"(a.sin_cache), "s"(a.cos_cache), "s"(a.k_new), "s"(a.v_new));
-        seq_len = max(0, min(*a.pos_dev, a.seq_len - 1)) + 1;
+        // (constant address space: a scalar load, where the compiler, not knowing that nothing in the launch writes the position, takes a
+        // vector one and its longer way: 36 layers 209.8 -> 205.5 us at 1100 positions, 194.5 -> 192.9 at 300, 64 layers of 64 Q heads at 5000
+        // 532.0 -> 530.5. The query's request and the heads' addresses ahead of its arrival: level.)
+        const auto pos_dev = reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(a.pos_dev));
+        seq_len = max(0, min(*pos_dev, a.seq_len - 1)) + 1;
         const int tiles = (seq_len - (APPEND ? 1 : 0) + kTile - 1) / kTile;
         const bool few = tiles < a.dyn_half, medium = tiles <= 4 * a.dyn_half;
         n_active = few ? a.dyn_quarter : medium ? a.dyn_half : a.num_splits;
