@@ -11,6 +11,7 @@
 // variant build is picked up here too.
 #include <Python.h>
 
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
@@ -475,8 +476,16 @@ PyObject* bind(PyObject*, PyObject* args) {
     return PyLong_FromLong(LLMI_HIP_ABI_VERSION);
 }
 
+// What torch throws at a tensor without storage of its own (one under vmap, say) is a Python error, not the process's end.
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t, PyObject*)>
+PyObject* entry(PyObject* self, PyObject* const* args, Py_ssize_t n_args, PyObject* names) {
+    HANDLE_TH_ERRORS
+    return F(self, args, n_args, names);
+    END_HANDLE_TH_ERRORS
+}
+
 #define LLMI_METHOD(name, signature, doc) \
-    {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL | METH_KEYWORDS, #name signature "\n--\n\n" doc}
+    {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(entry<name>)), METH_FASTCALL | METH_KEYWORDS, #name signature "\n--\n\n" doc}
 
 PyMethodDef g_methods[] = {
     {"bind", bind, METH_VARARGS, "Hands over the C ABI's addresses and the Python side's helpers; returns the ABI version compiled in."},

@@ -35,6 +35,18 @@ def test_refused_arguments(call, error, text):
         call(_t())
 
 
+def test_tensors_without_storage_raise():
+    """Under vmap (over tensors that only claim to be the device's) torch refuses to give an address: an error like any other."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        x = torch.empty((4, 128), dtype=torch.bfloat16, device="cuda")
+        w = torch.empty((16, 128), dtype=torch.bfloat16, device="cuda")
+        with pytest.raises(RuntimeError, match="data pointer"):
+            torch.vmap(lambda row: ops.gemv(row, w, w[0, :16]))(x)
+        with pytest.raises(RuntimeError, match="data pointer"):
+            torch.vmap(lambda row: ops.mha_decode(None, None, None, None, None, pos_device=row, **SCALARS))(x)
+
+
 def test_signatures_are_the_documented_ones():
     sig = inspect.signature(ops.mha_decode_append)
     assert list(sig.parameters)[:10] == ["query_raw", "key_new", "value_new", "norm_weight", "sin_cache", "cos_cache", "key_cache",
