@@ -214,7 +214,7 @@ def run_gemv(args):
                                % (what, n, k)},
         "us_per_launch": round(us, 3),
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "gemv_kernel",
+                     "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "gemv_row_kernel",
                      "avg_launch_us": round(us, 3), "avg_launch_bytes": nbytes},
     }))
     return 0
