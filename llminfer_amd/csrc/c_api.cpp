@@ -242,8 +242,13 @@ static int make_plan(const llmi_mha_args* a, llmi_mha_plan* p, int wave_cap = kM
     if (path != LLMI_PATH_SINGLE_PASS) {
         const bool fused = path == LLMI_PATH_SPLIT_FUSED;
         // Four waves per workgroup; eight for groups of 8 query heads, where the wider
-        // merge pays (measured at 64 Q / 8 KV heads, ctx 4K..128K).
-        int auto_waves = (group_pad == 8 && wave_cap >= 8) ? 8 : 4;
+        // merge pays (measured at 64 Q / 8 KV heads, ctx 4K..128K). With one or two KV heads, so many splits of so few
+        // tiles, four are ahead there too, 8 : 4 waves: 16 Q / 2 KV heads 5.17 : 5.00 us at 700 positions, 6.23 : 6.00 at 3001,
+        // 8.05 : 7.65 at 12001, 11.8 : 11.3 at 40001, 20.2 : 19.9 at 100001; 8 Q / 1 KV head 6.28 : 5.82 at 3001, 7.71 : 7.37 at
+        // 12001, 13.8 : 13.6 at 100001. (Not the append variant: the multi-layer launch stands for its eight, and a forced
+        // split count keeps them.)
+        const bool few_heads = n_kv <= 2 && new_rows == 0 && a->num_splits == 0;
+        int auto_waves = (group_pad == 8 && wave_cap >= 8 && !few_heads) ? 8 : 4;
         if (auto_waves > max_waves) auto_waves = max_waves;
         waves = a->waves_per_group ? a->waves_per_group : auto_waves;
         int want = a->num_splits;

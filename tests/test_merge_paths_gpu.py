@@ -15,7 +15,9 @@ HEAD, POS = B.KV_LAYOUT_HEAD_MAJOR, B.KV_LAYOUT_POS_MAJOR
 
 
 @pytest.mark.parametrize("n_q,n_kv,ctx,layout,kw", [
-    (8, 1, 4500, HEAD, {}),                                                # 256 splits, eight wavefronts
+    (8, 1, 4500, HEAD, {}),                                                # 256 splits, four wavefronts for a group of 8
+    (8, 1, 4500, HEAD, dict(num_splits=256)),                              # ... eight
+    (14, 2, 517, POS, {}),                                                 # four wavefronts, 7 heads in a group
     (8, 2, 2100, POS, {}),                                                 # 128 splits, four wavefronts
     (16, 2, 1040, HEAD, dict(num_splits=65)),                              # the last wavefronts' shares are short or empty
     (4, 1, 4200, HEAD, dict(num_splits=250, waves_per_group=4)),           # 63 splits for each wavefront
