@@ -108,14 +108,41 @@ int poll_limit() { return g_poll_limit.load(std::memory_order_relaxed); }
 static std::atomic<int> g_test_far_home{0};
 int test_far_home() { return g_test_far_home.load(std::memory_order_relaxed); }
 
+// Compute units of the current device (asked once per process), or 0 if the device cannot be asked.
+static int compute_units() {
+    static std::atomic<int> cu_count{0};
+    int cus = cu_count.load(std::memory_order_relaxed);
+    if (cus == 0) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+            (void)hipGetLastError();
+            return 0;
+        }
+        cu_count.store(cus, std::memory_order_relaxed);
+    }
+    return cus;
+}
+
+// A spread merge's workgroups, one per query head, wait for each other and for every other split of their KV head, and a compute
+// unit may hold no more than one of them (the rings of a workgroup of four wavefronts and 16 heads are more than half of its
+// LDS). Handed out last, they must leave room for those that have not started, or the wait only ends at its limit: at most one
+// for every second compute unit, so that two launches on two streams have it too. Unlike them the last splits' workgroups of
+// the other merge, one per KV head, wait only for workgroups started before them.
+static bool spread_merge_fits(int head_num) {
+    const int cus = compute_units();
+    return head_num <= (cus > 0 ? cus : kTargetGroups) / 2;
+}
+
 // With 32 splits and more (16 for groups of eight query heads) the merge of a KV head's query heads is spread over as
 // many workgroups; with fewer, the workgroup of the last split merges them all. Measured, 32 Q / 8 KV heads, spread
 // against not: 16 splits 5.08 : 4.98 us at 1024 positions, 5.87 : 5.77 at 2048; 8 splits 4.51 : 4.41 at 256; 32 splits
 // 5.03 : 5.14 at 1024, 5.71 : 5.80 at 2048, 6.86 : 7.08 at 4096, 7.88 : 8.10 at 6000; 64 Q heads, 16 splits 5.55 : 5.68 at
 // 1024, 7.63 : 7.81 at 4096, 32 splits at 32768 24.4 : 25.3. Groups of 16 (four wavefronts): always, as soon as there is a
-// split for every head. LLMI_HIP_SPREAD_MIN_SPLITS moves the boundary.
-int spread_merge_min_splits(int group_pad) {
+// split for every head. LLMI_HIP_SPREAD_MIN_SPLITS moves the boundary. Never where the merging workgroups have no room to
+// wait in (spread_merge_fits).
+int spread_merge_min_splits(int group_pad, int head_num) {
     static const int v = env_int("LLMI_HIP_SPREAD_MIN_SPLITS", 1, 1 << 20, 0);
+    if (!spread_merge_fits(head_num)) return INT32_MAX;
     return v ? v : group_pad >= 16 ? 1 : group_pad >= 8 ? 16 : 32;
 }
 
@@ -161,17 +188,18 @@ int check_launch() { return record_hip_error(hipGetLastError(), "kernel launch")
 // 208 positions; at 256, where 16 splits have a tile each, 5.51 against 5.34).
 // Groups of more than 8 heads stay with it until there is a split per head to merge them (32 Q / 2 KV heads, single pass : 14 or
 // 17 splits: 6.1 : 9.5 us at 220 positions, 6.8 : 5.9 at 260, where the 17 can take a head each).
-static int single_pass_limit(int kv_mul, int group_pad, bool eight_waves) {
+// (Without room for that a workgroup merges all heads whatever the split count: the limit of the smaller groups.)
+static int single_pass_limit(int kv_mul, int group_pad, int head_num, bool eight_waves) {
     if (env_tuning().single_pass_max >= 0) return env_tuning().single_pass_max;
-    if (group_pad > 8) return kTile * kv_mul - 1 > kSinglePassMaxLen ? kTile * kv_mul - 1 : kSinglePassMaxLen;
+    if (group_pad > 8 && spread_merge_fits(head_num)) return kTile * kv_mul - 1 > kSinglePassMaxLen ? kTile * kv_mul - 1 : kSinglePassMaxLen;
     return group_pad == 8 && eight_waves ? 240 : kSinglePassMaxLen;
 }
 
 // Split counts below the full grid's: half of the workgroups, a quarter of them.
-// (Never fewer than heads in a group of more than 8: see single_pass_limit.)
-static int fewest_splits(int kv_mul) { return kv_mul > 8 ? kv_mul : 2; }
-static int half_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv, fewest_splits(kv_mul)); }
-static int quarter_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv / 2, fewest_splits(kv_mul)); }
+// (Never fewer than heads in a group of more than 8 whose merge is spread: see single_pass_limit.)
+static int fewest_splits(int n_kv, int kv_mul) { return kv_mul > 8 && spread_merge_fits(n_kv * kv_mul) ? kv_mul : 2; }
+static int half_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv, fewest_splits(n_kv, kv_mul)); }
+static int quarter_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv / 2, fewest_splits(n_kv, kv_mul)); }
 
 void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, int* single, int* quarter, int* half) {
     *single = *quarter = *half = 0;
@@ -180,7 +208,7 @@ void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, int* s
     // (the launch has the split path's waves: four, eight for groups of 8 heads. At four a single pass still is the faster one
     // up to the same length as at the eight that a launch planned for it would have: 4.34 : 4.51 us at 176 positions,
     // 4.96 : 4.67 at 220)
-    *single = single_pass_limit(args.kv_mul, plan.group_pad, plan.waves_per_group >= 8) / kTile;
+    *single = single_pass_limit(args.kv_mul, plan.group_pad, args.head_num, plan.waves_per_group >= 8) / kTile;
     // (no more than the launch has workgroups for)
     const int q = quarter_splits(n_kv, args.kv_mul), h = half_splits(n_kv, args.kv_mul);
     *quarter = q < plan.num_splits ? q : plan.num_splits;
@@ -227,7 +255,7 @@ static int make_plan(const llmi_mha_args* a, llmi_mha_plan* p, int wave_cap = kM
     const size_t per_split_fused = (size_t)a->head_num * (a->head_dim * sizeof(float) + 2 * sizeof(unsigned long long));
 
     const int single_waves_max = (max_waves < wave_cap ? max_waves : wave_cap);  // 8 where the kernel variant allows
-    const int single_pass_max = single_pass_limit(a->kv_mul, group_pad, wave_cap >= 8);
+    const int single_pass_max = single_pass_limit(a->kv_mul, group_pad, a->head_num, wave_cap >= 8);
     int path = a->force_path;
     if (path == LLMI_PATH_AUTO) {
         if (a->num_splits == 1) path = LLMI_PATH_SINGLE_PASS;
@@ -269,7 +297,7 @@ static int make_plan(const llmi_mha_args* a, llmi_mha_plan* p, int wave_cap = kM
             // traffic and lengthen the combine (64 splits: +1 us everywhere).
             // And no more splits than the caller's workspace can hold.
             int target = kTargetGroups / n_kv;
-            if (target < fewest_splits(a->kv_mul)) target = fewest_splits(a->kv_mul);
+            if (target < fewest_splits(n_kv, a->kv_mul)) target = fewest_splits(n_kv, a->kv_mul);
             if (target > kMaxSplits) target = kMaxSplits;
             const int half = half_splits(n_kv, a->kv_mul), quarter = quarter_splits(n_kv, a->kv_mul);
             // One workgroup per CU pays as soon as half as many splits would hold more than four tiles each (more than
@@ -415,21 +443,6 @@ int llmi_hip_mha_decode_append(const llmi_mha_append_args* args) {
     llmi_mha_plan plan;
     if (int rc = make_plan(&args->mha, &plan, kMaxWaves, 1)) return rc;
     return launch_mha_decode(args->mha, plan, args);
-}
-
-// Compute units of the current device (asked once per process), or 0 if the device cannot be asked.
-static int compute_units() {
-    static std::atomic<int> cu_count{0};
-    int cus = cu_count.load(std::memory_order_relaxed);
-    if (cus == 0) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-            (void)hipGetLastError();
-            return 0;
-        }
-        cu_count.store(cus, std::memory_order_relaxed);
-    }
-    return cus;
 }
 
 // Validates the arguments and decides between the one-launch form (*fused = true, plan filled) and the pair.
@@ -848,6 +861,8 @@ int llmi_hip_abi_version(void) { return LLMI_HIP_ABI_VERSION; }
 int32_t llmi_hip_set_test_far_home(int32_t mode) {
     return llmi::g_test_far_home.exchange(mode < 0 || mode > 2 ? 0 : mode, std::memory_order_relaxed);
 }
+
+int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t head_num) { return spread_merge_min_splits(pow2_ceil(kv_mul), head_num); }
 
 int32_t llmi_hip_stagger_mask(int32_t kv_layout, int64_t run_bytes, int32_t ragged) {
     return llmi::stagger_mask(kv_layout, run_bytes, ragged != 0);

@@ -658,12 +658,13 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
 
     // ---- fused combine ----
     // The workgroup of the LAST split of this KV head merges the partials of its
-    // query heads, so no second launch is needed. Every split publishes, per query
-    // head, a record {epoch | max} {epoch | sum} as soon as the head's partial outputs have
-    // been acknowledged; the last split's workgroup waits for all records but its own (it
+    // query heads, or (spread) those of the last splits a head each, so no second launch is needed. Every split publishes, per
+    // query head, a record {epoch | max} {epoch | sum} as soon as the head's partial outputs have
+    // been acknowledged; who merges a head waits for all its records but its own (it
     // has its own pair in LDS and its own partials acknowledged). Workgroups are
-    // dispatched in index order and the others never wait for anything, so whoever
-    // it waits for is already running or done.
+    // dispatched in index order and those that merge nothing never wait for anything, so the workgroup of the last split
+    // waits only for some that are running or done. The workgroups of a spread merge wait for each other too: the host asks for
+    // it only where all of them fit the chip with room to spare (spread_merge_fits).
     // A record carries the epoch of the call that wrote it; anything else (an
     // uninitialised workspace, an earlier call) reads as "not arrived", so the
     // workspace needs no clearing. The combiner zeroes the records again so that a

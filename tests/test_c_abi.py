@@ -416,6 +416,28 @@ def test_stagger_rule_of_the_split_path():
     assert run(LLMI_HIP_STAGGER_MASK="junk") == run()
 
 
+@pytest.mark.parametrize("pos", [100, 200, 250, 700, 2999, 40000])
+def test_workgroups_that_wait_for_each_other_leave_room(pos):
+    """A spread merge has a workgroup per query head wait for the other splits of its KV head; a compute unit may hold one of
+    them. So only up to 128 heads (of 256 units) are merged that way, with split counts to match; more take the last workgroup's
+    merge and the split counts of the smaller groups."""
+    spread_min = B.lib().llmi_hip_spread_min_splits
+    tiles = -(-(pos + 1) // 16)
+    for n_kv in (1, 2, 4, 7, 8, 9, 12, 14, 16, 20, 32, 40, 64, 200):
+        for kv_mul in (1, 2, 3, 4, 5, 8, 9, 12, 16):
+            heads = n_kv * kv_mul
+            rc, p = plan(good_args(head_num=heads, kv_mul=kv_mul, kv_dim=n_kv * 128, pos=pos, max_seq_len=65536, workspace_bytes=1 << 40))
+            fits = heads <= 128
+            assert rc == 0
+            assert spread_min(kv_mul, heads) == ((1 if kv_mul > 8 else 16 if kv_mul > 4 else 32) if fits else 2**31 - 1)
+            if fits:
+                continue
+            half = max(128 // n_kv, 2)
+            want = max(256 // n_kv, 2) if tiles >= 4 * half + 1 else half if tiles >= half else max(128 // n_kv // 2, 2)
+            single = pos + 1 <= (240 if 4 < kv_mul <= 8 else 176)
+            assert p.num_splits == (1 if single else min(want, tiles)), (n_kv, kv_mul)
+
+
 def test_side_decision_from_injected_timings():
     """The decision behind llmi_hip_mha_workspace_side as a pure function of the ping-pong probe's result words:
     clear cases, noise below the threshold, ties, pairs that lost a number or did not share an XCD, a side of the

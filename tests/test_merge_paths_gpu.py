@@ -8,6 +8,7 @@ from llminfer_amd import _binding as B
 from llminfer_amd import ops, synth
 
 from helpers import assert_parity, assert_tap_parity, from_dev_bf16, run_hip, run_oracle, to_dev
+from test_resident_stack_gpu import timeouts
 
 pytestmark = pytest.mark.gpu
 
@@ -43,7 +44,26 @@ def test_merges_of_many_splits_and_large_groups(oracle, dev, n_q, n_kv, ctx, lay
     assert_tap_parity(got32, ref, what)
 
 
+@pytest.mark.parametrize("n_q,n_kv,ctx,kw", [
+    (512, 32, 3000, {}), (320, 20, 1000, {}), (288, 32, 700, {}), (144, 9, 250, {}),
+    (288, 32, 700, dict(num_splits=16)),    # more splits than heads in the group
+    (256, 32, 2100, dict(num_splits=32)),   # groups of 8
+    (128, 8, 700, {}), (126, 9, 900, {}),   # the most heads that are merged a workgroup each
+])
+def test_many_heads_do_not_wait_for_each_other(oracle, dev, n_q, n_kv, ctx, kw):
+    """More query heads than half the compute units: no workgroup per head waits (the launch would not fit the chip)."""
+    case = synth.make_case(3 + n_q, n_q=n_q, n_kv=n_kv, ctx=ctx)
+    force = dict(force_path=B.PATH_SPLIT_FUSED) if kw else {}
+    before = timeouts()
+    got16, got32, plan = run_hip(case, dev, kv_layout=HEAD, want_plan=True, workspace_bytes=64 << 20, **force, **kw)
+    ref = run_oracle(oracle, case)
+    assert plan.num_splits > 1 and timeouts() == before
+    assert_parity(got16, ref, "splits %d" % plan.num_splits)
+    assert_tap_parity(got32, ref, "splits %d" % plan.num_splits)
+
+
 @pytest.mark.parametrize("n_q,n_kv,msl,layout,short_workspace", [
+    (288, 18, 1024, HEAD, False),   # more heads than may wait for each other: the counts of the smaller groups
     (32, 8, 4096, HEAD, False), (64, 8, 4096, POS, False), (32, 2, 4096, HEAD, False),
     (8, 1, 4096, HEAD, False),      # 256 splits and a reciprocal for each count
     (16, 8, 4096, HEAD, True),      # a workspace for 11 splits: every count is capped by it
@@ -66,7 +86,7 @@ def test_device_position_takes_the_planned_split_counts(oracle, dev, n_q, n_kv, 
     with torch.cuda.stream(stream):
         with torch.cuda.graph(g, stream=stream):
             ops.mha_decode(q, k, v, out, ws, stream=stream, **kw)
-    half = max(128 // n_kv, n_q // n_kv if n_q // n_kv > 8 else 2)
+    half = max(128 // n_kv, n_q // n_kv if n_q // n_kv > 8 and n_q <= 128 else 2)
     edges = [11 * 16, 12 * 16, 15 * 16, 16 * 16, 16 * half, 16 * (4 * half), 16 * (256 // n_kv)]
     lengths = sorted({1, 2, 16, 17, 100, 777, msl - 1, msl} | {e + d for e in edges for d in (-16, -1, 0, 1, 16)})
     for n in [x for x in lengths if 0 < x <= msl]:
