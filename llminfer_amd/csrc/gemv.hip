@@ -103,27 +103,56 @@ __global__ __launch_bounds__(W * 64) void gemv_row_kernel(GemvArgs a) {
     if (lane == 0) write_row(a, row, acc);
 }
 
-// Longer rows: kMaxSteps steps at a time.
+// Longer rows, of any step count: the same window, its steps in a ring of registers. Graph replays over distinct matrices, batches
+// of four steps (each waited for) : twenty at a time and the rest one by one : the ring, us and TB/s of the latter:
+//   2560 x 12288   11.3 : 13.1 : 11.4 (5.5)   5120 x 13824   24.8 : 25.5 : 23.0 (6.2)   5120 x 17408  30.6 : 32.2 : 29.4 (6.1)
+//   5120 x 25600   44.1 : 46.1 : 41.7 (6.3)   8192 x 28672   73.6 : 82.5 : 70.0 (6.7)   1000 x 11008  7.39 : 7.73 : 6.20 (3.6)
+//   500 x 53248    18.8 : 20.7 : 12.8 (4.2)   16384 x 16384  82.7 : 84.5 : 80.4 (6.7)
 template <int W>
 __global__ __launch_bounds__(W * 64) void gemv_long_row_kernel(GemvArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = blockIdx.x * W + wave;
     if (row >= a.n) return;
-    const u32x4* x4 = reinterpret_cast<const u32x4*>(a.x);
-    const u32x4* w4 = reinterpret_cast<const u32x4*>(a.w) + (int64_t)row * a.k8;
+    const u32x4* x4 = reinterpret_cast<const u32x4*>(a.x) + lane;
+    const u32x4* w4 = reinterpret_cast<const u32x4*>(a.w) + (int64_t)row * a.k8 + lane;
+    const int whole = a.k8 >> 6;  // steps all lanes have (kMaxSteps or more)
+    u32x4 wv[kWindow], xv[kWindow];
+    auto request = [&](int u) {  // (the first of the steps not asked for yet, into place u)
+        xv[u] = *x4;
+        wv[u] = __builtin_nontemporal_load(w4);
+        x4 += 64;
+        w4 += 64;
+    };
     float acc = 0.0f;
-    int c = lane;
-    for (; c + 64 * (kMaxSteps - 1) < a.k8; c += 64 * kMaxSteps) {
-        u32x4 wv[kMaxSteps], xv[kMaxSteps];
 #pragma unroll
-        for (int s = 0; s < kMaxSteps; ++s) wv[s] = __builtin_nontemporal_load(w4 + c + 64 * s);
-#pragma unroll
-        for (int s = 0; s < kMaxSteps; ++s) xv[s] = x4[c + 64 * s];
-#pragma unroll
-        for (int s = 0; s < kMaxSteps; ++s) acc = dot8_bf16(xv[s], wv[s], acc);
+    for (int u = 0; u < kWindow; ++u) {
+        request(u);
+        asm volatile("" ::: "memory");
     }
-    for (; c < a.k8; c += 64) acc = dot8_bf16(x4[c], __builtin_nontemporal_load(w4 + c), acc);
+    int asked = kWindow;
+    for (; asked + kWindow <= whole; asked += kWindow) {
+#pragma unroll
+        for (int u = 0; u < kWindow; ++u) {
+            acc = dot8_bf16(xv[u], wv[u], acc);
+            asm volatile("" : "+v"(acc)::"memory");
+            request(u);
+            asm volatile("" ::: "memory");
+        }
+    }
+    // What is left to ask for: fewer whole steps than places, and a part of one.
+    const int left = whole - asked;
+    const bool part = lane < (a.k8 & 63);
+#pragma unroll
+    for (int u = 0; u < kWindow; ++u) {
+        acc = dot8_bf16(xv[u], wv[u], acc);
+        asm volatile("" : "+v"(acc)::"memory");
+        xv[u] = wv[u] = u32x4{0u, 0u, 0u, 0u};
+        if (u < left || (u == left && part)) request(u);
+        asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int u = 0; u < kWindow; ++u) acc = dot8_bf16(xv[u], wv[u], acc);
     acc = wave_sum(acc);
     if (lane == 0) write_row(a, row, acc);
 }

@@ -13,7 +13,7 @@ from test_gemv_gpu import _case, _gate
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("k", [8, 512, 520] + [512 * s + d for s in range(2, 20) for d in (0, 8)] + [10232, 10240, 10248, 20480, 20488, 21000])
+@pytest.mark.parametrize("k", [8, 512, 520] + [512 * s + d for s in range(2, 20) for d in (0, 8)] + [10232, 10240, 10248] + [512 * s + d for s in range(21, 34) for d in (-8, 0, 8)] + [21000])
 def test_every_step_count(oracle, dev, k):
     n = 7
     x, w, sumabs = _case(k, n, k)
