@@ -33,7 +33,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kMaxSteps = 20;  // longest row, in steps, with a kernel of its own
-constexpr int kWindow = 6;     // steps ahead in longer rows than 8 steps
+constexpr int kWindow = 6;     // steps ahead in longer rows than 8 steps, unless launch_rows says otherwise
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __builtin_bit_cast(float, (uint32_t)h << 16); }
 
@@ -65,8 +65,8 @@ __device__ __forceinline__ void write_row(const GemvArgs& a, int row, float sum)
     }
 }
 
-// Rows of (S - 1, S] steps, W wavefronts per workgroup: kWindow steps (weights and input) ahead of the one being added.
-template <int S, int W>
+// Rows of (S - 1, S] steps, W wavefronts per workgroup: WINDOW steps (weights and input) ahead of the one being added.
+template <int S, int W, int WINDOW>
 __global__ __launch_bounds__(W * 64) void gemv_row_kernel(GemvArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(W * 64) void gemv_row_kernel(GemvArgs a) {
     if (row >= a.n) return;
     const u32x4* x4 = reinterpret_cast<const u32x4*>(a.x) + lane;
     const u32x4* w4 = reinterpret_cast<const u32x4*>(a.w) + (int64_t)row * a.k8 + lane;
-    constexpr int kAhead = S <= kWindow + 2 ? S : kWindow;
+    constexpr int kAhead = S <= WINDOW + 2 ? S : WINDOW;
     u32x4 wv[S], xv[S];
     auto request = [&](int s) {
         xv[s] = wv[s] = u32x4{0u, 0u, 0u, 0u};
@@ -162,20 +162,82 @@ __global__ __launch_bounds__(W * 64) void gemv_long_row_kernel(GemvArgs a) {
 // 109.9 : 109.5 at 152000 x 2560, level at 6144 x 2560; 4.83 : 5.09 at 2560 x 4096, 9.13 : 9.54 at 2560 x 9728, 14.0 : 14.3 at 5120 x 8192.
 constexpr int kRowsForFour = 6144;
 
+// More than two and up to five workgroups of two rows on each of 256 compute units is where the window gains least, and where rows start
+// a multiple of 4 KiB apart it loses: k a multiple of 2048, at which batches of four have no remainder. us, batches of four : windows
+// of 4 : 6 : 10:
+//   1000 x 6144  4.27 : 4.05 : 3.89 : 3.93    1000 x 8192   4.92 : 4.65 : 4.43 : 4.70    1000 x 10240  5.61 : 5.23 : 5.12 : 5.26
+//   1500 x 6144  4.69 : 4.65 : 4.86 : 4.70    1500 x 10240  6.35 : 6.29 : 6.45 : 6.52    1500 x 7000   5.82 : 5.23 : 5.36 : 5.40
+//   2560 x 6144  6.49 : 6.71 : 6.69 : 6.52    2560 x 10240  9.56 : 10.03 : 9.73 : 9.49   2560 x 12288 (ring) 10.8 : - : 11.5
+//   2600 x 6144, of the batches' time, 0.94 : 0.92 : 0.88     4000 x 10240  14.5 : 13.9 : 13.6 : 13.6
+// So batches there, but for sixteen steps up to 2048 rows, where six ahead is level or better (1500 x 8192 5.80 : 5.71 : 5.66 : 5.73, but 2300 x
+// 8192, of the batches' time, 1.05 : 1.03 : 1.02). With three wavefronts on a SIMD (from 2049 rows on) the other lengths want ten steps ahead: 2560 x 8704 8.84 : 8.92 :
+// 8.99 : 8.55, 2300 x 9728, of the batches' time, 1.00 : 0.97 : 0.94.
+constexpr int kRowsOfTwo = 1024, kRowsOfFour = 2048, kRowsOfFive = 2560;
+// Eight steps, otherwise asked for at once (71 registers: a wavefront less per SIMD than the window of four's 44), are a window of four where
+// rows start 4 KiB apart and are many. Batches : window of 4 : at once, us: 151936 x 4096 175.3 : 174.7 : 178.2, 60000 rows 69.9 : 69.6 : 70.7,
+// 20000 25.1 : 24.9 : 24.8.
+constexpr int kManyRows = 24576;
+
+// Rows of whole batches of four steps, each batch waited for before the next is asked for (when: see launch_rows).
+__global__ __launch_bounds__(2 * 64) void gemv_batch_kernel(GemvArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = blockIdx.x * 2 + wave;
+    if (row >= a.n) return;
+    const u32x4* x4 = reinterpret_cast<const u32x4*>(a.x);
+    const u32x4* w4 = reinterpret_cast<const u32x4*>(a.w) + (int64_t)row * a.k8;
+    float acc = 0.0f;
+    for (int c = lane; c < a.k8; c += 64 * 4) {
+        u32x4 xv[4], wv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            xv[u] = x4[c + 64 * u];
+            wv[u] = __builtin_nontemporal_load(w4 + c + 64 * u);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = dot8_bf16(xv[u], wv[u], acc);
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) write_row(a, row, acc);
+}
+
+template <int S, int W, int WINDOW>
+void launch_row_kernel(const GemvArgs& a, hipStream_t stream) {
+    hipLaunchKernelGGL((gemv_row_kernel<S, W, WINDOW>), dim3((a.n + W - 1) / W), dim3(W * 64), 0, stream, a);
+}
+
+#define LLMI_GEMV_STEPS(S, WINDOW) \
+    case S: return launch_row_kernel<S, W, WINDOW>(a, stream);
+
 template <int W>
 void launch_rows(const GemvArgs& a, hipStream_t stream) {
-    const dim3 grid((a.n + W - 1) / W), block(W * 64);
-    switch ((a.k8 + 63) / 64) {
-#define LLMI_GEMV_STEPS(S) \
-    case S: hipLaunchKernelGGL((gemv_row_kernel<S, W>), grid, block, 0, stream, a); break;
-        LLMI_GEMV_STEPS(1) LLMI_GEMV_STEPS(2) LLMI_GEMV_STEPS(3) LLMI_GEMV_STEPS(4) LLMI_GEMV_STEPS(5)
-        LLMI_GEMV_STEPS(6) LLMI_GEMV_STEPS(7) LLMI_GEMV_STEPS(8) LLMI_GEMV_STEPS(9) LLMI_GEMV_STEPS(10)
-        LLMI_GEMV_STEPS(11) LLMI_GEMV_STEPS(12) LLMI_GEMV_STEPS(13) LLMI_GEMV_STEPS(14) LLMI_GEMV_STEPS(15)
-        LLMI_GEMV_STEPS(16) LLMI_GEMV_STEPS(17) LLMI_GEMV_STEPS(18) LLMI_GEMV_STEPS(19) LLMI_GEMV_STEPS(20)
-#undef LLMI_GEMV_STEPS
-        default: hipLaunchKernelGGL((gemv_long_row_kernel<W>), grid, block, 0, stream, a);
+    const int steps = (a.k8 + 63) / 64;
+    const bool apart_4k = a.k8 % 256 == 0;
+    if constexpr (W == 2) {
+        if (apart_4k && steps > 8 && a.n > kRowsOfTwo && a.n <= kRowsOfFive && !(steps == 16 && a.n <= kRowsOfFour)) {
+            hipLaunchKernelGGL(gemv_batch_kernel, dim3((a.n + 1) / 2), dim3(2 * 64), 0, stream, a);
+            return;
+        }
+        if (a.n > kRowsOfFour && a.n <= kRowsOfFive) {
+            switch (steps) {
+                LLMI_GEMV_STEPS(9, 10) LLMI_GEMV_STEPS(10, 10) LLMI_GEMV_STEPS(11, 10) LLMI_GEMV_STEPS(12, 10) LLMI_GEMV_STEPS(13, 10)
+                LLMI_GEMV_STEPS(14, 10) LLMI_GEMV_STEPS(15, 10) LLMI_GEMV_STEPS(16, 10) LLMI_GEMV_STEPS(17, 10) LLMI_GEMV_STEPS(18, 10)
+                LLMI_GEMV_STEPS(19, 10) LLMI_GEMV_STEPS(20, 10)
+            }
+        }
+    } else if (apart_4k && steps == 8 && a.n >= kManyRows) {
+        return launch_row_kernel<8, W, 4>(a, stream);
+    }
+    switch (steps) {
+        LLMI_GEMV_STEPS(1, kWindow) LLMI_GEMV_STEPS(2, kWindow) LLMI_GEMV_STEPS(3, kWindow) LLMI_GEMV_STEPS(4, kWindow)
+        LLMI_GEMV_STEPS(5, kWindow) LLMI_GEMV_STEPS(6, kWindow) LLMI_GEMV_STEPS(7, kWindow) LLMI_GEMV_STEPS(8, kWindow)
+        LLMI_GEMV_STEPS(9, kWindow) LLMI_GEMV_STEPS(10, kWindow) LLMI_GEMV_STEPS(11, kWindow) LLMI_GEMV_STEPS(12, kWindow)
+        LLMI_GEMV_STEPS(13, kWindow) LLMI_GEMV_STEPS(14, kWindow) LLMI_GEMV_STEPS(15, kWindow) LLMI_GEMV_STEPS(16, kWindow)
+        LLMI_GEMV_STEPS(17, kWindow) LLMI_GEMV_STEPS(18, kWindow) LLMI_GEMV_STEPS(19, kWindow) LLMI_GEMV_STEPS(20, kWindow)
+        default: hipLaunchKernelGGL((gemv_long_row_kernel<W>), dim3((a.n + W - 1) / W), dim3(W * 64), 0, stream, a);
     }
 }
+#undef LLMI_GEMV_STEPS
 
 }  // namespace
 

@@ -35,3 +35,10 @@ def test_row_counts(oracle, dev, n, k):
     got = out.cpu().numpy()
     _gate(got[:n], oracle.gemv_bf16(x, w), sumabs, False, "n = %d" % n)
     assert np.all(np.isnan(got[n:]))  # nothing written past the last row
+
+
+@pytest.mark.parametrize("n,k", [(n, k) for n in (1024, 1025, 2048, 2049, 2560, 2561) for k in (4096, 4104, 6144, 6152, 8192, 10232, 10240, 12288, 12296)] +
+                         [(24575, 4096), (24576, 4096), (24577, 4088)])
+def test_kernels_by_row_count(oracle, dev, n, k):
+    """Batches of four, windows of four and ten, on either side of the row counts between them."""
+    test_row_counts(oracle, dev, n, k)
