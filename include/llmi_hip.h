@@ -228,17 +228,19 @@ typedef struct llmi_mha_stack_args {
  * the layer before has published a "done" tag behind its acknowledged output. Workgroups wait for other workgroups of
  * the same launch there, so every workgroup of the grid has to be resident at once: call this only on a GPU that runs
  * nothing else at the time. Every wait is bounded (llmi_hip_set_poll_limit); one that gives up is counted
- * (llmi_hip_poll_timeouts) and turns the outputs of its layer and the following ones into NaN. The one-launch form
+ * (llmi_hip_poll_timeouts) and turns what depends on it into NaN: a wait for the layer before (or, below, for room in the
+ * workspace) the outputs of its workgroup's KV head in that layer and all following ones, a wait for a head's partial results
+ * that head's output; every other output is right. The one-launch form
  * needs: the fused split path with 2..64 splits and a host-side position, a query group of at most 4 heads, a grid no
  * larger than the device's compute unit count, and a workspace sized by llmi_hip_mha_workspace_bytes (the plan's need
- * plus 4.3 KiB for the tags). Anything else runs as layer_count launches of llmi_hip_mha_decode_append.
+ * plus 4.3 KiB for the tags). Other shapes run as layer_count launches of llmi_hip_mha_decode_append, except as said below.
  * llmi_hip_mha_stack_launches tells which: 1 or layer_count (or a negative status for invalid arguments).
- * In the one-launch form, layers that cannot see each other's writes do not wait for each other: if no address range that
+ * Layers that cannot see each other's writes do not wait for each other: if no address range that
  * the call writes (outputs, tap, the layers' caches, workspace; each from the first layer's first byte to the last layer's last
  * one) overlaps one it reads or another one it writes, and every layer has output rows of its own, the layers run as one
  * stream (same bits, less than half the time). From 32 KV heads on (layers x KV heads) such layers are also taken a KV head at a time
- * per workgroup where that is estimated to be faster: groups of up to 8 query heads, single passes and up to 32 splits, any workspace the
- * per-layer launches accept; only heads that are cut for an even load wait for workgroups started before theirs, under the
+ * per workgroup where that is estimated to be faster, one launch too: groups of up to 8 query heads, single passes and up to 32 splits, any
+ * workspace the per-layer launches accept; only heads that are cut for an even load wait for workgroups started before theirs, under the
  * same bounded waits (a give-up turns that head's output into NaN). The order described above holds wherever it can be observed. */
 int llmi_hip_mha_decode_append_stack(const llmi_mha_stack_args* args);
 int llmi_hip_mha_stack_launches(const llmi_mha_stack_args* args);

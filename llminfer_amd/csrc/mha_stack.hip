@@ -357,7 +357,8 @@ __global__ __launch_bounds__(NW * 64, 2) void mha_stack_kernel(StackArgs sa) {
                 lsum += lw[w] * f;
             }
             if (poisoned) lsum = __builtin_nanf("");
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), part_rsrc, u_po, 0, kCacheDevice);
+            // (after a give-up the layer before may not have been read back: its rows stay, and the record's NaN is all of this one)
+            else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), part_rsrc, u_po, 0, kCacheDevice);
             if (!u_own) {
                 // the head's record goes out as soon as this wavefront's stores are acknowledged (the 32 columns of a
                 // head are stored by one half of one wavefront)
@@ -760,7 +761,9 @@ __global__ __launch_bounds__(kLayersWaves * 64, 2) void mha_layers_kernel(StackA
                 }
                 next_check += step;
             }
-            if (active)
+            // (after a give-up the layer that had the region may not have been read back: its rows stay, and the record's NaN is all
+            // of this one)
+            if (active && !poisoned)
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), part_rsrc,
                                                        po + (uint32_t)region * (uint32_t)sa.region_bytes, 0, kCacheDevice);
             prev_m = mx;

@@ -206,6 +206,39 @@ def test_resident_stack_gives_up_with_nan_instead_of_hanging(dev):
     assert torch.equal(c["out"], a["out"]) and timeouts() == after
 
 
+@pytest.mark.parametrize("layers,ctx,n_q,chained,regions", [
+    (12, 2000, 32, True, None), (9, 1000, 16, True, None),           # a layer waits for the one before
+    (14, 2000, 32, False, 5), (16, 2000, 32, False, 3), (16, 2000, 32, False, 9),  # ... for room in the workspace
+])
+def test_a_wait_that_gives_up_spoils_nothing_else(dev, layers, ctx, n_q, chained, regions):
+    """With limits of a few polls some waits give up and some do not. Whoever gives up runs on beside those that are still merging the
+    layer before out of the same place in the workspace: a head's output is NaN throughout or has the right bits, in every layer."""
+    from test_independent_layers_gpu import _workspace_for
+    st = Stack(dev, layers, ctx, n_q=n_q, chained=chained, seed=41)
+    a = st.fresh()
+    st.run_per_layer(a)
+    want = a["out"][:layers * st.dim].view(layers, n_q, D)
+    full = st.ws
+    if regions is not None:
+        st.ws = _workspace_for(st, 32, regions)
+    for limit in (0, 1, 2, 3, 5, 8, 20, 60):
+        prev = B.lib().llmi_hip_set_poll_limit(limit)
+        try:
+            b = st.fresh()
+            assert st.run_stack(b) == 1
+        finally:
+            assert B.lib().llmi_hip_set_poll_limit(prev) == limit
+        got = b["out"][:layers * st.dim].view(layers, n_q, D)
+        right = (got == want).all(-1)
+        nan = torch.isnan(got.view(torch.bfloat16)).all(-1)
+        assert bool((right | nan).all()), "limit %d: %s" % (limit, torch.nonzero(~(right | nan))[:8].tolist())
+        assert limit > 0 or bool(nan[1:].all())
+    st.ws = full
+    c = st.fresh()
+    assert st.run_stack(c) == 1
+    assert torch.equal(c["out"], a["out"])
+
+
 def test_resident_stack_falls_back_to_one_launch_per_layer(dev):
     """Shapes the resident kernel is not built for run as one launch per layer, with the same results: a single pass
     (short context), groups of eight query heads, more splits than compute units, a length at which the per-layer launches
