@@ -105,7 +105,8 @@ def timeouts():
 ])
 def test_resident_stack_equals_one_launch_per_layer(oracle, dev, layers, ctx, n_q, layout, over):
     """One resident launch for all layers against one launch per layer on the same inputs: same outputs and same
-    appended cache rows, bit for bit; the outputs also against the oracle. Twice in a row on one workspace."""
+    appended cache rows, bit for bit; the outputs also against the oracle. Twice in a row on one workspace. (The buffers are
+    separate: more than one layer runs as a stream, a single one as the chain.)"""
     st = Stack(dev, layers, ctx, n_q=n_q, layout=layout)
     a = st.fresh()
     st.run_per_layer(a, **over)
@@ -123,8 +124,8 @@ def test_resident_stack_equals_one_launch_per_layer(oracle, dev, layers, ctx, n_
 
 def test_resident_stack_qwen3_4b_36_layers_at_4096(oracle, dev):
     """BASELINE config 4 at its full size through the one-launch form: 36 layers at 4096 cached positions + 1 new token,
-    32 Q / 8 KV heads, by-side workspace as an engine would set it up. Bits of the per-layer launches, oracle parity on a
-    sample of layers, and replays of a captured graph with eager work in between."""
+    32 Q / 8 KV heads, by-side workspace as an engine would set it up (layers that are independent use it in the plain layout).
+    Bits of the per-layer launches, oracle parity on a sample of layers, and replays of a captured graph with eager work in between."""
     st = Stack(dev, 36, 4096)
     side = ops.workspace_side(st.ws) or 0x55555555
     st.ws.fill_(float("nan"))
@@ -182,12 +183,50 @@ def test_resident_stack_honours_the_order_between_layers(dev, layers, ctx, layou
         assert torch.equal(c["q"], a["q"]), "replay %d" % rep
 
 
-def test_resident_stack_gives_up_with_nan_instead_of_hanging(dev):
+@pytest.mark.parametrize("layers,ctx,n_q,layout,over", [
+    (5, 700, 8, B.KV_LAYOUT_HEAD_MAJOR, {}),                     # one query head per KV head
+    (5, 1000, 16, B.KV_LAYOUT_POS_MAJOR, {}),                    # two
+    (4, 2500, 24, B.KV_LAYOUT_HEAD_MAJOR, {}),                   # three, padded to four
+    (3, 2500, 32, B.KV_LAYOUT_POS_MAJOR, {"num_splits": 7, "force_path": B.PATH_SPLIT_FUSED}),
+    (3, 700, 32, B.KV_LAYOUT_HEAD_MAJOR, {"num_splits": 3, "force_path": B.PATH_SPLIT_FUSED}),  # fewer splits than heads: the last one merges
+])
+@pytest.mark.parametrize("side", [0, "measure", 0x55555555])
+def test_chained_layers_equal_one_launch_per_layer(dev, layers, ctx, n_q, layout, over, side):
+    """Layers that read the outputs of the ones before, so that the launch walks them as a chain: every padded group, plain and by-side
+    workspaces. Same outputs and cache rows as one launch per layer; two calls on one workspace, and replays."""
+    st = Stack(dev, layers, ctx, n_q=n_q, layout=layout, chained=True, seed=5)
+    if side == "measure":
+        side = ops.workspace_side(st.ws) or 0x66666666
+        st.ws.fill_(float("nan"))
+    over = dict(over, workspace_side=side)
+    a = st.fresh()
+    st.run_per_layer(a, **over)
+    before = timeouts()
+    for call in range(2):
+        b = st.fresh()
+        assert st.run_stack(b, **over) == 1
+        assert torch.equal(b["q"], a["q"]) and torch.equal(b["k"], a["k"]) and torch.equal(b["v"], a["v"]), "call %d" % call
+    stream, g, c = torch.cuda.Stream(), torch.cuda.CUDAGraph(), st.fresh()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(g, stream=stream):
+            st.run_stack(c, stream=stream, **over)
+    for rep in range(3):
+        c["q"][st.dim:].fill_(0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c["q"], a["q"]), "replay %d" % rep
+    assert timeouts() == before
+
+
+@pytest.mark.parametrize("chained,n_q,side", [(False, 32, 0), (True, 32, 0), (True, 32, 0x55555555), (True, 16, 0), (True, 8, 0x66666666)])
+def test_resident_stack_gives_up_with_nan_instead_of_hanging(dev, chained, n_q, side):
     """With the poll limit forced to zero every wait of the resident launch gives up at once -- a merging workgroup's
-    wait for the other splits' records, and every workgroup's wait for the previous layer's tags: the launch still ends
+    wait for the other splits' records and, in a chain, every workgroup's wait for the previous layer's tags: the launch still ends
     normally, every output of every layer is NaN (never a plausible number computed from inputs that were not ready),
     the give-ups are counted. With the limit restored and the workspace cleared the same call is right again."""
-    st = Stack(dev, 5, 3000, seed=31)
+    st = Stack(dev, 5, 3000, n_q=n_q, seed=31, chained=chained)
+    st.kw["workspace_side"] = side
     a = st.fresh()
     st.run_per_layer(a)
     before = timeouts()
