@@ -114,11 +114,34 @@ def _native():
     return native
 
 
-_ops = _native()
-mha_decode = _ops.mha_decode
-mha_decode_append = _ops.mha_decode_append
-mha_decode_append_stack = _ops.mha_decode_append_stack
-qk_norm_rope_append = _ops.qk_norm_rope_append
-kv_restride = _ops.kv_restride
-gemv = _ops.gemv
-qkv_gemv = _ops.qkv_gemv
+# The native calls by name. They take their places in this module when the first of them is asked for: importing it, and its argument
+# helpers, need nothing built.
+_CALLS = ("mha_decode", "mha_decode_append", "mha_decode_append_stack", "qk_norm_rope_append", "kv_restride", "gemv", "qkv_gemv")
+__all__ = ["workspace_bytes", "make_mha_args", "workspace_side", "mha_plan", "mha_decode_raw", "sincos_table", *_CALLS]
+
+
+def _bind_calls():
+    native = _native()
+    globals().update({name: getattr(native, name) for name in _CALLS})
+    return native
+
+
+def _unbuilt(name):
+    """What stands for a native call while there is none: the call says what is missing."""
+    def call(*args, **kw):
+        return getattr(_bind_calls(), name)(*args, **kw)
+    call.__name__ = call.__qualname__ = name
+    return call
+
+
+def __getattr__(name):
+    if name not in _CALLS:
+        raise AttributeError("module %r has no attribute %r" % (__name__, name))
+    try:
+        return getattr(_bind_calls(), name)
+    except (RuntimeError, OSError):
+        return _unbuilt(name)
+
+
+def __dir__():
+    return sorted(set(globals()) | set(_CALLS))

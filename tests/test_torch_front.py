@@ -1,6 +1,9 @@
 """The native calls of llminfer_amd.ops: how they take their arguments and refuse wrong ones (no GPU needed: a refused call
 reaches neither the C ABI nor the device), and what they hand on where there is a GPU."""
 import inspect
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -8,6 +11,7 @@ import torch
 from llminfer_amd import _binding as B
 from llminfer_amd import ops
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SCALARS = dict(layer_id=0, pos=5, kv_dim=1024, kv_mul=4, head_num=32, head_dim=128, max_seq_len=64)
 
 
@@ -54,6 +58,26 @@ def test_signatures_are_the_documented_ones():
     assert sig.parameters["eps"].default == 1e-6 and sig.parameters["one_launch"].default is False
     assert inspect.signature(ops.gemv).parameters["mode"].default == B.GEMV_OUT_BF16
     assert inspect.signature(ops.mha_decode).parameters["kv_layout"].default == B.KV_LAYOUT_POS_MAJOR
+
+
+def test_import_needs_nothing_built():
+    """Importing the module, its argument helpers and the names of its calls load no library; what is missing is said by the call."""
+    code = ("from llminfer_amd import _binding as B, ops\n"
+            "from llminfer_amd.ops import *\n"
+            "assert B._lib is None\n"
+            "a = ops.make_mha_args(16, 16, 16, 16, None, **%r)\n"
+            "assert a.head_num == 32 and 'gemv' in dir(ops) and callable(gemv) and callable(ops.mha_decode)\n"
+            "for f in (ops.gemv, kv_restride):\n"
+            "    try:\n"
+            "        f(None, None, None)\n"
+            "    except RuntimeError as e:\n"
+            "        assert 'is not built' in str(e), e\n"
+            "    else:\n"
+            "        raise SystemExit('no error')\n" % SCALARS)
+    env = dict(os.environ, LLMI_HIP_LIBRARY=os.path.join(ROOT, "no_such_library.so"))
+    subprocess.run([sys.executable, "-c", code], check=True, env=env, cwd=ROOT)
+    with pytest.raises(AttributeError, match="no attribute 'gemm'"):
+        ops.gemm
 
 
 @pytest.mark.gpu
