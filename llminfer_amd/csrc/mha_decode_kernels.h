@@ -260,12 +260,15 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     };
 
     auto compute_tile = [&](int t, const TileRegs& r) {
+        const int row0 = t * kTile + 4 * kg;
+#if !LLMI_PV_VALU
+        fold_tile<G>(r, qb, row0, nrows, a.scale_log2e, m_run, l_run, o);
+#else
         f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, r.k[j]),
                                                         __builtin_bit_cast(bf16x8, qb[j]), c, 0, 0, 0);
-        const int row0 = t * kTile + 4 * kg;
         float s[4];
         float tmax = -INFINITY;
 #pragma unroll
@@ -282,7 +285,6 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         const float psum = (p[0] + p[1]) + (p[2] + p[3]);
         l_run = l_run * alpha + psum;
         m_run = m_new;
-#if LLMI_PV_VALU
         // Rescale only when some head's max moved (wave-uniform test); head h's factor sits in
         // lane h of every 16-lane row.
         if (__any(alpha != 1.0f)) {
@@ -308,42 +310,6 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 for (int j = 0; j < 8; ++j) ov[h.value][j] = fmaf(ph, vf[i][j], ov[h.value][j]);
             }
         });
-#else
-        // The probabilities enter the second MFMA as a sum of two bf16 numbers
-        // (p = hi + lo, relative error 2^-17), so that the product keeps fp32-like accuracy.
-        const uint32_t p01 = pack_bf16(p[0], p[1]);
-        const uint32_t p23 = pack_bf16(p[2], p[3]);
-        const uint32_t q01 = pack_bf16(p[0] - bf16_lo(p01), p[1] - bf16_hi(p01));
-        const uint32_t q23 = pack_bf16(p[2] - bf16_lo(p23), p[3] - bf16_hi(p23));
-
-        // Rescale only when some head's max moved (wave-uniform test). The factor of
-        // head 4*kg + r sits in lane 4*kg + r of this lane's 16-lane row.
-        if (__any(alpha != 1.0f)) {
-            static_for<0, 4>([&](auto r) {
-                float ar;
-                if constexpr (G <= 4) ar = row_bcast<r.value>(alpha);  // only row kg = 0 holds heads
-                else ar = row_bcast_per_row<r.value>(alpha);           // DPP row k takes lane 4*k + r of its own row
-#pragma unroll
-                for (int j = 0; j < 8; ++j) o[j][r.value] *= ar;
-            });
-        }
-        // O^T += P^T V on the matrix cores: A = P^T (head x position: this lane's four
-        // probabilities are exactly its A fragment), B = V (position x column, column
-        // 8*n + j for output lane n: element j of each of the lane's four V rows).
-        const i16x4 pa = __builtin_bit_cast(i16x4, u32x2{p01, p23});
-        const i16x4 pb = __builtin_bit_cast(i16x4, u32x2{q01, q23});
-        i16x4 vb[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;  // high or low halves
-            const uint32_t b01 = __builtin_amdgcn_perm(r.v[1][j >> 1], r.v[0][j >> 1], sel);
-            const uint32_t b23 = __builtin_amdgcn_perm(r.v[3][j >> 1], r.v[2][j >> 1], sel);
-            vb[j] = __builtin_bit_cast(i16x4, u32x2{b01, b23});
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, vb[j], o[j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pb, vb[j], o[j], 0, 0, 0);
 #endif
     };
 
@@ -475,40 +441,23 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         // weight 1, output = the V row -- while its first tiles are still on their way.
         if constexpr (APPEND) {
             if (holds_new_row) {
-                typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-                u32x4 kf[4];
+                u32x4 kf[4], vf;
+                start_from_new_row(sh4 + 64, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o, [&] {
+                    if (n16 == 0) {
+                        uint16_t* kd = const_cast<uint16_t*>(a.k) + (int64_t)(seq_len - 1) * a.row_stride + kvh * a.slot_head_stride;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) kf[j] = sh4[64 + j * 4 + kg];  // operand layout, as a K row of a tile
-                const u32x4 vf = sh4[64 + 16 + n16];                          // columns 8*n16 .. +7
-                if (n16 == 0) {
-                    uint16_t* kd = const_cast<uint16_t*>(a.k) + (int64_t)(seq_len - 1) * a.row_stride + kvh * a.slot_head_stride;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(kd + (j * 4 + kg) * 8) = kf[j];
-                }
-                if (kg == 0)
-                    *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(a.v) + (int64_t)(seq_len - 1) * a.row_stride +
-                                              kvh * a.slot_head_stride + n16 * 8) = vf;
-                float dot = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const uint32_t qw = qb[j][c], kw = kf[j][c];  // (bit_cast straight from a vector element reads element 0)
-                        dot = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, qw), __builtin_bit_cast(bf16x2, kw), dot, false);
+                        for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(kd + (j * 4 + kg) * 8) = kf[j];
                     }
-                dot = rows_sum(dot);
-                m_run = dot * a.scale_log2e;
-                l_run = kg == 0 ? 1.0f : 0.0f;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint32_t vw = vf[j >> 1];
-                    const float vj = (j & 1) ? bf16_hi(vw) : bf16_lo(vw);
-                    o[j] = f32x4{vj, vj, vj, vj};
+                    if (kg == 0)
+                        *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(a.v) + (int64_t)(seq_len - 1) * a.row_stride +
+                                                  kvh * a.slot_head_stride + n16 * 8) = vf;
+                });
 #if LLMI_PV_VALU
 #pragma unroll
-                    for (int h = 0; h < G; ++h) ov[h][j] = kg == 0 ? vj : 0.0f;
+                for (int h = 0; h < G; ++h)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) ov[h][j] = kg == 0 ? o[j][0] : 0.0f;
 #endif
-                }
             }
         }
     }

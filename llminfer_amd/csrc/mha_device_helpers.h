@@ -295,8 +295,9 @@ __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, co
     *hi_p = u32x2{pack_bf16(oh[0], oh[1]), pack_bf16(oh[2], oh[3])};
 }
 
-// One tile of 16 positions into a wavefront's running softmax: q.K^T, online softmax, P^T.V on the matrix cores (the
-// probabilities as hi + lo bf16), for groups of G query heads. row0: the lane's first position in the split.
+// One tile of 16 positions into a wavefront's running softmax: q.K^T, online softmax, P^T.V on the matrix cores, for groups of G
+// query heads. row0: the lane's first position in the split. The one definition for every kernel, which is what lets the
+// multi-layer kernels give the bits of the launches they stand for.
 template <int G>
 __device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4], int row0, int nrows, float scale_log2e,
                                           float& m_run, float& l_run, f32x4 (&o)[8]) {
@@ -319,10 +320,14 @@ __device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4
     for (int e = 0; e < 4; ++e) p[e] = fast_exp2(s[e] - m_new);
     l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
     m_run = m_new;
+    // The probabilities enter the second MFMA as a sum of two bf16 numbers
+    // (p = hi + lo, relative error 2^-17), so that the product keeps fp32-like accuracy.
     const uint32_t p01 = pack_bf16(p[0], p[1]);
     const uint32_t p23 = pack_bf16(p[2], p[3]);
     const uint32_t q01 = pack_bf16(p[0] - bf16_lo(p01), p[1] - bf16_hi(p01));
     const uint32_t q23 = pack_bf16(p[2] - bf16_lo(p23), p[3] - bf16_hi(p23));
+    // Rescale only when some head's max moved (wave-uniform test). The factor of
+    // head 4*kg + r sits in lane 4*kg + r of this lane's 16-lane row.
     if (__any(alpha != 1.0f)) {
         static_for<0, 4>([&](auto rr) {
             float ar;
@@ -332,12 +337,15 @@ __device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4
             for (int j = 0; j < 8; ++j) o[j][rr.value] *= ar;
         });
     }
+    // O^T += P^T V on the matrix cores: A = P^T (head x position: this lane's four
+    // probabilities are exactly its A fragment), B = V (position x column, column
+    // 8*n + j for output lane n: element j of each of the lane's four V rows).
     const i16x4 pa = __builtin_bit_cast(i16x4, u32x2{p01, p23});
     const i16x4 pb = __builtin_bit_cast(i16x4, u32x2{q01, q23});
     i16x4 vb4[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;  // high or low halves
         const uint32_t b01 = __builtin_amdgcn_perm(r.v[1][j >> 1], r.v[0][j >> 1], sel);
         const uint32_t b23 = __builtin_amdgcn_perm(r.v[3][j >> 1], r.v[2][j >> 1], sel);
         vb4[j] = __builtin_bit_cast(i16x4, u32x2{b01, b23});
@@ -349,13 +357,15 @@ __device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4
 }
 
 // A wavefront's running softmax of the new token alone: score q.k, weight 1, output = the V row. new_rows: its K row
-// (normalised and rotated, operand layout) and V row in LDS, 16-byte chunks.
+// (normalised and rotated, operand layout) and V row in LDS, 16-byte chunks. in_registers(): called once both are, ahead of the sums.
+template <typename F>
 __device__ __forceinline__ void start_from_new_row(const u32x4* new_rows, const u32x4 (&qb)[4], int kg, int n16, float scale_log2e,
-                                                   u32x4 (&kf)[4], u32x4& vf, float& m_run, float& l_run, f32x4 (&o)[8]) {
+                                                   u32x4 (&kf)[4], u32x4& vf, float& m_run, float& l_run, f32x4 (&o)[8], F&& in_registers) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int j = 0; j < 4; ++j) kf[j] = new_rows[j * 4 + kg];
     vf = new_rows[16 + n16];
+    in_registers();
     float dot = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
