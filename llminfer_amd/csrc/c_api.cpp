@@ -274,7 +274,8 @@ static int make_plan(const llmi_mha_args* a, llmi_mha_plan* p, int wave_cap = kM
         // tiles, four are ahead there too, 8 : 4 waves: 16 Q / 2 KV heads 5.17 : 5.00 us at 700 positions, 6.23 : 6.00 at 3001,
         // 8.05 : 7.65 at 12001, 11.8 : 11.3 at 40001, 20.2 : 19.9 at 100001; 8 Q / 1 KV head 6.28 : 5.82 at 3001, 7.71 : 7.37 at
         // 12001, 13.8 : 13.6 at 100001. (Not the append variant: the multi-layer launch stands for its eight, and a forced
-        // split count keeps them.)
+        // split count keeps them.) The split counts are those of the rule below all the same; with four waves half as many are ahead
+        // of one KV head's 256 up to some length: 128 : 256 splits 6.88 : 7.33 at 12001, 9.29 : 9.52 at 40001, behind at 100001.
         const bool few_heads = n_kv <= 2 && new_rows == 0 && a->num_splits == 0;
         int auto_waves = (group_pad == 8 && wave_cap >= 8 && !few_heads) ? 8 : 4;
         if (auto_waves > max_waves) auto_waves = max_waves;

@@ -6,9 +6,9 @@
 // (fused_gemv_add_bf16x8_kernel, :143-172).
 //
 // HBM-bound weight streams: every weight byte is read once, with non-temporal 16-byte loads, one row per wavefront
-// (64 lanes x 8 bf16 per step of 512 elements). A kernel per step count, unrolled: rows of up to 8 steps are asked for at once,
-// in longer ones the weights and the input run six steps ahead of the sum, each request taking the place of a step that has
-// been added. (In batches of four steps, each waited for, a row of 5120 was four trips to memory.) Graph replays over distinct
+// (64 lanes x 8 bf16 per step of 512 elements). A kernel per step count up to 20, unrolled: rows of up to 8 steps are asked for at once,
+// in longer ones the weights and the input run a window of steps ahead of the sum, each request taking the place of a step that has
+// been added; six steps, but where launch_rows says otherwise. Longer rows keep the window in a ring. (In batches of four steps, each waited for, a row of 5120 was four trips to memory.) Graph replays over distinct
 // matrices, batches of four : the window, us and TB/s of the latter:
 //   6144 x 2560    6.95 : 6.65 (4.7)      2560 x 4096   5.17 : 5.16 (4.1)     10240 x 5120   17.7 : 16.6 (6.3)
 //   5120 x 8192    15.5 : 14.9 (5.6)      2560 x 9728   9.58 : 9.13 (5.5)    152000 x 2560  110.1 : 109.0 (7.1)
@@ -18,7 +18,7 @@
 // 5 % slower); workgroups that stay and walk the rows (4-12 % slower); fewer of them in flight by LDS (level). K split
 // over the wavefronts of a workgroup is level, 3 % faster at 8192, 3 % slower at 9728. Products are formed in fp32 by
 // v_dot2_f32_bf16 (two bf16 pairs per instruction, fp32 accumulate), the 64 lanes fold with DPP row steps and four scalar
-// reads, lane 0 rounds once and writes.
+// reads, lane 0 rounds once and writes. All forms add a lane's steps in the same order: the same bits.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>

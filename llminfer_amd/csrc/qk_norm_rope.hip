@@ -104,7 +104,9 @@ __global__ void sincos_table_kernel(float* __restrict__ sin_cache, float* __rest
 // 16-byte chunk per thread, both ways past the caches (each byte is touched once). K and V, 8 KV heads, cached accesses and a 64-bit
 // division for each of layer, position and head : this, us: 36 layers of 3777 positions 184.5 : 177.7 (6.3 TB/s; a copy by torch of the
 // same bytes 207), 8 of 12000 135.6 : 128.7, 28 of 500 23.7 : 23.0, 60 of 100 14.6 : 12.8; a first pass on new buffers 223 : 191 and
-// 169 : 142. Cached reads with such stores 180 (first pass 230); two, four and eight chunks per thread 181, 187 and 280; positions of one KV
+// 169 : 142. Where both caches fit the 256 MB memory-side cache a conversion of the same buffers over again is slower for going past it (36 layers of 1000
+// 21.9 : 24.1, 28 of 2000 32.8 : 36.7, 28 of 500 level) and so is a reader of the result right behind it (copy included, 36 of 1000 49 : 53, but 28 of 2000 92 : 79); with the
+// source just written it is faster (30 : 23, 50 : 34). A prompt is converted once, out of buffers that its prefill wrote. Cached reads with such stores 180 (first pass 230); two, four and eight chunks per thread 181, 187 and 280; positions of one KV
 // head per workgroup (whole runs on the writing side) 184 ... 215.
 constexpr int kRestrideThreads = 256;
 __global__ __launch_bounds__(kRestrideThreads) void kv_restride_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst,
