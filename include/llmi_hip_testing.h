@@ -42,8 +42,8 @@ void llmi_hip_workspace_side_stats(uint64_t out[3]);
 int32_t llmi_hip_stagger_mask(int32_t kv_layout, int64_t run_bytes, int32_t ragged);
 
 /* The launcher's rule for the merge of the split path's results: the fewest splits at which the heads of a KV head are
- * merged by as many workgroups, for a group of `kv_mul` of `head_num` query heads in all; INT32_MAX = never. */
-int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t head_num);
+ * merged by as many workgroups of `waves` wavefronts, for a group of `kv_mul` of `head_num` query heads in all; INT32_MAX = never. */
+int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t waves, int32_t head_num);
 
 #ifdef __cplusplus
 }

@@ -138,12 +138,14 @@ static bool spread_merge_fits(int head_num) {
 // against not: 16 splits 5.08 : 4.98 us at 1024 positions, 5.87 : 5.77 at 2048; 8 splits 4.51 : 4.41 at 256; 32 splits
 // 5.03 : 5.14 at 1024, 5.71 : 5.80 at 2048, 6.86 : 7.08 at 4096, 7.88 : 8.10 at 6000; 64 Q heads, 16 splits 5.55 : 5.68 at
 // 1024, 7.63 : 7.81 at 4096, 32 splits at 32768 24.4 : 25.3. Groups of 16 (four wavefronts): always, as soon as there is a
-// split for every head. LLMI_HIP_SPREAD_MIN_SPLITS moves the boundary. Never where the merging workgroups have no room to
+// split for every head. So do groups of 8 on four wavefronts (make_plan: few KV heads), whose one workgroup would take the heads
+// in turn; spread from 16 splits on : from 8 on, a device-side position of 177 that leaves 12 splits: 8 Q / 1 KV head 6.87 : 5.10 us,
+// 16 Q / 2 KV heads 6.55 : 5.14. LLMI_HIP_SPREAD_MIN_SPLITS moves the boundary. Never where the merging workgroups have no room to
 // wait in (spread_merge_fits).
-int spread_merge_min_splits(int group_pad, int head_num) {
+int spread_merge_min_splits(int group_pad, int waves, int head_num) {
     static const int v = env_int("LLMI_HIP_SPREAD_MIN_SPLITS", 1, 1 << 20, 0);
     if (!spread_merge_fits(head_num)) return INT32_MAX;
-    return v ? v : group_pad >= 16 ? 1 : group_pad >= 8 ? 16 : 32;
+    return v ? v : group_pad >= 16 || (group_pad >= 8 && waves == 4) ? 1 : group_pad >= 8 ? 16 : 32;
 }
 
 // Where the splits' runs start a multiple of 512 KiB apart, the workgroups of a KV head, walking in step, keep hitting
@@ -863,7 +865,9 @@ int32_t llmi_hip_set_test_far_home(int32_t mode) {
     return llmi::g_test_far_home.exchange(mode < 0 || mode > 2 ? 0 : mode, std::memory_order_relaxed);
 }
 
-int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t head_num) { return spread_merge_min_splits(pow2_ceil(kv_mul), head_num); }
+int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t waves, int32_t head_num) {
+    return spread_merge_min_splits(pow2_ceil(kv_mul), waves, head_num);
+}
 
 int32_t llmi_hip_stagger_mask(int32_t kv_layout, int64_t run_bytes, int32_t ragged) {
     return llmi::stagger_mask(kv_layout, run_bytes, ragged != 0);

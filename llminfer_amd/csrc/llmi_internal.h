@@ -66,7 +66,7 @@ constexpr bool by_side_variant(int group_pad, int waves) { return group_pad <= 8
 // Waits of the fused combine that gave up since the library was loaded (device counter of the current device).
 int read_poll_timeouts(unsigned long long* count);
 // Fewest splits at which the fused combine hands the heads of a KV head to different workgroups (INT32_MAX: never).
-int spread_merge_min_splits(int group_pad, int head_num);
+int spread_merge_min_splits(int group_pad, int waves, int head_num);
 // The dispatcher's rule for kernels that read the position on the device (KernelArgs::dyn_*): tiles up to which one split takes
 // them all, and the split counts of short contexts. Zeros where the caller or the environment forces a split count.
 void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, int* single, int* quarter, int* half);

@@ -182,7 +182,7 @@ static int fill_kernel_args(const llmi_mha_args& args, const llmi_mha_plan& plan
         ka.head_stride = (int64_t)args.max_seq_len * args.head_dim;
     }
     ka.seq_len = args.pos + 1;
-    ka.spread_min = spread_merge_min_splits(plan.group_pad, args.head_num);
+    ka.spread_min = spread_merge_min_splits(plan.group_pad, plan.waves_per_group, args.head_num);
     if (args.pos_device) {
         if (plan.num_splits > 1) dyn_split_rule(args, plan, &ka.dyn_single, &ka.dyn_quarter, &ka.dyn_half);
         const int32_t counts[3] = {ka.dyn_quarter, ka.dyn_half, plan.num_splits};

@@ -31,6 +31,10 @@ HEAD, POS = B.KV_LAYOUT_HEAD_MAJOR, B.KV_LAYOUT_POS_MAJOR
     (26, 2, 209, POS, {}),                                                 # 13 heads in a group
     (9, 1, 3000, HEAD, dict(num_splits=9)),
     (16, 1, 20000, HEAD, {}),                                              # 256 splits, 16 heads, two columns a thread
+    (8, 1, 200, HEAD, dict(num_splits=12, waves_per_group=4)),             # 8 heads, four wavefronts: a head each
+    (16, 2, 250, POS, dict(num_splits=15, waves_per_group=4)),
+    (14, 2, 130, HEAD, dict(num_splits=7, waves_per_group=4)),             # ... as many splits as heads
+    (8, 1, 120, POS, dict(num_splits=7, waves_per_group=4)),               # ... one split too few
 ])
 def test_merges_of_many_splits_and_large_groups(oracle, dev, n_q, n_kv, ctx, layout, kw):
     case = synth.make_case(7 + ctx, n_q=n_q, n_kv=n_kv, ctx=ctx)
