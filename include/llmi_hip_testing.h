@@ -7,6 +7,8 @@
 
 #include <stdint.h>
 
+#include "llmi_hip.h"
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -44,6 +46,10 @@ int32_t llmi_hip_stagger_mask(int32_t kv_layout, int64_t run_bytes, int32_t ragg
 /* The launcher's rule for the merge of the split path's results: the fewest splits at which the heads of a KV head are
  * merged by as many workgroups of `waves` wavefronts, for a group of `kv_mul` of `head_num` query heads in all; INT32_MAX = never. */
 int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t waves, int32_t head_num);
+
+/* The launcher's rule for a position read on the device (args->pos being the largest): tiles of 16 cached positions up to which
+ * one split takes them all, splits below rule[2] tiles (a tile each if there are fewer), splits up to 4 * rule[2] tiles. */
+int32_t llmi_hip_device_split_rule(const llmi_mha_args* args, int32_t append, int32_t rule[3]);
 
 #ifdef __cplusplus
 }

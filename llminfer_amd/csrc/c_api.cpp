@@ -203,16 +203,29 @@ static int fewest_splits(int n_kv, int kv_mul) { return kv_mul > 8 && spread_mer
 static int half_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv, fewest_splits(n_kv, kv_mul)); }
 static int quarter_splits(int n_kv, int kv_mul) { return std::max(kMinGroups / n_kv / 2, fewest_splits(n_kv, kv_mul)); }
 
-void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, int* single, int* quarter, int* half) {
+void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, bool append, int* single, int* quarter, int* half) {
     *single = *quarter = *half = 0;
     if (args.num_splits != 0 || args.force_path != LLMI_PATH_AUTO || env_tuning().num_splits) return;
     const int n_kv = args.kv_dim / args.head_dim;
-    // (the launch has the split path's waves: four, eight for groups of 8 heads. At four a single pass still is the faster one
-    // up to the same length as at the eight that a launch planned for it would have: 4.34 : 4.51 us at 176 positions,
+    // (the launch has the split path's waves: four, eight for groups of 8 heads. At four a single pass of the plain variant still is the
+    // faster one up to the same length as at the eight that a launch planned for it would have: 4.34 : 4.51 us at 176 positions,
     // 4.96 : 4.67 at 220)
     *single = single_pass_limit(args.kv_mul, plan.group_pad, args.head_num, plan.waves_per_group >= 8) / kTile;
+    int q = quarter_splits(n_kv, args.kv_mul);
+    const int h = half_splits(n_kv, args.kv_mul);
+    if (plan.group_pad <= 4) {
+        // Two differences to a launch planned for the length, groups of up to 4 heads. The rings of four wavefronts hold eight tiles. The append
+        // variant, whose wavefront with the most tiles may have the new token too, splits the ninth tile, a second trip to memory, rather than
+        // wait for it; the plain one does at 12 (us, single pass : split, a layer of the captured step, caches that are in no cache memory: append 32 Q / 8 KV
+        // heads 5.45 : 5.28 at 145 positions, 16 Q heads 5.33 : 5.07, 8 Q heads 5.29 : 5.00, 8 Q / 2 KV heads level; plain 32 Q heads 4.56 : 4.53
+        // at 145, 16 Q heads 4.40 : 4.46, 8 Q / 2 KV heads 4.50 : 4.99 at 161).
+        if (append && env_tuning().single_pass_max < 0) *single = std::min(*single, 4 * 2);
+        // And up to 15 tiles are split one by one, where a quarter of the splits (8 of 8 KV heads) would give some of them two
+        // (plain, 8 splits : a tile each: 32 Q / 8 KV heads 4.68 : 4.55 at 178, 4.76 : 4.58 at 225, 16 Q heads 4.55 : 4.47; append level). Not
+        // up to half of them at fewer KV heads: 16 Q / 4 KV heads, 19 tiles in 16 : 19 splits, 4.83 : 5.33.
+        q = std::max(q, std::min(h, 16));
+    }
     // (no more than the launch has workgroups for)
-    const int q = quarter_splits(n_kv, args.kv_mul), h = half_splits(n_kv, args.kv_mul);
     *quarter = q < plan.num_splits ? q : plan.num_splits;
     *half = h < plan.num_splits ? h : plan.num_splits;
 }
@@ -867,6 +880,14 @@ int32_t llmi_hip_set_test_far_home(int32_t mode) {
 
 int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t waves, int32_t head_num) {
     return spread_merge_min_splits(pow2_ceil(kv_mul), waves, head_num);
+}
+
+int32_t llmi_hip_device_split_rule(const llmi_mha_args* args, int32_t append, int32_t rule[3]) {
+    llmi_mha_plan plan;
+    if (!args || !rule) return LLMI_ERR_NULL_POINTER;
+    if (int rc = make_plan(args, &plan, kMaxWaves, append ? 1 : 0)) return rc;
+    dyn_split_rule(*args, plan, append != 0, &rule[0], &rule[1], &rule[2]);
+    return LLMI_OK;
 }
 
 int32_t llmi_hip_stagger_mask(int32_t kv_layout, int64_t run_bytes, int32_t ragged) {

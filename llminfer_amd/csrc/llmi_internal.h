@@ -69,7 +69,7 @@ int read_poll_timeouts(unsigned long long* count);
 int spread_merge_min_splits(int group_pad, int waves, int head_num);
 // The dispatcher's rule for kernels that read the position on the device (KernelArgs::dyn_*): tiles up to which one split takes
 // them all, and the split counts of short contexts. Zeros where the caller or the environment forces a split count.
-void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, int* single, int* quarter, int* half);
+void dyn_split_rule(const llmi_mha_args& args, const llmi_mha_plan& plan, bool append, int* single, int* quarter, int* half);
 // The mask of the staggered walk (KernelArgs::stagger) for splits whose runs are `run_bytes` long (the shorter ones,
 // when they differ by a tile: `ragged`).
 int stagger_mask(int kv_layout, int64_t run_bytes, bool ragged);

@@ -184,7 +184,7 @@ static int fill_kernel_args(const llmi_mha_args& args, const llmi_mha_plan& plan
     ka.seq_len = args.pos + 1;
     ka.spread_min = spread_merge_min_splits(plan.group_pad, plan.waves_per_group, args.head_num);
     if (args.pos_device) {
-        if (plan.num_splits > 1) dyn_split_rule(args, plan, &ka.dyn_single, &ka.dyn_quarter, &ka.dyn_half);
+        if (plan.num_splits > 1) dyn_split_rule(args, plan, append != nullptr, &ka.dyn_single, &ka.dyn_quarter, &ka.dyn_half);
         const int32_t counts[3] = {ka.dyn_quarter, ka.dyn_half, plan.num_splits};
         for (int i = 0; i < 3; ++i) ka.dyn_magic[i] = counts[i] > 1 ? (uint32_t)(((1ull << 32) + counts[i] - 1) / counts[i]) : 0u;
     }

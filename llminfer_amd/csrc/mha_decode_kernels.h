@@ -99,9 +99,9 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     // and in the append variant the one that holds the new token -- never has the longest run.
     // With a position read from device memory the grid was sized for the largest position:
     // the same rules are applied to the tiles there are -- a single pass, a quarter or half of the
-    // splits or all of them, as the host would have planned --, and the splits that are not needed leave at once.
+    // splits or all of them, nearly as the host would have planned (dyn_split_rule) --, and the splits that are not needed leave at once.
     // 32 Q / 8 KV heads, append variant in a captured 36-layer step sized for 8192 positions, us per layer, all splits as far as
-    // there are tiles : the rule: 5.54 : 4.07 at 60 positions, 5.53 : 5.25 at 170, 5.65 : 5.41 at 300, 5.69 : 5.47 at 600.
+    // there are tiles : the rule: 5.58 : 4.02 at 60 positions, 5.51 : 5.33 at 170, 5.65 : 5.36 at 300, 5.73 : 5.40 at 600.
     // Append variant: the new token's row never comes from the cache (its K and V are in registers
     // and go straight into the running softmax of one wave), so the tiles cover positions 0 .. pos-1.
     int seq_len = a.seq_len, n_active = a.num_splits;

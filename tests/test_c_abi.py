@@ -416,6 +416,23 @@ def test_stagger_rule_of_the_split_path():
     assert run(LLMI_HIP_STAGGER_MASK="junk") == run()
 
 
+@pytest.mark.parametrize("append", [0, 1])
+@pytest.mark.parametrize("n_q,n_kv,single,quarter,half", [
+    (8, 8, (11, 8), 16, 16), (32, 8, (11, 8), 16, 16), (16, 16, (11, 8), 8, 8), (16, 4, (11, 8), 16, 32), (8, 2, (11, 8), 32, 64),
+    (64, 8, (15, 15), 8, 16), (16, 2, (11, 15), 32, 64), (32, 2, (15, 15), 32, 64),  # groups of 8 (four or eight wavefronts) and 16
+])
+def test_split_counts_of_a_device_position(append, n_q, n_kv, single, quarter, half):
+    """Groups of up to 4 heads: the append variant is split from the ninth tile on, the plain one from the twelfth, both a tile each
+    up to 15; larger groups as a launch planned for the length. A forced split count leaves no rule."""
+    a = good_args(pos=4095, pos_device=0x1000, head_num=n_q, kv_mul=n_q // n_kv, kv_dim=n_kv * 128)
+    rule = (ctypes.c_int32 * 3)()
+    assert B.lib().llmi_hip_device_split_rule(ctypes.byref(a), append, rule) == 0
+    assert tuple(rule) == (single[append], quarter, half)
+    a.num_splits, a.force_path = 8, B.PATH_SPLIT_FUSED
+    assert B.lib().llmi_hip_device_split_rule(ctypes.byref(a), append, rule) == 0
+    assert tuple(rule) == (0, 0, 0)
+
+
 @pytest.mark.parametrize("pos", [100, 200, 250, 700, 2999, 40000])
 def test_workgroups_that_wait_for_each_other_leave_room(pos):
     """A spread merge has a workgroup per query head wait for the other splits of its KV head; a compute unit may hold one of
