@@ -761,13 +761,9 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         const bool wide = NW >= 4 && spread && SA > kWideMergeMin;
         if (spread ? wave != 0 && !wide : wave >= a.group) return;
         const int h = spread ? merge_head : wave;
-        const int share = wide ? (SA + NW - 1) / NW : SA;  // (at most 64: 256 splits, four wavefronts)
-        const int first = wide ? wave * share : 0;
-        const int count = wide ? max(0, min(share, SA - first)) : SA;
         const int c4 = lane & 31;
         const int part = lane >> 5;
         const int hq = kvh * a.group + h;
-        const float* w = s_w + h * kMaxSplits + first;
         const WsHead wh = ws_head<BYSIDE>(a, hq);
         // Byte offset of split sp's partial row, in both layouts with the same few instructions: plain, it is
         // B = row * 512; by side, the row's pair of 8 KiB blocks starts at twice B's block start and the home adds 8 KiB
@@ -775,16 +771,21 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         const uint32_t row0_bytes = (uint32_t)wh.rbase * (kHeadDim * 4u);
         const uint32_t block_mask = BYSIDE ? ~(uint32_t)(kSideBlockBytes - 1) : 0u;
         const uint32_t lane_bytes = (uint32_t)c4 * 16u;
-        auto load_partial = [&](int sp, uint32_t home_bytes) {  // (sp counted from `first`)
-            const int spc = first + min(sp, count - 1);  // in range, a row whose record is in; the weight drops the repeat
-            const uint32_t B = row0_bytes + (uint32_t)spc * (kHeadDim * 4u);
-            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ws_rsrc, B + (B & block_mask) + home_bytes + lane_bytes, 0, kCoherent));
-        };
         // The first batch of partials is requested as soon as the records are in and travels
         // while the weights are worked out (they need the maximum over all records first).
-        auto run = [&](auto slots, auto batch) {
+        auto run = [&](auto slots, auto batch, auto wide_tag) {
             constexpr int kSlots = decltype(slots)::value;
             constexpr int kBatch = decltype(batch)::value;
+            constexpr bool kWide = decltype(wide_tag)::value;
+            const int share = (SA + NW - 1) / NW;  // (at most 64: 256 splits, four wavefronts)
+            const int first = kWide ? wave * share : 0;
+            const int count = kWide ? max(0, min(share, SA - first)) : SA;
+            const float* w = s_w + h * kMaxSplits + first;
+            auto load_partial = [&](int sp, uint32_t home_bytes) {  // (sp counted from `first`)
+                const int spc = first + min(sp, count - 1);  // in range, a row whose record is in; the weight drops the repeat
+                const uint32_t B = row0_bytes + (uint32_t)spc * (kHeadDim * 4u);
+                return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ws_rsrc, B + (B & block_mask) + home_bytes + lane_bytes, 0, kCoherent));
+            };
             float m_reg[kSlots], l_reg[kSlots];
             bool home[kSlots];
             const bool arrived = wait_records(h, first, count, slots, m_reg, l_reg, home);
@@ -838,37 +839,35 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 return sum;
             };
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (wide && count == 0) {
+            if (kWide && count == 0) {
                 // (fewer splits than the shares have room for: nothing to read)
             } else if constexpr (BYSIDE) acc = __builtin_expect(mixed, 0) ? gather(std::true_type{}) : gather(std::false_type{});
             else acc = gather(std::false_type{});
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = halves_sum(acc[e]);
             bool all_in = arrived;
-            if constexpr (NW >= 4 && !OPROJ) {
-                if (wide) {
-                    // (the epilogue's per-wavefront pairs have been read: their place takes the parts' maxima and sums)
-                    if (part == 0) s_part[wave * 32 + c4] = acc;
-                    if (lane == 0) {
-                        s_m[wave][0] = mx;
-                        s_l[wave][0] = den;
-                        s_ok[wave] = arrived ? 1 : 0;
-                    }
-                    __syncthreads();
-                    if (wave != 0) return;
-                    float top = -INFINITY;
+            if constexpr (kWide) {
+                // (the epilogue's per-wavefront pairs have been read: their place takes the parts' maxima and sums)
+                if (part == 0) s_part[wave * 32 + c4] = acc;
+                if (lane == 0) {
+                    s_m[wave][0] = mx;
+                    s_l[wave][0] = den;
+                    s_ok[wave] = arrived ? 1 : 0;
+                }
+                __syncthreads();
+                if (wave != 0) return;
+                float top = -INFINITY;
 #pragma unroll
-                    for (int x = 0; x < NW; ++x) top = fmaxf(top, s_m[x][0]);
-                    acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                    den = 0.0f;
+                for (int x = 0; x < NW; ++x) top = fmaxf(top, s_m[x][0]);
+                acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                den = 0.0f;
 #pragma unroll
-                    for (int x = 0; x < NW; ++x) {
-                        const float mw = s_m[x][0];
-                        const float f = (mw == -INFINITY) ? 0.0f : fast_exp2(mw - top);
-                        acc += s_part[x * 32 + c4] * f;
-                        den += s_l[x][0] * f;
-                        all_in = all_in && s_ok[x] != 0;
-                    }
+                for (int x = 0; x < NW; ++x) {
+                    const float mw = s_m[x][0];
+                    const float f = (mw == -INFINITY) ? 0.0f : fast_exp2(mw - top);
+                    acc += s_part[x * 32 + c4] * f;
+                    den += s_l[x][0] * f;
+                    all_in = all_in && s_ok[x] != 0;
                 }
             }
             if (part == 0) {
@@ -912,10 +911,23 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 }
             }
         };
+        const std::integral_constant<int, 1> one{};
+        const std::integral_constant<int, 8> eight{};
+        const std::integral_constant<int, 16> sixteen{};
+        // The wide merge is a copy of its own: with the shares' arithmetic in the path of the usual merges those took 0.04 - 0.08 us longer
+        // (shared : apart, append 64 Q / 8 KV heads 5.93 : 5.87 us at 400 positions, 6.06 : 5.99 at 700, plain 40 Q heads 4.99 : 4.92 at 400,
+        // 32 Q heads 4.87 : 4.83 at 700; the wide ones level).
+        if constexpr (NW >= 4 && kSpreadMerge) {
+            if (__builtin_expect(wide, 0)) {
+                if (SA <= 16 * NW) run(one, eight, std::true_type{});
+                else run(one, sixteen, std::true_type{});
+                return;
+            }
+        }
         // (a lane polls one split unless a single wavefront has more than 64: a rare case, kept out of the way of the usual ones)
-        if (__builtin_expect(count > 64, 0)) run(std::integral_constant<int, kMaxSplits / 64>{}, std::integral_constant<int, 16>{});
-        else if (count <= 16) run(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{});
-        else run(std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
+        if (__builtin_expect(SA > 64, 0)) run(std::integral_constant<int, kMaxSplits / 64>{}, sixteen, std::false_type{});
+        else if (SA <= 16) run(one, eight, std::false_type{});
+        else run(one, sixteen, std::false_type{});
         return;
     }
 
