@@ -117,7 +117,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         // the position known to the host).
         asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.row_stride), "s"(a.head_stride), "s"(a.group), "s"(a.num_splits), "s"(a.seq_len),
                      "s"(a.dyn_single), "s"(a.dyn_half), "s"(a.dyn_quarter), "s"(a.dyn_magic[0]), "s"(a.dyn_magic[1]), "s"(a.dyn_magic[2]));
-        if constexpr (APPEND) asm volatile("" ::"s"(a.norm_w), "s"(a.sin_cache), "s"(a.cos_cache), "s"(a.k_new), "s"(a.v_new));
+        if constexpr (APPEND) asm volatile("" ::"s"(a.norm_w), "s"(a.sin_cache), "s"(a.cos_cache), "s"(a.k_new), "s"(a.v_new), "s"(a.eps));
         // (constant address space: a scalar load, where the compiler, not knowing that nothing in the launch writes the position, takes a
         // vector one and its longer way: 36 layers 209.8 -> 205.5 us at 1100 positions, 194.5 -> 192.9 at 300, 64 layers of 64 Q heads at 5000
         // 532.0 -> 530.5. The query's request and the heads' addresses ahead of its arrival: level.)
@@ -154,6 +154,14 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     u32x4 qb[4];                       // query group, MFMA B operand
     // Append variant: wave 0 of the last split (the one with the shortest run) takes the new token.
     const bool holds_new_row = APPEND && split == n_active - 1 && wave == 0;
+    // Append variant: the rows of this workgroup -- the query heads, in the last split's the new K and V rows too -- are dealt to the waves in
+    // pairs, the last wave first: the first pair of this one (the next is NW on). With two waves on a SIMD those that have rows go first
+    // until the rows are done: their requests would else queue behind the tiles of the others (64 Q / 8 KV heads, a layer of a captured step at
+    // 1000 positions, without : with 6.49 : 6.32 us).
+    const int work_rows = a.group + (split == n_active - 1 ? 2 : 0);
+    const int first_pair = NW - 1 - wave;
+    const bool has_rows = APPEND && 2 * first_pair < work_rows;
+    if (NW > 4 && has_rows) __builtin_amdgcn_s_setprio(3);
 
     // Wave-uniform 64-bit bases of this split; lanes add 32-bit byte offsets
     // (scalar-base + vector-offset addressing, no 64-bit multiplies per load).
@@ -210,19 +218,22 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     constexpr int kMergeTail = (2 * NW * G + 2 * G) * (int)sizeof(float);
     constexpr int kCombineBase = kRingBytes + ((kMergeTail + 15) & ~15);
     constexpr int kCombineBytes = (G * kMaxSplits + G + NW) * (int)sizeof(float) + NW * 64 * 16;
-    // 1 KiB LDS-DMA slots for the small operands. Per wave: the query rows of the group (16 chunks
-    // of 16 bytes per head, four heads to a slot; normalised in place in the append variant).
-    // Append variant, in front of them and shared by the workgroup (every wave fills them with
-    // the same bytes and waits only for its own loads): slot 0 = q_norm | k_norm | sin row |
-    // cos row, 16 chunks each; slot 1 = new K row | new V row, used by one wave only. The slots
+    // 1 KiB LDS-DMA slots for the small operands, one wavefront's rows of 256 bytes four to a slot. Plain variant: every wave fetches all
+    // query rows of the group for itself. Append variant, in front of them: a slot shared by the workgroup, q_norm | k_norm | sin row |
+    // cos row (every wave that works on rows fills it with the same bytes and waits only for its own loads). The query rows, and in the
+    // workgroup of the last split the new K and V rows behind them, are dealt to the waves two at a time, 32 lanes a row, the last wave
+    // first (it has the fewest tiles); a wave fetches its own, raw, and leaves them normalised and rotated (V: as it is) behind the
+    // slots, where all waves read them after a barrier. The slots
     // lie over the combine area, which nobody touches before the barrier of the epilogue, so they
     // cost no LDS: with more than 80 KiB per workgroup the compiler assumes one wave per SIMD, puts
     // the MFMA accumulators into AGPRs and copies all 32 of them to VGPRs and back around the
     // rescaling of every tile.
-    constexpr int kQSlots = (G * 16 + 63) / 64;
-    constexpr int kSharedSlots = APPEND ? 2 : 0;
+    constexpr int kRowPasses = (G + 2 + 2 * NW - 1) / (2 * NW);  // append variant: rows per half wavefront
+    constexpr int kRowSlots = APPEND ? (2 * kRowPasses + 3) / 4 : (G * 16 + 63) / 64;
+    constexpr int kSharedSlots = APPEND ? 1 : 0;
+    constexpr int kReadyBytes = APPEND ? (G + 2) * 256 : 0;  // the finished rows: G query rows, the new K row, the new V row
     constexpr int kStagingBase = (kCombineBase + 1023) & ~1023;
-    constexpr int kStagingBytes = (kSharedSlots + NW * kQSlots) * 1024;
+    constexpr int kStagingBytes = (kSharedSlots + NW * kRowSlots) * 1024 + kReadyBytes;
     constexpr int kSmemBytes =
         kCombineBase + kCombineBytes > kStagingBase + kStagingBytes ? kCombineBase + kCombineBytes : kStagingBase + kStagingBytes;
     __shared__ __attribute__((aligned(1024))) char smem[kSmemBytes];
@@ -347,35 +358,48 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         // the tiles, so that nothing near the end of the kernel has to wait for it.
         proj.gen_base = __hip_atomic_load(a.ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    char* shared_staging = smem + kStagingBase;                                     // append variant only
-    char* my_rows = smem + kStagingBase + (kSharedSlots + wave * kQSlots) * 1024;  // this wave's query rows
+    char* shared_staging = smem + kStagingBase;                                       // append variant only
+    char* my_rows = smem + kStagingBase + (kSharedSlots + wave * kRowSlots) * 1024;  // this wave's rows
+    char* ready_rows = smem + kStagingBase + (kSharedSlots + NW * kRowSlots) * 1024;  // append variant only
     {
         const uint32_t st = (uint32_t)(uintptr_t)shared_staging;
         const uint32_t st_rows = (uint32_t)(uintptr_t)my_rows;
         const int c16 = lane & 15, which = lane >> 4;
         if constexpr (APPEND) {
-            const float* sin_row = a.sin_cache + (int64_t)(seq_len - 1) * 64;
-            const float* cos_row = a.cos_cache + (int64_t)(seq_len - 1) * 64;
-            // (integer selects: as pointer conditionals this becomes a chain of branches)
-            const uint64_t w_base = reinterpret_cast<uint64_t>(a.norm_w) + (uint64_t)(which & 1) * 256u;
-            const uint64_t t_base = reinterpret_cast<uint64_t>(which == 2 ? sin_row : cos_row);
-            const uint64_t p0 = (which < 2 ? w_base : t_base) + (uint64_t)c16 * 16u;
-            dma16_gather(reinterpret_cast<const void*>(p0), st);
-            if (holds_new_row) {
-                const uint64_t p1 = reinterpret_cast<uint64_t>((which & 1) == 0 ? a.k_new : a.v_new) +
-                                    (uint64_t)(kvh * kHeadDim * 2 + c16 * 16);
-                dma16_gather(reinterpret_cast<const void*>(p1), st + 1024);
+            if (has_rows) {
+                const float* sin_row = a.sin_cache + (int64_t)(seq_len - 1) * 64;
+                const float* cos_row = a.cos_cache + (int64_t)(seq_len - 1) * 64;
+                // (integer selects: as pointer conditionals this becomes a chain of branches)
+                const uint64_t w_base = reinterpret_cast<uint64_t>(a.norm_w) + (uint64_t)(which & 1) * 256u;
+                const uint64_t t_base = reinterpret_cast<uint64_t>(which == 2 ? sin_row : cos_row);
+                const uint64_t p0 = (which < 2 ? w_base : t_base) + (uint64_t)c16 * 16u;
+                dma16_gather(reinterpret_cast<const void*>(p0), st);
             }
         }
 #pragma unroll
-        for (int i = 0; i < kQSlots; ++i) {
-            const int head = min(which + 4 * i, a.group - 1);  // chunk lane + 64*i: head (lane + 64*i) / 16
-            dma16_gather(a.q + (int64_t)(kvh * a.group + head) * kHeadDim + c16 * 8, st_rows + i * 1024);
+        for (int i = 0; i < kRowSlots; ++i) {
+            uint64_t src;
+            if constexpr (APPEND) {
+                const int pair = first_pair + 2 * NW * i;  // the slot holds this one and the one NW on
+                if (2 * pair >= work_rows) continue;
+                const int row = 2 * (pair + NW * (which >> 1)) + (which & 1);
+                // (rows behind the last one repeat a row that is there and are not used)
+                const uint64_t q_row = reinterpret_cast<uint64_t>(a.q) + (uint64_t)(uint32_t)((kvh * a.group + min(row, a.group - 1)) * 256);
+                const uint64_t new_row = reinterpret_cast<uint64_t>(row == a.group ? a.k_new : a.v_new) + (uint64_t)(uint32_t)(kvh * 256);
+                src = (row >= a.group && work_rows > a.group ? new_row : q_row) + (uint64_t)c16 * 16u;
+            } else {
+                const int head = min(which + 4 * i, a.group - 1);  // chunk lane + 64*i: head (lane + 64*i) / 16
+                src = reinterpret_cast<uint64_t>(a.q + (int64_t)(kvh * a.group + head) * kHeadDim + c16 * 8);
+            }
+            dma16_gather(reinterpret_cast<const void*>(src), st_rows + i * 1024);
         }
     }
+    // Append variant: one tile ahead of the rows' work, the others behind it. (32 Q / 8 KV heads, a layer of a captured step at 4000 positions, both
+    // tiles of the ring ahead : one 7.42 : 7.21 us: a wave is held up by its requests once some 40 KiB of its compute unit's are on their way.)
+    const int first_tiles = min(APPEND ? 1 : NSTAGE, n_my);
 #pragma unroll
-    for (int s0 = 0; s0 < NSTAGE; ++s0)
-        if (s0 < n_my) issue_tile(tile_of(s0), s0);
+    for (int s0 = 0; s0 < (APPEND ? 1 : NSTAGE); ++s0)
+        if (s0 < first_tiles) issue_tile(tile_of(s0), s0);
     // What the end of the kernel needs to know about where its results go is worked out here, while the first tiles
     // are on their way and the wavefront has nothing else to do: behind the last tile every instruction is on the
     // path of whoever waits for this split (the empty asm statements keep the compiler from moving the work there).
@@ -417,47 +441,72 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     // were filled with copies of its last row).
     {
         // Everything issued before the tiles has landed once only the tiles are in flight.
-        wait_tiles_in_flight(min(NSTAGE, n_my));
-        const u32x4* sh4 = reinterpret_cast<const u32x4*>(shared_staging);
-        const u32x4* rows4 = reinterpret_cast<const u32x4*>(my_rows);
-        if constexpr (APPEND) {
-            // Four rows at a time, one per DPP row.
+        // (the accumulators are cleared here, in front of the wait, not behind it)
 #pragma unroll
-            for (int b4 = 0; b4 < kQSlots; ++b4)
-                norm_rope_rows_lds(my_rows, shared_staging, shared_staging + 512, shared_staging + 768, 4 * b4 + kg, n16, a.eps);
-            if (holds_new_row)  // the new K row: all four DPP rows work on the one row
-                norm_rope_rows_lds(shared_staging + 1024, shared_staging + 256, shared_staging + 512, shared_staging + 768, 0, n16,
-                                   a.eps);
-        }
+        for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(o[j]));
+        wait_tiles_in_flight(first_tiles);
         const int hq_local = min(n16, a.group - 1);
         const bool live = n16 < a.group;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const u32x4 qv = rows4[hq_local * 16 + j * 4 + kg];
-            qb[j] = live ? qv : u32x4{0u, 0u, 0u, 0u};
-        }
-        // Fused append: this wave files the new token's K row (normalised + rotated above) and V
-        // row in the cache and starts its running softmax from that one position -- score q.k,
-        // weight 1, output = the V row -- while its first tiles are still on their way.
         if constexpr (APPEND) {
+            const int half = lane >> 5, p32 = lane & 31;
+            // Two rows a wave, finished once for the workgroup. Every wave on its own took four rows at a time, 16 lanes each, groups of eight in two
+            // passes, and the one with the new token another for its K row, which in the workgroup that merges was the launch's
+            // longest way. A layer of a captured step, us, so : two rows a wave: 32 Q / 8 KV heads 4.89 : 4.27 at 100 positions, 5.33 : 5.13 at 300, 5.68 :
+            // 5.47 at 1100, 7.38 : 7.21 at 4000; 64 Q heads 5.97 : 5.74 at 200, 6.52 : 6.32 at 1000, 8.25 : 8.06 at 5000.
+            // (finished query rows: the 16-byte chunks swizzled by row & 7, so that the operand read below, one chunk of every row
+            // at once, spreads over the LDS banks)
+#pragma unroll
+            for (int j = 0; j < kRowPasses; ++j) {
+                const int pair = first_pair + NW * j;
+                if (2 * pair >= work_rows) continue;
+                const int row = 2 * pair + half;
+                const bool is_new = row >= a.group, is_v = row > a.group;
+                uint32_t xl, xh, lo, hi;
+                norm_rope_row32(my_rows + (2 * j + half) * 256, shared_staging + (is_new ? 256 : 0), shared_staging + 512, shared_staging + 768,
+                                p32, a.eps, xl, xh, lo, hi);
+                lo = is_v ? xl : lo;
+                hi = is_v ? xh : hi;
+                if (row < work_rows) {
+                    const int at = is_new ? (is_v ? G + 1 : G) * 256 + p32 * 4 : row * 256 + ((p32 >> 2) ^ (row & 7)) * 16 + (p32 & 3) * 4;
+                    *reinterpret_cast<uint32_t*>(ready_rows + at) = lo;
+                    *reinterpret_cast<uint32_t*>(ready_rows + at + 128) = hi;
+                    if (is_new) {  // the new token's rows, filed in the cache
+                        uint32_t* dst = reinterpret_cast<uint32_t*>(const_cast<uint16_t*>(is_v ? a.v : a.k) + (int64_t)(seq_len - 1) * a.row_stride +
+                                                                    kvh * a.slot_head_stride);
+                        dst[p32] = lo;
+                        dst[p32 + 32] = hi;
+                    }
+                }
+            }
+            if (NW > 4 && has_rows) __builtin_amdgcn_s_setprio(0);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+            for (int s0 = 1; s0 < NSTAGE; ++s0)
+                if (s0 < n_my) issue_tile(tile_of(s0), s0);
+            const u32x4* rows4 = reinterpret_cast<const u32x4*>(ready_rows);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u32x4 qv = rows4[hq_local * 16 + ((j * 4 + kg) ^ (hq_local & 7))];
+                qb[j] = live ? qv : u32x4{0u, 0u, 0u, 0u};
+            }
+            // Fused append: this wave starts its running softmax from the new token's position -- score q.k, weight 1, output = the V
+            // row -- while its first tiles are still on their way.
             if (holds_new_row) {
                 u32x4 kf[4], vf;
-                start_from_new_row(sh4 + 64, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o, [&] {
-                    if (n16 == 0) {
-                        uint16_t* kd = const_cast<uint16_t*>(a.k) + (int64_t)(seq_len - 1) * a.row_stride + kvh * a.slot_head_stride;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(kd + (j * 4 + kg) * 8) = kf[j];
-                    }
-                    if (kg == 0)
-                        *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(a.v) + (int64_t)(seq_len - 1) * a.row_stride +
-                                                  kvh * a.slot_head_stride + n16 * 8) = vf;
-                });
+                start_from_new_row(rows4 + G * 16, rows4 + G * 16 + 16, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o);
 #if LLMI_PV_VALU
 #pragma unroll
                 for (int h = 0; h < G; ++h)
 #pragma unroll
                     for (int j = 0; j < 8; ++j) ov[h][j] = kg == 0 ? o[j][0] : 0.0f;
 #endif
+            }
+        } else {
+            const u32x4* rows4 = reinterpret_cast<const u32x4*>(my_rows);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u32x4 qv = rows4[hq_local * 16 + j * 4 + kg];
+                qb[j] = live ? qv : u32x4{0u, 0u, 0u, 0u};
             }
         }
     }

@@ -249,16 +249,36 @@ __device__ __forceinline__ int package_side() {
     return (int)((xcc >> 2) & 1u);
 }
 
-// RMSNorm * weight + half-rotation RoPE of 128-wide bf16 rows held in LDS, in place, by one
-// wavefront: the 16 lanes of DPP row r take row `row` of `rows` (256 bytes each); lane p of them
+// RMSNorm * weight + half-rotation RoPE of 128-wide bf16 rows held in LDS, the arithmetic of the stand-alone kernel (x*w*r, then
+// a*cos - b*sin / a*sin + b*cos on the pairs (i, i+64)), rounded to bf16 once. Two forms, a row on 16 lanes or on 32, with the same
+// bits: four squares of two neighbouring pairs are added in order, the sums of neighbours folded lane by lane from there, and
+// the products that enter a sum are named (left to itself the compiler may contract the two forms differently).
+__device__ __forceinline__ float two_pairs_squared(float a0, float a1, float b0, float b1) {
+    return __builtin_fmaf(b1, b1, __builtin_fmaf(b0, b0, __builtin_fmaf(a1, a1, a0 * a0)));
+}
+// 1 / sqrt(mean square + eps). In the usual range the hardware's reciprocal root (1 ulp) and one Newton step, where a root and a division,
+// each rounded correctly, are 30 dependent instructions on the way to the query. (Largest error against 64 bits over 2^-98 ... 2^98:
+// 7.4e-8, with root and division 8.9e-8.)
+__device__ __forceinline__ float inverse_rms(float ss, float eps) {
+    const float x = ss / (float)kHeadDim + eps;
+    if (__builtin_expect(__any(!(x > 1e-30f && x < 1e30f)), 0)) return 1.0f / sqrtf(x);
+    const float y = __builtin_amdgcn_rsqf(x);
+    return __builtin_fmaf(0.5f * y, __builtin_fmaf(-x * y, y, 1.0f), y);
+}
+__device__ __forceinline__ void rotate_pair(float a, float b, float wa, float wb, float r, float sn, float cs, float& lo, float& hi) {
+    const float av = a * wa * r, bv = b * wb * r;
+    const float bs = bv * sn, bc = bv * cs;
+    lo = __builtin_fmaf(av, cs, -bs);
+    hi = __builtin_fmaf(av, sn, bc);
+}
+
+// In place, by one wavefront: the 16 lanes of DPP row r take row `row` of `rows` (256 bytes each); lane p of them
 // takes elements 4*(p&1) .. +3 of 16-byte chunk p>>1 and of its rotary partner, chunk (p>>1) + 8,
 // so a lane touches 8 elements, reads only what it overwrites, and the sum of squares is one
 // DPP row fold. `w`: the 256-byte norm weights; `sin16` / `cos16`: the 64 sines / cosines of the
-// position (lane p needs exactly 16-byte chunk p of each). Same chain as the stand-alone kernel
-// (x*w*r, then a*cos - b*sin / a*sin + b*cos on the pairs (i, i+64)), rounded to bf16 once.
+// position (lane p needs exactly 16-byte chunk p of each).
 __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, const char* sin16, const char* cos16,
                                                    int row, int p, float eps) {
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     const int c = p >> 1, hf = p & 1;
     u32x2* lo_p = reinterpret_cast<u32x2*>(rows + (row * 16 + c) * 16 + hf * 8);
     u32x2* hi_p = reinterpret_cast<u32x2*>(rows + (row * 16 + c + 8) * 16 + hf * 8);
@@ -273,26 +293,46 @@ __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, co
     const float b[4] = {bf16_lo(xh0), bf16_hi(xh0), bf16_lo(xh1), bf16_hi(xh1)};
     const float wa[4] = {bf16_lo(wl0), bf16_hi(wl0), bf16_lo(wl1), bf16_hi(wl1)};
     const float wb[4] = {bf16_lo(wh0), bf16_hi(wh0), bf16_lo(wh1), bf16_hi(wh1)};
-    float ss = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss += a[e] * a[e];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss += b[e] * b[e];
+    float ss = two_pairs_squared(a[0], a[1], b[0], b[1]) + two_pairs_squared(a[2], a[3], b[2], b[3]);
     ss += dpp_partner<0xB1>(ss);
     ss += dpp_partner<0x4E>(ss);
     ss += dpp_partner<0x141>(ss);
     ss += dpp_partner<0x140>(ss);
-    const float r = 1.0f / sqrtf(ss / (float)kHeadDim + eps);
+    const float r = inverse_rms(ss, eps);
     float ol[4], oh[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float av = a[e] * wa[e] * r;
-        const float bv = b[e] * wb[e] * r;
-        ol[e] = av * cs[e] - bv * sn[e];
-        oh[e] = av * sn[e] + bv * cs[e];
-    }
+    for (int e = 0; e < 4; ++e) rotate_pair(a[e], b[e], wa[e], wb[e], r, sn[e], cs[e], ol[e], oh[e]);
     *lo_p = u32x2{pack_bf16(ol[0], ol[1]), pack_bf16(ol[2], ol[3])};
     *hi_p = u32x2{pack_bf16(oh[0], oh[1]), pack_bf16(oh[2], oh[3])};
+}
+
+// A row on 32 lanes, half a wavefront, into registers: lane p of them takes the pairs 2p and 2p + 1, i.e. dword p of the row (lo) and
+// dword p + 32 (hi); xl, xh: the same two as they were. Half the instructions of the form above (a lane's share is half as long).
+__device__ __forceinline__ void norm_rope_row32(const char* row, const char* w, const char* sin16, const char* cos16, int p, float eps,
+                                                uint32_t& xl, uint32_t& xh, uint32_t& lo, uint32_t& hi) {
+    xl = *reinterpret_cast<const uint32_t*>(row + p * 4);
+    xh = *reinterpret_cast<const uint32_t*>(row + 128 + p * 4);
+    const uint32_t wl = *reinterpret_cast<const uint32_t*>(w + p * 4), wh = *reinterpret_cast<const uint32_t*>(w + 128 + p * 4);
+    const u32x2 sn = *reinterpret_cast<const u32x2*>(sin16 + p * 8), cs = *reinterpret_cast<const u32x2*>(cos16 + p * 8);
+    const uint32_t sn0 = sn[0], sn1 = sn[1], cs0 = cs[0], cs1 = cs[1];
+    const float a0 = bf16_lo(xl), a1 = bf16_hi(xl), b0 = bf16_lo(xh), b1 = bf16_hi(xh);
+    float ss = two_pairs_squared(a0, a1, b0, b1);
+    ss += dpp_partner<0xB1>(ss);
+    ss += dpp_partner<0x4E>(ss);
+    ss += dpp_partner<0x141>(ss);
+    ss += dpp_partner<0x140>(ss);
+    {
+        const unsigned u = __builtin_bit_cast(unsigned, ss);
+        const auto q = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        const unsigned q0 = q[0], q1 = q[1];
+        ss = __builtin_bit_cast(float, q0) + __builtin_bit_cast(float, q1);
+    }
+    const float r = inverse_rms(ss, eps);
+    float l0, l1, h0, h1;
+    rotate_pair(a0, b0, bf16_lo(wl), bf16_lo(wh), r, __builtin_bit_cast(float, sn0), __builtin_bit_cast(float, cs0), l0, h0);
+    rotate_pair(a1, b1, bf16_hi(wl), bf16_hi(wh), r, __builtin_bit_cast(float, sn1), __builtin_bit_cast(float, cs1), l1, h1);
+    lo = pack_bf16(l0, l1);
+    hi = pack_bf16(h0, h1);
 }
 
 // One tile of 16 positions into a wavefront's running softmax: q.K^T, online softmax, P^T.V on the matrix cores, for groups of G
@@ -356,16 +396,14 @@ __device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4
     for (int j = 0; j < 8; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pb, vb4[j], o[j], 0, 0, 0);
 }
 
-// A wavefront's running softmax of the new token alone: score q.k, weight 1, output = the V row. new_rows: its K row
-// (normalised and rotated, operand layout) and V row in LDS, 16-byte chunks. in_registers(): called once both are, ahead of the sums.
-template <typename F>
-__device__ __forceinline__ void start_from_new_row(const u32x4* new_rows, const u32x4 (&qb)[4], int kg, int n16, float scale_log2e,
-                                                   u32x4 (&kf)[4], u32x4& vf, float& m_run, float& l_run, f32x4 (&o)[8], F&& in_registers) {
+// A wavefront's running softmax of the new token alone: score q.k, weight 1, output = the V row. k_row, v_row: its K row
+// (normalised and rotated) and V row in LDS, 16-byte chunks, handed on in registers.
+__device__ __forceinline__ void start_from_new_row(const u32x4* k_row, const u32x4* v_row, const u32x4 (&qb)[4], int kg, int n16, float scale_log2e,
+                                                   u32x4 (&kf)[4], u32x4& vf, float& m_run, float& l_run, f32x4 (&o)[8]) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) kf[j] = new_rows[j * 4 + kg];
-    vf = new_rows[16 + n16];
-    in_registers();
+    for (int j = 0; j < 4; ++j) kf[j] = k_row[j * 4 + kg];
+    vf = v_row[n16];
     float dot = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; ++j)

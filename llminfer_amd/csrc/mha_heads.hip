@@ -267,7 +267,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
         for (int j = 0; j < 8; ++j) o[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         if (split == S - 1 && wave == 0) {
             u32x4 kf[4], vf;
-            start_from_new_row(ops4 + 64, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o, [] {});
+            start_from_new_row(ops4 + 64, ops4 + 80, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o);
         }
         for (int i = 0; i < u.n_my; ++i) {
             TileRegs r;

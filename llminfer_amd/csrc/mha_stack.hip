@@ -292,7 +292,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mha_stack_kernel(StackArgs sa) {
             }
             // The new token's row starts the running softmax; it is filed in this layer's cache slot behind the tiles (the
             // stores' acknowledgement must not sit in front of a tile's wait).
-            if (holds_new_row) start_from_new_row(sh4 + 64, qb, kg, n16, a.scale_log2e, new_k, new_v, m_run, l_run, o, [] {});
+            if (holds_new_row) start_from_new_row(sh4 + 64, sh4 + 80, qb, kg, n16, a.scale_log2e, new_k, new_v, m_run, l_run, o);
         }
 
         // ---- (3) this layer's tiles ----
@@ -662,7 +662,7 @@ __global__ __launch_bounds__(kLayersWaves * 64, 2) void mha_layers_kernel(StackA
             for (int j = 0; j < 8; ++j) o[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             if (holds_new_row && wave == 0) {
                 u32x4 kf[4], vf;
-                start_from_new_row(ops4 + 64, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o, [] {});
+                start_from_new_row(ops4 + 64, ops4 + 80, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o);
             }
             for (int i = 0; i < n_my; ++i) {
                 TileRegs r;
