@@ -585,11 +585,12 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         float mx = -INFINITY;
 #pragma unroll
         for (int w = 0; w < NW; ++w) mx = fmaxf(mx, mw[w]);
+        const float ref = mx == -INFINITY ? 0.0f : mx;  // (one select for a wave without a tile, not one per wave)
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         float lsum = 0.0f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            const float f = (mw[w] == -INFINITY) ? 0.0f : fast_exp2(mw[w] - mx);
+            const float f = fast_exp2(mw[w] - ref);
             acc += ow[w] * f;
             lsum += lw[w] * f;
         }
