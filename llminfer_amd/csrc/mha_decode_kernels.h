@@ -751,7 +751,9 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     };
     // From the polled (max, sum) pairs: M = max m_s, the weights e^(m_s - M) into the head's row
     // of s_w, the denominator sum l_s * weight; the records are zeroed for the next use.
-    auto make_weights = [&](int h, int first, int count, auto slots, const float* m_reg, const float* l_reg, const bool* home,
+    // (`alone`: nobody else writes weights of the head, so all 64 * kSlots places are written, zeros behind the last split: the sum of the
+    // partial rows then reads them without a test for each)
+    auto make_weights = [&](int h, int first, int count, auto slots, auto alone, const float* m_reg, const float* l_reg, const bool* home,
                             float& mx) -> float {
         constexpr int kSlots = decltype(slots)::value;
         const WsHead wh = ws_head<BYSIDE>(a, kvh * a.group + h);
@@ -763,11 +765,11 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) {
             const int sp = first + lane + 64 * j;
-            if (lane + 64 * j < count) {
+            if (decltype(alone)::value || lane + 64 * j < count) {  // (places without a split: weight and sum are zero)
                 const float f = (m_reg[j] == -INFINITY) ? 0.0f : fast_exp2(m_reg[j] - mx);
                 s_w[h * kMaxSplits + sp] = f;
                 den += l_reg[j] * f;
-                if (sp != split) {
+                if (sp != split && lane + 64 * j < count) {
                     unsigned long long* rec = a.records + (int64_t)ws_row<9>(wh, sp, home[j] ? 1 : 0) * 2;
                     __hip_atomic_store(rec, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     __hip_atomic_store(rec + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -782,7 +784,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         bool home[kSlots];  // (plain layout on this path: one home)
         const bool arrived = wait_records(h, 0, SA, slots, m_reg, l_reg, home);
         float mx;
-        den_out = make_weights(h, 0, SA, slots, m_reg, l_reg, home, mx);
+        den_out = make_weights(h, 0, SA, slots, std::true_type{}, m_reg, l_reg, home, mx);
         return arrived;
     };
     auto poll_head = [&](int h, float& den_out) -> bool {
@@ -841,10 +843,24 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             for (int j = 0; j < kSlots; ++j) other = other || home[j] != (my_xs != 0);
             const bool mixed = BYSIDE && __any(other);
             const uint32_t near_bytes = BYSIDE ? (uint32_t)(wh.ppar ^ my_xs) * kSideBlockBytes : 0u;
-            float den = 0.0f, mx = -INFINITY;
+            float den = 0.0f, mx = -INFINITY, inv = 0.0f;
             // The read-back, once for the usual case (every split in this side's home: one constant, nothing between the
             // loads) and once for the other one: two copies of the code rather than a test in front of every load.
-            auto gather = [&](auto mixed_tag) -> f32x4 {
+            // Where the heads' rows start at whole blocks of 16 (the launch's split count is a multiple of it, as the dispatcher's usual ones are) and
+            // the batch is full, a lane's rows lie at constant distances, which the loads carry as they are: five instructions less
+            // each. With the weights read without a test each and the division made while the rows travel (some 200 instructions in
+            // all, between the records' arrival and the output on the launch's last way), us, before : now: 32 Q / 8 KV heads 4.62 : 4.55 at 500 positions,
+            // 5.09 : 4.95 at 1100, 8.11 : 7.95 at 6007 (position-major), 64 Q heads 5.38 : 5.25 at 1100; a layer of a captured step 5.26 : 5.09
+            // at 1100, 7.19 : 7.03 at 4000, 64 Q heads 5.97 : 5.83 at 1000, 8.07 : 7.87 at 5000. (The rows' and the records' addresses ahead of
+            // the waits: level.)
+            const bool regular = !kWide && kSlots == 1 && (S & 15) == 0 && count >= 2 * kBatch;
+            const uint32_t regular_base = (BYSIDE ? 2 * row0_bytes + near_bytes : row0_bytes) + (uint32_t)part * (kHeadDim * 4u) + lane_bytes;
+            auto load_regular = [&](auto j_tag) {
+                constexpr int j = decltype(j_tag)::value;
+                constexpr uint32_t at = BYSIDE ? (j >> 3) * 2 * kSideBlockBytes + (j & 7) * 1024u : j * 1024u;
+                return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ws_rsrc, regular_base + (at & 4095u), at & ~4095u, kCoherent));
+            };
+            auto gather = [&](auto mixed_tag, auto regular_tag) -> f32x4 {
                 auto home_bytes = [&](int sp) -> uint32_t {
                     if constexpr (!decltype(mixed_tag)::value) return near_bytes;
                     // (the flag of split spc sits in lane spc % 64, slot spc / 64 of the polling layout: the slot's flags
@@ -861,16 +877,24 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                     return (uint32_t)(wh.ppar ^ xs) * kSideBlockBytes;
                 };
                 f32x4 v[kBatch];
+                if constexpr (decltype(regular_tag)::value) {
+                    static_for<0, kBatch>([&](auto j) { v[j.value] = load_regular(j); });
+                } else {
 #pragma unroll
-                for (int j = 0; j < kBatch; ++j) v[j] = load_partial(part + 2 * j, home_bytes(part + 2 * j));
-                den = make_weights(h, first, count, slots, m_reg, l_reg, home, mx);
+                    for (int j = 0; j < kBatch; ++j) v[j] = load_partial(part + 2 * j, home_bytes(part + 2 * j));
+                }
+                den = make_weights(h, first, count, slots, std::bool_constant<!kWide>{}, m_reg, l_reg, home, mx);
+                if constexpr (!kWide) {  // (the division while the rows travel)
+                    inv = 1.0f / den;
+                    asm volatile("" : "+v"(inv));
+                }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own weights are in LDS
                 __builtin_amdgcn_wave_barrier();
                 f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int j = 0; j < kBatch; ++j) {
                     const int sp = part + 2 * j;
-                    sum += v[j] * (sp < count ? w[sp] : 0.0f);
+                    sum += v[j] * (!kWide || sp < count ? w[sp] : 0.0f);
                 }
                 for (int s0 = part + 2 * kBatch; s0 < count; s0 += kBatch * 2) {
 #pragma unroll
@@ -878,7 +902,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
 #pragma unroll
                     for (int j = 0; j < kBatch; ++j) {
                         const int sp = s0 + 2 * j;
-                        sum += v[j] * (sp < count ? w[sp] : 0.0f);
+                        sum += v[j] * (!kWide || sp < count ? w[sp] : 0.0f);
                     }
                 }
                 return sum;
@@ -886,8 +910,13 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
             if (kWide && count == 0) {
                 // (fewer splits than the shares have room for: nothing to read)
-            } else if constexpr (BYSIDE) acc = __builtin_expect(mixed, 0) ? gather(std::true_type{}) : gather(std::false_type{});
-            else acc = gather(std::false_type{});
+            } else if (BYSIDE && __builtin_expect(mixed, 0)) {
+                acc = gather(std::bool_constant<BYSIDE>{}, std::false_type{});
+            } else if (!kWide && kSlots == 1 && regular) {
+                acc = gather(std::false_type{}, std::bool_constant<!kWide && kSlots == 1>{});
+            } else {
+                acc = gather(std::false_type{}, std::false_type{});
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] = halves_sum(acc[e]);
             bool all_in = arrived;
@@ -917,7 +946,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             }
             if (part == 0) {
                 // A wait that ran out of patience poisons the output rather than returning a partial sum.
-                const float inv = all_in ? 1.0f / den : __builtin_nanf("");
+                if constexpr (kWide) inv = 1.0f / den;
+                inv = all_in ? inv : __builtin_nanf("");
                 const f32x4 r = acc * inv;
                 const unsigned long long packed = (unsigned long long)pack_bf16(r[0], r[1]) | ((unsigned long long)pack_bf16(r[2], r[3]) << 32);
                 unsigned long long* op = reinterpret_cast<unsigned long long*>(a.out + (int64_t)hq * kHeadDim + c4 * 4);
