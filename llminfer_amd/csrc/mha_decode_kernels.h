@@ -540,11 +540,12 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
 #endif
 
     // This wave's ring is drained (every tile it issued was waited for and read).
-    typedef float (*MergeS)[G];
     auto s_o = [&](int w, int h) { return reinterpret_cast<float*>(smem + w * kWaveRingBytes) + h * kHeadDim; };
-    MergeS s_m = reinterpret_cast<MergeS>(smem + kRingBytes);
-    MergeS s_l = s_m + NW;
-    float* s_fin = reinterpret_cast<float*>(s_l + NW);  // [G][2]: merged (max, sum) per head
+    // [G][NW] maxima, then sums: a head's side by side, read 16 bytes at a time (one by one, wave by wave : so, us: 32 Q / 8 KV heads 4.94 : 4.87 at 1100
+    // positions, 64 Q heads 5.24 : 5.15; a layer of a captured step 64 Q heads 5.68 : 5.59 at 300, 5.82 : 5.76 at 1000, 7.92 : 7.81 at 5000).
+    float* s_m = reinterpret_cast<float*>(smem + kRingBytes);
+    float* s_l = s_m + G * NW;
+    float* s_fin = s_l + G * NW;  // [G][2]: merged (max, sum) per head
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int h = 4 * kg + r;
@@ -555,8 +556,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         }
     }
     if (kg == 0 && n16 < G) {
-        s_m[wave][n16] = m_run;
-        s_l[wave][n16] = l_run;
+        s_m[n16 * NW + wave] = m_run;
+        s_l[n16 * NW + wave] = l_run;
     }
     __syncthreads();
 
@@ -577,8 +578,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         f32x4 ow[NW];
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            mw[w] = s_m[w][h];
-            lw[w] = s_l[w][h];
+            mw[w] = s_m[h * NW + w];
+            lw[w] = s_l[h * NW + w];
             ow[w] = *reinterpret_cast<const f32x4*>(s_o(w, h) + c4 * 4);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -924,23 +925,23 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 // (the epilogue's per-wavefront pairs have been read: their place takes the parts' maxima and sums)
                 if (part == 0) s_part[wave * 32 + c4] = acc;
                 if (lane == 0) {
-                    s_m[wave][0] = mx;
-                    s_l[wave][0] = den;
+                    s_m[wave] = mx;
+                    s_l[wave] = den;
                     s_ok[wave] = arrived ? 1 : 0;
                 }
                 __syncthreads();
                 if (wave != 0) return;
                 float top = -INFINITY;
 #pragma unroll
-                for (int x = 0; x < NW; ++x) top = fmaxf(top, s_m[x][0]);
+                for (int x = 0; x < NW; ++x) top = fmaxf(top, s_m[x]);
                 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 den = 0.0f;
 #pragma unroll
                 for (int x = 0; x < NW; ++x) {
-                    const float mw = s_m[x][0];
+                    const float mw = s_m[x];
                     const float f = (mw == -INFINITY) ? 0.0f : fast_exp2(mw - top);
                     acc += s_part[x * 32 + c4] * f;
-                    den += s_l[x][0] * f;
+                    den += s_l[x] * f;
                     all_in = all_in && s_ok[x] != 0;
                 }
             }
