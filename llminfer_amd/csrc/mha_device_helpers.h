@@ -249,21 +249,32 @@ __device__ __forceinline__ int package_side() {
     return (int)((xcc >> 2) & 1u);
 }
 
-// RMSNorm * weight + half-rotation RoPE of 128-wide bf16 rows held in LDS, the arithmetic of the stand-alone kernel (x*w*r, then
-// a*cos - b*sin / a*sin + b*cos on the pairs (i, i+64)), rounded to bf16 once. Two forms, a row on 16 lanes or on 32, with the same
-// bits: four squares of two neighbouring pairs are added in order, the sums of neighbours folded lane by lane from there, and
-// the products that enter a sum are named (left to itself the compiler may contract the two forms differently).
-__device__ __forceinline__ float two_pairs_squared(float a0, float a1, float b0, float b1) {
-    return __builtin_fmaf(b1, b1, __builtin_fmaf(b0, b0, __builtin_fmaf(a1, a1, a0 * a0)));
+// RMSNorm * weight + half-rotation RoPE of 128-wide bf16 rows held in LDS, the formula of the stand-alone kernel (x*w*r, then
+// a*cos - b*sin / a*sin + b*cos on the pairs (i, i+64)), rounded to bf16 once; the stand-alone kernel adds its squares in another order, so a
+// value of it may round the other way. Two forms, a row on 16 lanes or on 32, with the same bits whatever the other rows of the wavefront hold:
+// the squares of four neighbouring pairs are one chain, a1 first, the chains folded neighbour by neighbour from there, and the products that
+// enter a sum are named (left to itself the compiler may contract the two forms differently).
+__device__ __forceinline__ float four_pairs_squared(const float (&a)[4], const float (&b)[4]) {
+    float ss = __builtin_fmaf(a[0], a[0], a[1] * a[1]);
+    ss = __builtin_fmaf(a[3], a[3], __builtin_fmaf(a[2], a[2], ss));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(b[e], b[e], ss);
+    return ss;
 }
-// 1 / sqrt(mean square + eps). In the usual range the hardware's reciprocal root (1 ulp) and one Newton step, where a root and a division,
-// each rounded correctly, are 30 dependent instructions on the way to the query. (Largest error against 64 bits over 2^-98 ... 2^98:
-// 7.4e-8, with root and division 8.9e-8.)
+// 1 / sqrt(mean square + eps), root and division each rounded correctly, in a third of the 30 dependent instructions that the compiler has for
+// them: the hardware's reciprocal root (1 ulp), a root from it and its residual, a reciprocal from both and its residual. Such a reciprocal
+// is the correctly rounded one unless the mantissa it divides by is all ones (P. Markstein, IBM J. Res. Dev. 34 (1990) 111), which is the root of
+// the two largest mantissas: those and what is out of range go the general way. (Every float in 1e-30 ... 1e30 compared with 1.0f / sqrtf(x):
+// all the same but the 198 of those two mantissas, so which way a row's neighbours send it leaves no trace in its bits.)
 __device__ __forceinline__ float inverse_rms(float ss, float eps) {
-    const float x = ss / (float)kHeadDim + eps;
-    if (__builtin_expect(__any(!(x > 1e-30f && x < 1e30f)), 0)) return 1.0f / sqrtf(x);
+    const float x = __builtin_fmaf(ss, 1.0f / kHeadDim, eps);
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    constexpr uint32_t lo = __builtin_bit_cast(uint32_t, 1e-30f), hi = __builtin_bit_cast(uint32_t, 1e30f);
+    if (__builtin_expect(__any(u - lo > hi - lo || (u & 0x7ffffeu) == 0x7ffffeu), 0)) return 1.0f / sqrtf(x);
     const float y = __builtin_amdgcn_rsqf(x);
-    return __builtin_fmaf(0.5f * y, __builtin_fmaf(-x * y, y, 1.0f), y);
+    const float s0 = x * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0);
+    return __builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y);
 }
 __device__ __forceinline__ void rotate_pair(float a, float b, float wa, float wb, float r, float sn, float cs, float& lo, float& hi) {
     const float av = a * wa * r, bv = b * wb * r;
@@ -293,7 +304,7 @@ __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, co
     const float b[4] = {bf16_lo(xh0), bf16_hi(xh0), bf16_lo(xh1), bf16_hi(xh1)};
     const float wa[4] = {bf16_lo(wl0), bf16_hi(wl0), bf16_lo(wl1), bf16_hi(wl1)};
     const float wb[4] = {bf16_lo(wh0), bf16_hi(wh0), bf16_lo(wh1), bf16_hi(wh1)};
-    float ss = two_pairs_squared(a[0], a[1], b[0], b[1]) + two_pairs_squared(a[2], a[3], b[2], b[3]);
+    float ss = four_pairs_squared(a, b);
     ss += dpp_partner<0xB1>(ss);
     ss += dpp_partner<0x4E>(ss);
     ss += dpp_partner<0x141>(ss);
@@ -307,17 +318,18 @@ __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, co
 }
 
 // A row on 32 lanes, half a wavefront, into registers: lane p of them takes the pairs 2p and 2p + 1, i.e. dword p of the row (lo) and
-// dword p + 32 (hi); xl, xh: the same two as they were. Half the instructions of the form above (a lane's share is half as long).
+// dword p + 32 (hi); xl, xh: the same two as they were. Half the instructions of the form above behind the root (a lane's share is half as
+// long); in front of it both lanes of a neighbouring two have the chain of their four pairs.
 __device__ __forceinline__ void norm_rope_row32(const char* row, const char* w, const char* sin16, const char* cos16, int p, float eps,
                                                 uint32_t& xl, uint32_t& xh, uint32_t& lo, uint32_t& hi) {
-    xl = *reinterpret_cast<const uint32_t*>(row + p * 4);
-    xh = *reinterpret_cast<const uint32_t*>(row + 128 + p * 4);
+    const u32x2 xl2 = *reinterpret_cast<const u32x2*>(row + (p >> 1) * 8), xh2 = *reinterpret_cast<const u32x2*>(row + 128 + (p >> 1) * 8);
     const uint32_t wl = *reinterpret_cast<const uint32_t*>(w + p * 4), wh = *reinterpret_cast<const uint32_t*>(w + 128 + p * 4);
     const u32x2 sn = *reinterpret_cast<const u32x2*>(sin16 + p * 8), cs = *reinterpret_cast<const u32x2*>(cos16 + p * 8);
     const uint32_t sn0 = sn[0], sn1 = sn[1], cs0 = cs[0], cs1 = cs[1];
-    const float a0 = bf16_lo(xl), a1 = bf16_hi(xl), b0 = bf16_lo(xh), b1 = bf16_hi(xh);
-    float ss = two_pairs_squared(a0, a1, b0, b1);
-    ss += dpp_partner<0xB1>(ss);
+    const uint32_t xl0 = xl2[0], xl1 = xl2[1], xh0 = xh2[0], xh1 = xh2[1];
+    const float a[4] = {bf16_lo(xl0), bf16_hi(xl0), bf16_lo(xl1), bf16_hi(xl1)};
+    const float b[4] = {bf16_lo(xh0), bf16_hi(xh0), bf16_lo(xh1), bf16_hi(xh1)};
+    float ss = four_pairs_squared(a, b);
     ss += dpp_partner<0x4E>(ss);
     ss += dpp_partner<0x141>(ss);
     ss += dpp_partner<0x140>(ss);
@@ -328,9 +340,11 @@ __device__ __forceinline__ void norm_rope_row32(const char* row, const char* w, 
         ss = __builtin_bit_cast(float, q0) + __builtin_bit_cast(float, q1);
     }
     const float r = inverse_rms(ss, eps);
+    xl = (p & 1) ? xl1 : xl0;
+    xh = (p & 1) ? xh1 : xh0;
     float l0, l1, h0, h1;
-    rotate_pair(a0, b0, bf16_lo(wl), bf16_lo(wh), r, __builtin_bit_cast(float, sn0), __builtin_bit_cast(float, cs0), l0, h0);
-    rotate_pair(a1, b1, bf16_hi(wl), bf16_hi(wh), r, __builtin_bit_cast(float, sn1), __builtin_bit_cast(float, cs1), l1, h1);
+    rotate_pair(bf16_lo(xl), bf16_lo(xh), bf16_lo(wl), bf16_lo(wh), r, __builtin_bit_cast(float, sn0), __builtin_bit_cast(float, cs0), l0, h0);
+    rotate_pair(bf16_hi(xl), bf16_hi(xh), bf16_hi(wl), bf16_hi(wh), r, __builtin_bit_cast(float, sn1), __builtin_bit_cast(float, cs1), l1, h1);
     lo = pack_bf16(l0, l1);
     hi = pack_bf16(h0, h1);
 }

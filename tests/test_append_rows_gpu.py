@@ -75,3 +75,57 @@ def test_rows_of_any_size(oracle, dev, scale, eps):
     """Mean squares in and out of the range of the reciprocal root."""
     got, ref, rows, k_n, v_new = _append(oracle, dev, 4, 8, 40, scale=scale, eps=eps)
     _check(got, ref, rows, k_n, v_new, "rows of size %g" % scale)
+
+
+def _bf16(bits):
+    return synth.bf16_bits_to_f32(bits)
+
+
+def _fma(a, b, c):
+    return (np.asarray(a, np.longdouble) * b + c).astype(np.float32)
+
+
+def _chain(rows, w, sin, cos, eps):
+    """Norm and rotation of raw bf16 rows [..., 128], operation by operation as the append kernels declare them: squares of four neighbouring
+    pairs in a chain, folded neighbour by neighbour, root and division each rounded, bf16 once. sin, cos: [..., 64]."""
+    x, w = _bf16(rows).reshape(rows.shape[:-1] + (2, 16, 4)), _bf16(w).reshape(2, 16, 4)
+    a, b = x[..., 0, :, :], x[..., 1, :, :]
+    ss = _fma(a[..., 0], a[..., 0], a[..., 1] * a[..., 1])
+    for v in (a[..., 2], a[..., 3], b[..., 0], b[..., 1], b[..., 2], b[..., 3]):
+        ss = _fma(v, v, ss)
+    while ss.shape[-1] > 1:
+        ss = ss[..., 0::2] + ss[..., 1::2]
+    r = np.float32(1) / np.sqrt(_fma(ss, np.float32(1 / 128), np.float32(eps)))[..., None]
+    sn, cs = (t.reshape(t.shape[:-1] + (16, 4)) for t in (sin, cos))
+    av, bv = a * w[0] * r, b * w[1] * r
+    lo, hi = _fma(av, cs, -(bv * sn)), _fma(av, sn, bv * cs)
+    return synth.f32_to_bf16_bits(np.stack([lo, hi], axis=-3).reshape(rows.shape).astype(np.float32))
+
+
+def _append_positions(dev, n_q, n_kv, count, k_new, v_new, w, eps=1e-6):
+    """`count` positions appended one call after the other to an empty cache; the cached K rows and the tables' rows."""
+    kv_dim = n_kv * D
+    kc, vc = (torch.zeros(count, kv_dim, dtype=torch.int16, device=dev) for _ in "kv")
+    ws = torch.zeros(ops.workspace_bytes(n_q, D, count) // 4, dtype=torch.float32, device=dev)
+    sin, cos = ops.sincos_table(D, count, dev)
+    k_d, v_d, w_d = to_dev(k_new, dev), to_dev(v_new, dev), to_dev(w, dev)
+    q_d, out = torch.zeros(n_q * D, dtype=torch.int16, device=dev), torch.zeros(n_q * D, dtype=torch.int16, device=dev)
+    for pos in range(count):
+        ops.mha_decode_append(q_d, k_d[pos], v_d[pos], w_d, sin, cos, kc, vc, out, ws, layer_id=0, pos=pos, kv_dim=kv_dim, kv_mul=n_q // n_kv,
+                              head_num=n_q, head_dim=D, max_seq_len=count, kv_layout=B.KV_LAYOUT_POS_MAJOR, eps=eps)
+    torch.cuda.synchronize()
+    assert np.array_equal(vc.cpu().numpy().view(np.uint16), v_new)
+    tables = (t.cpu().numpy().reshape(count, 1, D // 2) for t in (sin, cos))
+    return (kc.cpu().numpy().view(np.uint16).reshape(count, n_kv, D), *tables)
+
+
+@pytest.mark.parametrize("group", [1, 3, 4, 8, 16])
+def test_key_rows_have_the_bits_of_the_declared_chain(dev, group):
+    """A last fp32 bit turns a bf16 rounding once in some ten thousand values: half a million of them, every one the chain's."""
+    n_kv, count = 32, 128
+    rng = np.random.RandomState(group)
+    bits = lambda *shape: synth.f32_to_bf16_bits(rng.standard_normal(shape).astype(np.float32))
+    k_new, v_new, w = bits(count, n_kv * D), bits(count, n_kv * D), synth.f32_to_bf16_bits(1 + 0.02 * rng.standard_normal(2 * D).astype(np.float32))
+    got, sin, cos = _append_positions(dev, group * n_kv, n_kv, count, k_new, v_new, w)
+    want = _chain(k_new.reshape(count, n_kv, D), w[D:], sin, cos, 1e-6)
+    assert np.array_equal(got, want), "%d of %d values differ" % ((got != want).sum(), want.size)
