@@ -129,3 +129,51 @@ def test_key_rows_have_the_bits_of_the_declared_chain(dev, group):
     got, sin, cos = _append_positions(dev, group * n_kv, n_kv, count, k_new, v_new, w)
     want = _chain(k_new.reshape(count, n_kv, D), w[D:], sin, cos, 1e-6)
     assert np.array_equal(got, want), "%d of %d values differ" % ((got != want).sum(), want.size)
+
+
+# Value rows whose mean square, with eps, lies outside the range of the reciprocal root, or is nothing at all.
+NEIGHBOURS = [(1e16, 1e-6), (float("inf"), 1e-6), (float("nan"), 1e-6), (0.0, 0.0)]
+
+
+def _with_values(count, n_kv, value, seed):
+    rng = np.random.RandomState(seed)
+    row = lambda *shape: rng.standard_normal(shape).astype(np.float32)
+    k_new, w = synth.f32_to_bf16_bits(row(count, n_kv * D)), synth.f32_to_bf16_bits(1 + 0.02 * row(2 * D))
+    return k_new, np.broadcast_to(synth.f32_to_bf16_bits(np.float32([value])), k_new.shape).copy(), w
+
+
+@pytest.mark.parametrize("value,eps", NEIGHBOURS)
+@pytest.mark.parametrize("group", [2, 4, 5])  # (the key row's neighbour: the value row, or the last query row, here all zeros)
+def test_a_rows_neighbours_leave_no_trace(dev, group, value, eps):
+    n_kv, count = 32, 128
+    k_new, v_new, w = _with_values(count, n_kv, value, group)
+    got, sin, cos = _append_positions(dev, group * n_kv, n_kv, count, k_new, v_new, w, eps)
+    assert np.array_equal(got, _chain(k_new.reshape(count, n_kv, D), w[D:], sin, cos, eps))
+
+
+@pytest.mark.parametrize("value,eps", NEIGHBOURS)
+@pytest.mark.parametrize("chained", [False, True])
+def test_a_rows_neighbours_leave_no_trace_in_a_stack(dev, chained, value, eps):
+    """The same in the multi-layer launches, whose key rows have a wavefront to themselves: independent layers and a chain. From 300 cached
+    positions on, where each is one launch."""
+    n_q, n_kv, layers, first, count = 32, 8, 32, 300, 16
+    dim, kv_dim = n_q * D, n_kv * D
+    k_new, v_new, w = _with_values(count * layers, n_kv, value, 77)
+    k_d, v_d, w_d = (to_dev(x, dev) for x in (k_new, v_new, np.tile(w, (layers, 1))))
+    kc, vc = (torch.zeros(layers, first + count, kv_dim, dtype=torch.int16, device=dev) for _ in "kv")
+    ws = torch.zeros(ops.workspace_bytes(n_q, D, first + count) // 4, dtype=torch.float32, device=dev)
+    sin, cos = ops.sincos_table(D, first + count, dev)
+    q = torch.full(((layers + 1) * dim,), 0x3F80, dtype=torch.int16, device=dev)
+    out = q[dim:] if chained else torch.zeros(layers * dim, dtype=torch.int16, device=dev)
+    for i in range(count):
+        rows = slice(i * layers, (i + 1) * layers)
+        n = ops.mha_decode_append_stack(q, k_d[rows], v_d[rows], w_d, sin, cos, kc, vc, out, ws, layer_id=0, layer_count=layers, pos=first + i,
+                                        kv_dim=kv_dim, kv_mul=n_q // n_kv, head_num=n_q, head_dim=D, max_seq_len=first + count,
+                                        kv_layout=B.KV_LAYOUT_POS_MAJOR, query_stride=dim, key_new_stride=kv_dim, value_new_stride=kv_dim,
+                                        norm_weight_stride=2 * D, output_stride=dim, eps=eps)
+        assert n == 1
+    torch.cuda.synchronize()
+    got = kc[:, first:].cpu().numpy().view(np.uint16).reshape(layers, count, n_kv, D)
+    tables = (t.cpu().numpy().reshape(-1, 1, D // 2)[first:] for t in (sin, cos))
+    raw = k_new.reshape(count, layers, n_kv, D).transpose(1, 0, 2, 3)
+    assert np.array_equal(got, _chain(raw, w[D:], *tables, eps))
