@@ -378,8 +378,8 @@ __device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4
     float p[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) p[e] = fast_exp2(s[e] - m_new);
+    const float l_old = l_run;
     l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
-    const float m_old = m_run;
     m_run = m_new;
     // The probabilities enter the second MFMA as a sum of two bf16 numbers
     // (p = hi + lo, relative error 2^-17), so that the product keeps fp32-like accuracy.
@@ -387,10 +387,12 @@ __device__ __forceinline__ void fold_tile(const TileRegs& r, const u32x4 (&qb)[4
     const uint32_t p23 = pack_bf16(p[2], p[3]);
     const uint32_t q01 = pack_bf16(p[0] - bf16_lo(p01), p[1] - bf16_hi(p01));
     const uint32_t q23 = pack_bf16(p[2] - bf16_lo(p23), p[3] - bf16_hi(p23));
-    // Rescale only when some head's max moved from one there was (wave-uniform test): a wavefront's first tile finds zeros. (Short contexts are
+    // Rescale only when the max moved of some head that has summed anything (wave-uniform test): a wavefront's first tile finds zeros. (The sum
+    // says so, not the max: a wavefront that started from the new token holds its V row with weight 1 whatever its score, -inf
+    // included; where a head has accumulators some lane of its column has a sum, that of its largest score.) (Short contexts are
     // one tile a wavefront; a layer of a captured step, 64 Q / 8 KV heads, first tile rescaled : not, us: 6.28 : 6.14 at 1000 positions,
     // 7.22 : 7.04 at 2500.) The factor of head 4*kg + r sits in lane 4*kg + r of this lane's 16-lane row.
-    if (__any(alpha != 1.0f && m_old != -INFINITY)) {
+    if (__any(alpha != 1.0f && l_old != 0.0f)) {
         static_for<0, 4>([&](auto rr) {
             float ar;
             if constexpr (G <= 4) ar = row_bcast<rr.value>(alpha);  // only row kg = 0 holds heads
