@@ -13,7 +13,7 @@
 //     inside the same launch (fused combine).
 // Three more template switches: APPEND folds the per-token QK-Norm + RoPE and the
 // K/V cache append of the reference's layer loop into the launch (the new row
-// enters the softmax from registers), DYN reads the position from device memory
+// enters the softmax from the workgroup's own LDS), DYN reads the position from device memory
 // so that one captured launch serves every token, STAGGER makes the splits of the
 // position-major layout walk their tiles from different starting points.
 //
@@ -102,8 +102,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     // splits or all of them, nearly as the host would have planned (dyn_split_rule) --, and the splits that are not needed leave at once.
     // 32 Q / 8 KV heads, append variant in a captured 36-layer step sized for 8192 positions, us per layer, all splits as far as
     // there are tiles : the rule: 5.58 : 4.02 at 60 positions, 5.51 : 5.33 at 170, 5.65 : 5.36 at 300, 5.73 : 5.40 at 600.
-    // Append variant: the new token's row never comes from the cache (its K and V are in registers
-    // and go straight into the running softmax of one wave), so the tiles cover positions 0 .. pos-1.
+    // Append variant: the new token's row never comes from the cache (its K and V rows lie finished in LDS, where the running
+    // softmax of one wave starts from them), so the tiles cover positions 0 .. pos-1.
     int seq_len = a.seq_len, n_active = a.num_splits;
     // (the host never asks for more splits than tiles; 0 tiles: 1 split). The division is done on
     // the host when the position is known there: it is 33 instructions in front of the first load.
@@ -324,7 +324,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
 #endif
     };
 
-    // Wave w owns tiles w, w+NW, ...: NSTAGE of them are always in flight.
+    // Wave w owns tiles w, w+NW, ...: NSTAGE of them are in flight throughout the loop (append variant: one until the rows are done).
     const int n_my = wave < ntiles ? (ntiles - wave + NW - 1) / NW : 0;
     // STAGGER: the splits of a head walk their tiles from different starting points (split s starts
     // s & a.stagger tiles into its wave's sequence and wraps round), so that workgroups running in
