@@ -261,6 +261,7 @@ __device__ __forceinline__ float four_pairs_squared(const float (&a)[4], const f
     for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(b[e], b[e], ss);
     return ss;
 }
+__device__ __forceinline__ float mean_square(float ss, float eps) { return __builtin_fmaf(ss, 1.0f / kHeadDim, eps); }
 // 1 / sqrt(mean square + eps), root and division each rounded correctly, in six dependent instructions where the compiler has some 30
 // for them: the hardware's reciprocal root (1 ulp), a root from it and its residual, a reciprocal from both and its residual. Such a reciprocal
 // is the correctly rounded one unless the mantissa it divides by is all ones (P. Markstein, IBM J. Res. Dev. 34 (1990) 111), which is the root of
@@ -269,7 +270,7 @@ __device__ __forceinline__ float four_pairs_squared(const float (&a)[4], const f
 // 1.0f / sqrtf(x) for all : this, us: 32 Q / 8 KV heads 4.79 : 4.81 at 300 positions, 5.11 : 5.08 at 1100, 7.07 : 7.02 at 4000, 64 Q heads 5.79 : 5.78 at
 // 1000, 7.87 : 7.83 at 5000.)
 __device__ __forceinline__ float inverse_rms(float ss, float eps) {
-    const float x = __builtin_fmaf(ss, 1.0f / kHeadDim, eps);
+    const float x = mean_square(ss, eps);
     const uint32_t u = __builtin_bit_cast(uint32_t, x);
     constexpr uint32_t lo = __builtin_bit_cast(uint32_t, 1e-30f), hi = __builtin_bit_cast(uint32_t, 1e30f);
     if (__builtin_expect(__any(u - lo > hi - lo || (u & 0x7ffffeu) == 0x7ffffeu), 0)) return 1.0f / sqrtf(x);
@@ -289,7 +290,11 @@ __device__ __forceinline__ void rotate_pair(float a, float b, float wa, float wb
 // takes elements 4*(p&1) .. +3 of 16-byte chunk p>>1 and of its rotary partner, chunk (p>>1) + 8,
 // so a lane touches 8 elements, reads only what it overwrites, and the sum of squares is one
 // DPP row fold. `w`: the 256-byte norm weights; `sin16` / `cos16`: the 64 sines / cosines of the
-// position (lane p needs exactly 16-byte chunk p of each).
+// position (lane p needs exactly 16-byte chunk p of each). SHORT_ROOT: both ways have the same bits. The chain of layers, whose
+// every wavefront waits for this, loses more by the short root's test and branch than it saves (36 layers of 32 Q / 8 KV heads at 4096 positions
+// short root : without, us: 253.3 : 252.1, 28 of 16 Q heads at 1100 156.7 : 155.3); a KV head at a time it is the better one (36 layers
+// at 4096 94.66 : 94.95).
+template <bool SHORT_ROOT>
 __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, const char* sin16, const char* cos16,
                                                    int row, int p, float eps) {
     const int c = p >> 1, hf = p & 1;
@@ -311,7 +316,7 @@ __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, co
     ss += dpp_partner<0x4E>(ss);
     ss += dpp_partner<0x141>(ss);
     ss += dpp_partner<0x140>(ss);
-    const float r = inverse_rms(ss, eps);
+    const float r = SHORT_ROOT ? inverse_rms(ss, eps) : 1.0f / sqrtf(mean_square(ss, eps));
     float ol[4], oh[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) rotate_pair(a[e], b[e], wa[e], wb[e], r, sn[e], cs[e], ol[e], oh[e]);

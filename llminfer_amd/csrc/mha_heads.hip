@@ -200,9 +200,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
         char* ops = operands + set * kOperandBytes;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-        for (int b4 = 0; b4 < kQSlots; ++b4) norm_rope_rows_lds(ops + 2048, ops, ops + 512, ops + 768, 4 * b4 + kg, n16, a.eps);
+        for (int b4 = 0; b4 < kQSlots; ++b4) norm_rope_rows_lds<true>(ops + 2048, ops, ops + 512, ops + 768, 4 * b4 + kg, n16, a.eps);
         if (it.hi == S) {
-            norm_rope_rows_lds(ops + 1024, ops + 256, ops + 512, ops + 768, 0, n16, a.eps);
+            norm_rope_rows_lds<true>(ops + 1024, ops + 256, ops + 512, ops + 768, 0, n16, a.eps);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             const u32x4* rows = reinterpret_cast<const u32x4*>(ops + 1024);
             const int64_t row_off = (int64_t)it.layer * ha.st.cache_stride + (int64_t)cached_len * a.row_stride + it.kvh * a.slot_head_stride;

@@ -280,9 +280,9 @@ __global__ __launch_bounds__(NW * 64, 2) void mha_stack_kernel(StackArgs sa) {
             const u32x4* rows4 = reinterpret_cast<const u32x4*>(my_rows);
 #pragma unroll
             for (int b4 = 0; b4 < kQSlots; ++b4)
-                norm_rope_rows_lds(my_rows, shared_staging, shared_staging + 512, shared_staging + 768, 4 * b4 + kg, n16, a.eps);
+                norm_rope_rows_lds<false>(my_rows, shared_staging, shared_staging + 512, shared_staging + 768, 4 * b4 + kg, n16, a.eps);
             if (holds_new_row)
-                norm_rope_rows_lds(shared_staging + 1024, shared_staging + 256, shared_staging + 512, shared_staging + 768, 0, n16, a.eps);
+                norm_rope_rows_lds<false>(shared_staging + 1024, shared_staging + 256, shared_staging + 512, shared_staging + 768, 0, n16, a.eps);
             const int hq_local = min(n16, a.group - 1);
             const bool live = n16 < a.group;
 #pragma unroll
@@ -799,9 +799,9 @@ __global__ __launch_bounds__(kLayersWaves * 64, 2) void mha_layers_kernel(StackA
             set = set + 1 == kOperandSets ? 0 : set + 1;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (p + 1 < L) fetch(p + 1, set);
-            norm_rope_rows_lds(ops + 2048, ops, ops + 512, ops + 768, kg, n16, a.eps);
+            norm_rope_rows_lds<true>(ops + 2048, ops, ops + 512, ops + 768, kg, n16, a.eps);
             if (holds_new_row) {
-                norm_rope_rows_lds(ops + 1024, ops + 256, ops + 512, ops + 768, 0, n16, a.eps);
+                norm_rope_rows_lds<true>(ops + 1024, ops + 256, ops + 512, ops + 768, 0, n16, a.eps);
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 const u32x4* rows = reinterpret_cast<const u32x4*>(ops + 1024);
                 const int64_t row_off = (int64_t)p * sa.cache_stride + (int64_t)(seq_len - 1) * a.row_stride + kvh * a.slot_head_stride;
