@@ -122,6 +122,9 @@ __global__ __launch_bounds__(NW * 64) void stream_tiles_kernel(const char* __res
     const int begin = split * run + min(split, longer);
     const char* kb = k + kvh * head_bytes + (int64_t)begin * 16 * rs;
     const char* vb = v + kvh * head_bytes + (int64_t)begin * 16 * rs;
+    // (the division above runs on the vector ALU: a scalar register it ends up in may be read by a memory instruction five wait states after the
+    // lane read that fills it, which the compiler does not see to in front of an asm statement)
+    asm volatile("s_nop 4" : "+s"(kb), "+s"(vb));
     const int n_my = wave < ntiles ? (ntiles - wave + NW - 1) / NW : 0;
     const int rot = min(split & rot_mask, max(n_my - 1, 0));
     auto tile_of = [&](int i) {
