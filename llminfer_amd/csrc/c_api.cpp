@@ -612,13 +612,14 @@ static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan,
     if (cus <= 0 || heads > INT32_MAX / 64) return false;
     if (heads < kFewestHeads) return false;
     // What either side takes, in us (fitted to sweeps of 4 to 64 layers, 32 to 20000 positions, groups of 1 to 8; within a tenth
-    // mostly). Here a split costs a workgroup a fixed part (folding, the barrier) and its wavefronts' tiles, all of them share the
+    // mostly). Here a split, or a round of splits side by side (short ones: within a quarter), costs a workgroup a fixed part (folding, the barrier) and its wavefronts' tiles, all of them share the
     // memory's rate, and cut heads are handed over at the end: 8 layers at 2048 positions, 2 : 4 : 8 : 16 : 32 splits, 26.9 : 28.8 : 31.8 :
     // 38.0 : 48.8 (four wavefronts), 27.3 : 28.4 : 31.3 : 38.2 : 62.9 (eight). Both sides near the line, this form : the other one: 36 layers
     // of 32 Q heads at 4096 96 : 107, 30 at 3000 69 : 75, 24 at 4000 75 : 74, 28 at 2000 50 : 55, 16 at 2000 50 : 33, 10 of 16 Q heads at
     // 600 16 : 17, 6 of 32 Q heads at 20000 89 : 81; groups of 8 (one launch per layer) 8 at 300 33 : 50, 4 at 6000 26 : 34.
     const double head_bytes = 4.0 * m.pos * m.head_dim, rate = 6.4e6;
-    const int tiles_per_wave = ceil_div(std::max(ceil_div(tiles, plan.num_splits), 1), waves);
+    const int most = std::max(ceil_div(tiles, plan.num_splits), 1), at_once = heads_splits_at_once(plan.num_splits, most, waves);
+    const int tiles_per_wave = ceil_div(most, waves);
     const double split_us = waves == 8 ? 0.8 + 1.2 * tiles_per_wave : 0.75 + 0.57 * tiles_per_wave;
     const int64_t rounds = heads / cus;
     const int rest = (int)(heads % cus);
@@ -630,8 +631,8 @@ static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan,
         f.grid = (int)std::min<int64_t>(items, cus);
         if (parts > 1 && (rest == 0 || (int64_t)rest * parts > cus || f.grid % parts != 0)) continue;
         if (heads_workspace(m, f, plan.num_splits) > (m.workspace ? m.workspace_bytes : 0)) continue;
-        double us = 4.0 + (double)rounds * phase(cus, plan.num_splits);
-        if (rest > 0) us += phase(rest, ceil_div(plan.num_splits, parts)) + (parts > 1 ? 3.0 : 0.0);
+        double us = 4.0 + (double)rounds * phase(cus, ceil_div(plan.num_splits, at_once));
+        if (rest > 0) us += phase(rest, ceil_div(ceil_div(plan.num_splits, parts), at_once)) + (parts > 1 ? 3.0 + 0.05 * ceil_div(plan.num_splits, parts) : 0.0);
         if (form->grid == 0 || us < best) {
             best = us;
             *form = f;

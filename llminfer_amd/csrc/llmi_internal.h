@@ -108,6 +108,12 @@ int stack_regions(const llmi_mha_args& m, const llmi_mha_plan& plan, int layer_c
 struct HeadsForm {
     int grid, parts, cut_heads, waves;
 };
+// Splits of a head mha_heads.hip takes at a time: `waves` wavefronts stream, a split has `most` tiles at most.
+inline int heads_splits_at_once(int splits, int most, int waves) {
+    int p = 1;
+    while (2 * p <= splits && 2 * p <= waves && 2 * p * most <= waves) p *= 2;
+    return p;
+}
 int launch_mha_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan, const HeadsForm& form);
 // Bytes of the workspace the parts hand their results over in.
 size_t heads_workspace(const llmi_mha_args& m, const HeadsForm& form, int num_splits);

@@ -146,10 +146,19 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 
+// The bases of the dma16 loads that follow, in scalar registers and there for long enough: a scalar register that a vector instruction has
+// written (v_readfirstlane, which is how the compiler brings a value it has computed in vector registers, a clamp by v_med3 is enough, over to
+// dma16's operand) may be read by a memory instruction five wait states later at the earliest, and the compiler, which counts them
+// elsewhere, does not look into an asm statement. For callers whose bases are computed as they go.
+__device__ __forceinline__ void scalar_bases(const char*& a, const char*& b) {
+    asm volatile("s_nop 4" : "+s"(a), "+s"(b));
+}
+
 // 16 bytes per lane from global memory straight into LDS, no VGPR round trip:
 // lane L's bytes land at lds_off + 16*L. `base` and `lds_off` are wave-uniform,
 // `voff` is the lane's byte offset from base. Counted by vmcnt like any load.
 __device__ __forceinline__ void dma16(const char* base, uint32_t voff, uint32_t lds_off) {
+    // (`base` in scalar registers already: see scalar_bases.)
     // The instruction takes its base and the LDS offset (through M0) from scalar
     // registers; readfirstlane guarantees that whatever the surrounding code
     // made of these wave-uniform values (it is free when they already are scalar).

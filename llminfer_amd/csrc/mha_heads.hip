@@ -13,9 +13,9 @@
 // parts of a head, the last part the highest: the only wait (bounded) is for workgroups that were started earlier and wait for nobody.
 //
 // us, this form : the stream by layers (mha_layers_kernel), 32 Q / 8 KV heads: 36 layers at 4096 + 1 positions 96-102 : 108 (6.1 TB/s), at
-// 300 32 : 54, 64 layers at 1000 55 : 109; 28 layers of 16 Q heads at 1000 27 : 45. Against one launch per layer, 64 Q / 8 KV heads:
-// 64 layers at 3000 144 : 476, 36 at 1000 45 : 234, 8 at 300 33 : 50; single passes, 12 layers of 32 Q heads at 150 9 : 55. With one tile
-// per wavefront and split it is the work between tiles that bounds it, 0.75 us per split (0.57 per tile): instructions, one or two
+// 300 22 : 54, 64 layers at 1000 55 : 109; 28 layers of 16 Q heads at 1000 27 : 45. Against one launch per layer, 64 Q / 8 KV heads:
+// 64 layers at 3000 144 : 476, 36 at 1100 52 : 234, 8 at 300 11 : 50; single passes, 12 layers of 32 Q heads at 150 9 : 55. With one tile
+// per wavefront and round it is the work between tiles that bounds it, 0.75 us per round (0.57 per tile): instructions, one or two
 // wavefronts to a SIMD.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -30,11 +30,19 @@ constexpr int kMaxSplitsKept = 32;  // splits of a head, at most: half of their 
 
 // NW wavefronts (of eight) stream, with a ring of NSTAGE tiles each: as many as a split has in the launch this stands for. With four
 // the others fold and bring in operands.
-template <int G, int NW, int NSTAGE>
+// P: splits at a time. Where a split has no more than NW / P tiles, P consecutive splits are taken side by side, T = NW / P wavefronts each, a tile or
+// none to a wavefront: a round (its tile, the barrier, the folds) costs about the same whatever it holds, and with one split a round most
+// wavefronts had nothing to do in it. A wavefront without a tile adds nothing to a fold (weight zero), so the bits are those of NW wavefronts.
+// us, one split at a time : side by side, groups of 8 (eight wavefronts): 64 layers at 250 positions 56.2 : 25.6, 23 at 384 31.0 : 16.8, 64 at 900 62.0 : 48.3,
+// 36 at 1100 71.5 : 52.1, 20 at 1900 59.9 : 43.9, 4 at 300 12.2 : 10.4; groups of 4 (four wavefronts) 36 at 300 29.5 : 21.8, 64 at 400 44.3 : 29.5, 20 at 200
+// 13.7 : 10.2; groups of 2 28 at 500 21.7 : 15.8, 4 at 200 level.
+template <int G, int NW, int NSTAGE, int P>
 __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha) {
     const KernelArgs& a = ha.st.a;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int T = NW / P;
+    const int sub = P == 1 ? 0 : wave / T, tw = P == 1 ? wave : wave % T;  // streaming: which split of a round, which of its tiles first
     const int n16 = lane & 15;
     const int kg = lane >> 4;
     const int S = a.num_splits;
@@ -92,14 +100,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
         return it;
     };
     struct Unit {
-        int begin, nrows, n_my;
+        int nrows, n_my;
     };
     auto unit_at = [&](int split) {
         Unit u;
         const int ntiles = run + (split < longer ? 1 : 0);
-        u.begin = (split * run + min(split, longer)) * kTile;
-        u.nrows = min(ntiles * kTile, cached_len - u.begin);
-        u.n_my = wave < ntiles ? (ntiles - wave + NW - 1) / NW : 0;
+        u.nrows = min(ntiles * kTile, cached_len - (split * run + min(split, longer)) * kTile);
+        u.n_my = tw < ntiles ? (ntiles - tw + T - 1) / T : 0;
         return u;
     };
 
@@ -120,26 +127,28 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
     int is_begin = 0, is_nrows = 0, is_n = 0;  // the split's first position and rows, the wavefront's tiles of it
     const char *is_kb = nullptr, *is_vb = nullptr;
     auto open_item = [&]() {
-        is_split = is_it.lo;
+        is_split = is_it.lo + sub;
         is_begin = (is_split * run + min(is_split, longer)) * kTile;
         const int64_t off = (int64_t)is_it.layer * ha.st.cache_stride + (int64_t)is_it.kvh * a.head_stride + (int64_t)is_begin * a.row_stride;
         is_kb = reinterpret_cast<const char*>(a.k + off);
         is_vb = reinterpret_cast<const char*>(a.v + off);
     };
     auto open_split = [&]() {
-        const int ntiles = run + (is_split < longer ? 1 : 0);
+        const int ntiles = P > 1 && is_split >= is_it.hi ? 0 : run + (is_split < longer ? 1 : 0);
         is_nrows = min(ntiles * kTile, cached_len - is_begin);
-        is_n = wave < ntiles ? (ntiles - wave + NW - 1) / NW : 0;
+        is_n = tw < ntiles ? (ntiles - tw + T - 1) / T : 0;
         is_tile = 0;
     };
     // To the wavefront's next split with a tile for it. (A head's splits follow one another in memory.)
     auto next_split = [&]() {
         do {
-            const int ntiles = run + (is_split < longer ? 1 : 0);
-            is_begin += ntiles * kTile;
-            is_kb += (uint32_t)(ntiles * kTile) * rs;
-            is_vb += (uint32_t)(ntiles * kTile) * rs;
-            if (++is_split >= is_it.hi) {
+            // (rows of this split and the P - 1 behind it)
+            const int rows = (P == 1 ? run + (is_split < longer ? 1 : 0) : P * run + min(is_split + P, longer) - min(is_split, longer)) * kTile;
+            is_begin += rows;
+            is_kb += (uint32_t)rows * rs;
+            is_vb += (uint32_t)rows * rs;
+            is_split += P;
+            if (is_split >= is_it.hi) {
                 is_item += stride;
                 if (is_item >= items) {
                     is_live = false;
@@ -155,8 +164,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
         if (!is_live) return;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's previous contents have reached the VGPRs
         const uint32_t last_off = (uint32_t)(is_nrows - 1) * rs;  // (rows past the split's last one: masked out of the softmax)
-        const uint32_t base = (uint32_t)(wave + is_tile * NW) * (kTile * rs);
+        const uint32_t base = (uint32_t)(tw + is_tile * T) * (kTile * rs);
         const uint32_t slot = my_ring_lds + (uint32_t)is_stage * kStageBytes;
+        if constexpr (P > 1) scalar_bases(is_kb, is_vb);  // (one split at a time they are scalar throughout)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t ko = min(base + k_row + (uint32_t)(4 * i) * rs, last_off) + ((i & 1) ? k_col1 : k_col0);
@@ -257,15 +267,17 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
             qb[j] = live ? qv : u32x4{0u, 0u, 0u, 0u};
         }
     };
-    // A split's tiles folded, and the wavefront's result left in LDS.
-    auto stream_split = [&](int split, int op_set, int fold_set) {
+    // The wavefront's tiles of its split of the round, `round` the first one, folded, and its result left in LDS.
+    auto stream_round = [&](const Item& it, int round, int op_set, int fold_set) {
+        const int split = round + sub;
+        if (P > 1 && split >= it.hi) return;  // (nobody folds it)
         const u32x4* ops4 = reinterpret_cast<const u32x4*>(operands + op_set * kOperandBytes);
         const Unit u = unit_at(split);
         float m_run = -INFINITY, l_run = 0.0f;
         f32x4 o[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (split == S - 1 && wave == 0) {
+        if (split == S - 1 && tw == 0) {
             u32x4 kf[4], vf;
             start_from_new_row(ops4 + 64, ops4 + 80, qb, kg, n16, a.scale_log2e, kf, vf, m_run, l_run, o);
         }
@@ -283,7 +295,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
             rd_stage = rd_stage + 1 == NSTAGE ? 0 : rd_stage + 1;
             --in_flight;
             issue_next();
-            fold_tile<G>(r, qb, (wave + i * NW) * kTile + 4 * kg, u.nrows, a.scale_log2e, m_run, l_run, o);
+            fold_tile<G>(r, qb, (tw + i * T) * kTile + 4 * kg, u.nrows, a.scale_log2e, m_run, l_run, o);
         }
         l_run = rows_sum(l_run);
 #pragma unroll
@@ -301,22 +313,23 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
         }
     };
     // The wavefronts' results of a split into one row.
-    auto fold_split = [&](const Item& it, int split, int fold_set) {
-        float mw[NW], lw[NW];
-        f32x4 ow[NW];
+    auto fold_split = [&](const Item& it, int round, int split, int fold_set) {
+        const int w0 = P == 1 ? 0 : (split - round) * T;
+        float mw[T], lw[T];
+        f32x4 ow[T];
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            mw[w] = *fold_m(fold_set, w, fh);
-            lw[w] = *fold_l(fold_set, w, fh);
-            ow[w] = *reinterpret_cast<const f32x4*>(fold_o(fold_set, w, fh) + c4 * 4);
+        for (int w = 0; w < T; ++w) {
+            mw[w] = *fold_m(fold_set, w0 + w, fh);
+            lw[w] = *fold_l(fold_set, w0 + w, fh);
+            ow[w] = *reinterpret_cast<const f32x4*>(fold_o(fold_set, w0 + w, fh) + c4 * 4);
         }
         float mx = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) mx = fmaxf(mx, mw[w]);
+        for (int w = 0; w < T; ++w) mx = fmaxf(mx, mw[w]);
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         float lsum = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
+        for (int w = 0; w < T; ++w) {
             const float f = (mw[w] == -INFINITY) ? 0.0f : fast_exp2(mw[w] - mx);
             acc += ow[w] * f;
             lsum += lw[w] * f;
@@ -447,8 +460,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
             for (int item = item0; item < items; item += stride) {
                 const Item it = item_at(item);
                 read_query(op_set);
-                for (int split = it.lo; split < it.hi; ++split) {
-                    stream_split(split, op_set, fold_set);
+                for (int round = it.lo; round < it.hi; round += P) {
+                    stream_round(it, round, op_set, fold_set);
                     meet();
                     fold_set ^= 1;
                 }
@@ -464,11 +477,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
         const bool more = item + stride < items;
         if (wave == kOperandWave && more) fetch_operands(item_at(item + stride), op_set ^ 1);
         if constexpr (NW == 8) read_query(op_set);
-        for (int split = it.lo; split < it.hi; ++split) {
-            if constexpr (NW == 8) stream_split(split, op_set, fold_set);
-            if (wave == kOperandWave && more && split + 1 == it.hi) prepare_operands(item_at(item + stride), op_set ^ 1);
+        for (int round = it.lo; round < it.hi; round += P) {
+            if constexpr (NW == 8) stream_round(it, round, op_set, fold_set);
+            if (wave == kOperandWave && more && round + P >= it.hi) prepare_operands(item_at(item + stride), op_set ^ 1);
             meet();
-            if (folds_here && (split & 1) == parity) fold_split(it, split, fold_set);
+            if constexpr (P == 1) {
+                if (folds_here && (round & 1) == parity) fold_split(it, round, round, fold_set);
+            } else if (folds_here) {
+                for (int split = round + ((round ^ parity) & 1); split < min(round + P, it.hi); split += 2) fold_split(it, round, split, fold_set);
+            }
             fold_set ^= 1;
         }
         hand_over(it);
@@ -482,10 +499,26 @@ __global__ __launch_bounds__(kWaves * 64, 2) void mha_heads_kernel(HeadsArgs ha)
 
 template <int G>
 void launch_g(const HeadsArgs& ha, int grid, int waves, hipStream_t stream) {
-    if (waves == 4) {
-        if constexpr (G <= 4) hipLaunchKernelGGL((mha_heads_kernel<G, 4, 4>), dim3(grid), dim3(kWaves * 64), 0, stream, ha);
+    const int splits = ha.st.a.num_splits, most = ha.st.a.tiles_run + (ha.st.a.tiles_longer > 0 ? 1 : 0);  // tiles of a split, at most
+    const int at_once = heads_splits_at_once(splits, most, waves);
+    auto launch = [&](auto nw, auto stages, auto p) {
+        hipLaunchKernelGGL((mha_heads_kernel<G, decltype(nw)::value, decltype(stages)::value, decltype(p)::value>), dim3(grid), dim3(kWaves * 64), 0, stream, ha);
+    };
+    const std::integral_constant<int, 1> one{};
+    const std::integral_constant<int, 2> two{};
+    const std::integral_constant<int, 4> four{};
+    const std::integral_constant<int, 8> eight{};
+    if constexpr (G <= 4) {
+        // (eight wavefronts: a single pass)
+        if (waves == 8) launch(eight, one, one);
+        else if (at_once >= 4) launch(four, four, four);
+        else if (at_once >= 2) launch(four, four, two);
+        else launch(four, four, one);
     } else {
-        hipLaunchKernelGGL((mha_heads_kernel<G, 8, 1>), dim3(grid), dim3(kWaves * 64), 0, stream, ha);
+        if (at_once >= 8) launch(eight, one, eight);
+        else if (at_once >= 4) launch(eight, one, four);
+        else if (at_once >= 2) launch(eight, one, two);
+        else launch(eight, one, one);
     }
 }
 

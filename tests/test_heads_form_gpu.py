@@ -61,3 +61,25 @@ def test_cut_heads_give_up_with_nan_instead_of_hanging(dev):
     c = st.fresh()
     assert st.run_stack(c) == 1
     assert torch.equal(c["out"], a["out"]) and timeouts() == after
+
+
+@pytest.mark.parametrize("layers,ctx,n_q,n_kv,layout", [
+    (5, 250, 64, 8, HEAD),    # 16 splits of a tile each: eight at a time
+    (5, 257, 64, 8, POS),     # one of them has two: four
+    (33, 256, 40, 8, HEAD),   # ... cut heads, groups of five
+    (4, 512, 64, 8, HEAD),    # two each, whole
+    (4, 513, 64, 8, HEAD),    # three: two at a time
+    (6, 1023, 64, 8, POS),    # four, the last one ragged
+    (5, 1041, 64, 8, HEAD),   # 32 splits of two or three
+    (36, 2048, 64, 8, HEAD),  # ... of four, cut heads
+    (4, 2049, 64, 8, HEAD),   # five: one at a time
+    (9, 186, 32, 8, HEAD),    # four wavefronts: 8 splits of one or two, two at a time
+    (9, 256, 24, 8, POS),     # 16 of a tile each, four at a time, groups of three
+    (33, 256, 16, 8, HEAD),   # ... cut heads
+    (5, 500, 32, 8, HEAD),    # two each
+    (35, 512, 8, 8, HEAD),    # ... whole, cut heads
+    (5, 513, 32, 8, HEAD),    # three: one at a time
+    (12, 300, 16, 4, HEAD),   # 19 splits, an odd number, of a tile each
+])
+def test_splits_side_by_side_give_the_bits_of_one_launch_per_layer(dev, layers, ctx, n_q, n_kv, layout):
+    independent.test_independent_layers_give_the_bits_of_one_launch_per_layer(dev, layers, ctx, n_q, n_kv, layout, None, None, {})
