@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "llmi_internal.h"
@@ -186,6 +187,7 @@ static int fill_kernel_args(const llmi_mha_args& args, const llmi_mha_plan& plan
     if (args.pos_device) {
         if (plan.num_splits > 1) dyn_split_rule(args, plan, append != nullptr, &ka.dyn_single, &ka.dyn_quarter, &ka.dyn_half);
         const int32_t counts[3] = {ka.dyn_quarter, ka.dyn_half, plan.num_splits};
+        ka.dyn_full = plan.num_splits > 1 ? std::max({4 * ka.dyn_half, ka.dyn_single, plan.num_splits}) : INT32_MAX;
         for (int i = 0; i < 3; ++i) ka.dyn_magic[i] = counts[i] > 1 ? (uint32_t)(((1ull << 32) + counts[i] - 1) / counts[i]) : 0u;
     }
     ka.max_polls = poll_limit();

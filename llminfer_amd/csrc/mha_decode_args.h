@@ -56,6 +56,7 @@ struct KernelArgs {
     // has zeros: num_splits at every length); dyn_magic: 2^32 / count, rounded up, for the three counts in that order.
     int32_t dyn_single, dyn_quarter, dyn_half;
     uint32_t dyn_magic[3];
+    int32_t dyn_full;  // more tiles than this: num_splits of them, whatever the rule's other lines say (long contexts take no other look at it)
     int32_t far_home;  // testing aid: 1 = every split but the merging one, 2 = every second one uses the other side's home
 };
 

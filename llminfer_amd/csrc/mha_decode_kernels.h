@@ -93,6 +93,78 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     const int kvh = blockIdx.x;
     const int split = blockIdx.y;
 
+    // Each wave streams its tiles through a private ring of NSTAGE LDS slots
+    // (8 KiB each: 4 KiB of K rows, 4 KiB of V rows) filled by LDS-DMA loads,
+    // so the bytes in flight cost no VGPRs. A load lands at offset 16*lane of its
+    // 1 KiB block, i.e. as four whole rows; the operand reads pick their 16 bytes
+    // out of those rows (K through a row-dependent swizzle, V directly), both free
+    // of bank conflicts. Out-of-range rows of a ragged last
+    // tile read the last valid row and are masked out of the softmax.
+    constexpr int kStageBytes = 8192;
+    constexpr int kRingBytes = NW * NSTAGE * kStageBytes;
+    // Epilogue: a wave's G x 128 partial outputs go to the start of its own (drained) ring,
+    // so no wave has to wait for another one's ring. Behind the rings: per-wave and merged
+    // (max, sum) pairs, then the combine area (weights [G][kMaxSplits], denominators [G],
+    // per-wave arrival flags [NW], one 16-byte partial sum per thread).
+    constexpr int kWaveRingBytes = NSTAGE * kStageBytes;
+    static_assert(G * kHeadDim * (int)sizeof(float) <= kWaveRingBytes, "a wave's partial outputs must fit its ring");
+    constexpr int kMergeTail = (2 * NW * G + 2 * G) * (int)sizeof(float);
+    constexpr int kCombineBase = kRingBytes + ((kMergeTail + 15) & ~15);
+    constexpr int kCombineBytes = (G * kMaxSplits + G + NW) * (int)sizeof(float) + NW * 64 * 16;
+    // Position on the device, eight wavefronts: norm weights and raw query rows are asked for while the position travels and the sines and cosines as
+    // soon as it is in, ahead of the splits' rule, so that all of a row's work but the rotation is done when they land; and a long
+    // context branches past the rule's other lines. What bounds these launches is the instructions in front of the first score. Everything behind the
+    // position, the rule in selects : so, 36 layers of 64 Q / 8 KV heads, us: 197.6 : 196.8 at 200 positions, 210.8 : 206.8 at 1000, 240.8 : 236.1 at 2500,
+    // 280.3 : 277.2 at 5000; 8 layers' blocks at 3001 310.8 : 309.1. Not with four wavefronts, one to a SIMD, where those with rows have tiles too:
+    // 32 Q / 8 KV heads 177.8 : 185.8 at 300, 187.5 : 195.9 at 1100, 16 Q heads 143.4 : 151.4; the branch alone is as bad there.
+    constexpr bool kEarlyRows = APPEND && DYN && NW > 4;
+    // 1 KiB LDS-DMA slots for the small operands, rows of 256 bytes four to a slot. Plain variant: every wave fetches all
+    // query rows of the group for itself. Append variant: the query rows, and in the
+    // workgroup of the last split the new K and V rows behind them, are dealt to the waves two at a time, 32 lanes a row, the last wave
+    // first (it has the fewest tiles); a wave fetches its own, raw, and leaves them normalised and rotated (V: as it is) behind the
+    // slots, where all waves read them after a barrier. In front of the slots one that the workgroup shares, q_norm | k_norm | sin row | cos row
+    // (every wave that works on rows fills it with the same bytes and waits only for its own loads); kEarlyRows: sin row | cos row, and a wave's
+    // own slots begin with q_norm | k_norm. The slots
+    // lie over the combine area, which nobody touches before the barrier of the epilogue, so they
+    // cost no LDS: with more than 80 KiB per workgroup the compiler assumes one wave per SIMD, puts
+    // the MFMA accumulators into AGPRs and copies all 32 of them to VGPRs and back around the
+    // rescaling of every tile.
+    constexpr int kRowPasses = (G + 2 + 2 * NW - 1) / (2 * NW);  // append variant: rows per half wavefront
+    constexpr int kRowSlots = APPEND ? ((kEarlyRows ? 2 : 0) + 2 * kRowPasses + 3) / 4 : (G * 16 + 63) / 64;
+    constexpr int kSharedSlots = APPEND ? 1 : 0;
+    constexpr int kReadyBytes = APPEND ? (G + 2) * 256 : 0;  // the finished rows: G query rows, the new K row, the new V row
+    constexpr int kStagingBase = (kCombineBase + 1023) & ~1023;
+    constexpr int kStagingBytes = (kSharedSlots + NW * kRowSlots) * 1024 + kReadyBytes;
+    constexpr int kSmemBytes =
+        kCombineBase + kCombineBytes > kStagingBase + kStagingBytes ? kCombineBase + kCombineBytes : kStagingBase + kStagingBytes;
+    __shared__ __attribute__((aligned(1024))) char smem[kSmemBytes];
+    char* shared_staging = smem + kStagingBase;                                       // append variant only
+    auto row_slots = [&]() { return smem + kStagingBase + (kSharedSlots + wave * kRowSlots) * 1024; };  // this wave's rows
+    char* ready_rows = smem + kStagingBase + (kSharedSlots + NW * kRowSlots) * 1024;  // append variant only
+    // Append variant: the rows of this workgroup -- the query heads, in the last split's the new K and V rows too -- are dealt to the waves in
+    // pairs, the last wave first: the first pair of this one (the next is NW on).
+    const int first_pair = NW - 1 - wave;
+    const bool has_queries = APPEND && 2 * first_pair < a.group;
+    // (early, wavefronts with nothing but the new K and V rows wait for the position all the same: they are the last split's business)
+    auto issue_rows = [&]() {
+        const int which = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < kRowSlots; ++i) {
+            if (i > 0 && 2 * (first_pair + NW * (2 * i - 1)) >= a.group + 2) continue;
+            // pass j lies 512 * (j + 1) bytes into the slots
+            const int row = 2 * (first_pair + NW * (2 * i - 1 + (which >> 1))) + (which & 1);
+            const uint64_t q_row = reinterpret_cast<uint64_t>(a.q) + (uint64_t)(uint32_t)((kvh * a.group + min(row, a.group - 1)) * 256);
+            const uint64_t new_row = reinterpret_cast<uint64_t>(row == a.group ? a.k_new : a.v_new) + (uint64_t)(uint32_t)(kvh * 256);
+            uint64_t src = row >= a.group ? new_row : q_row;  // (rows behind the last one repeat a row that is there and are not used)
+            if (i == 0) src = which < 2 ? reinterpret_cast<uint64_t>(a.norm_w) + (uint64_t)which * 256u : src;
+            dma16_gather(reinterpret_cast<const void*>(src + (uint64_t)n16 * 16u), (uint32_t)(uintptr_t)row_slots() + i * 1024);
+        }
+    };
+    auto issue_sincos = [&](int seq_len) {
+        const uint64_t row = reinterpret_cast<uint64_t>((lane & 16) ? a.cos_cache : a.sin_cache) + (uint64_t)(uint32_t)(seq_len - 1) * 256u;
+        dma16_gather(reinterpret_cast<const void*>(row + (uint64_t)n16 * 16u), (uint32_t)(uintptr_t)shared_staging);
+    };
+
     // A KV head's 16-position tiles are dealt to the splits in contiguous runs whose lengths
     // differ by at most one tile (the first tiles % S splits get the longer run), so every split
     // has work whenever there are at least S tiles and the last split -- the one that merges,
@@ -117,33 +189,47 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         // the position known to the host).
         asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.row_stride), "s"(a.head_stride), "s"(a.group), "s"(a.num_splits), "s"(a.seq_len),
                      "s"(a.dyn_single), "s"(a.dyn_half), "s"(a.dyn_quarter), "s"(a.dyn_magic[0]), "s"(a.dyn_magic[1]), "s"(a.dyn_magic[2]));
+        if constexpr (kEarlyRows) asm volatile("" ::"s"(a.dyn_full));
         if constexpr (APPEND) asm volatile("" ::"s"(a.norm_w), "s"(a.sin_cache), "s"(a.cos_cache), "s"(a.k_new), "s"(a.v_new), "s"(a.eps));
         // (constant address space: a scalar load, where the compiler, not knowing that nothing in the launch writes the position, takes a
         // vector one and its longer way: 36 layers 209.8 -> 205.5 us at 1100 positions, 194.5 -> 192.9 at 300, 64 layers of 64 Q heads at 5000
-        // 532.0 -> 530.5. The query's request and the heads' addresses ahead of its arrival: level.)
+        // 532.0 -> 530.5. The heads' addresses ahead of its arrival: level.)
         const auto pos_dev = reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(a.pos_dev));
-        seq_len = max(0, min(*pos_dev, a.seq_len - 1)) + 1;
+        const int32_t pos = *pos_dev;
+        if (kEarlyRows && has_queries) issue_rows();
+        seq_len = max(0, min(pos, a.seq_len - 1)) + 1;
+        if (kEarlyRows && has_queries) issue_sincos(seq_len);
         const int tiles = (seq_len - (APPEND ? 1 : 0) + kTile - 1) / kTile;
-        const bool few = tiles < a.dyn_half, medium = tiles <= 4 * a.dyn_half;
-        n_active = few ? a.dyn_quarter : medium ? a.dyn_half : a.num_splits;
-        const uint32_t magic = few ? a.dyn_magic[0] : medium ? a.dyn_magic[1] : a.dyn_magic[2];
-        run = (int)(((uint64_t)(uint32_t)tiles * magic) >> 32);
-        longer = tiles - run * n_active;
-        if (longer < 0) {  // (the rounded-up reciprocal is one too high at most, and only beyond 2^24 tiles)
-            --run;
-            longer += n_active;
+        // (the rounded-up reciprocal is one too high at most, and only beyond 2^24 tiles)
+        auto deal = [&](int count, uint32_t magic) {
+            n_active = count;
+            run = (int)(((uint64_t)(uint32_t)tiles * magic) >> 32);
+            longer = tiles - run * count;
+            if (longer < 0) {
+                --run;
+                longer += count;
+            }
+        };
+        if (kEarlyRows && tiles > a.dyn_full) {
+            deal(a.num_splits, a.dyn_magic[2]);
+        } else {
+            const bool few = tiles < a.dyn_half, medium = tiles <= 4 * a.dyn_half;
+            deal(few ? a.dyn_quarter : medium ? a.dyn_half : a.num_splits, few ? a.dyn_magic[0] : medium ? a.dyn_magic[1] : a.dyn_magic[2]);
+            if (tiles < n_active) {  // a tile each
+                n_active = tiles;
+                run = 1;
+                longer = 0;
+            }
+            if (tiles <= a.dyn_single || n_active <= 1) {
+                n_active = 1;
+                run = tiles;
+                longer = 0;
+            }
         }
-        if (tiles < n_active) {  // a tile each
-            n_active = tiles;
-            run = 1;
-            longer = 0;
+        if (split >= n_active) {
+            if constexpr (kEarlyRows) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (what is on its way to this workgroup's LDS lands first)
+            return;
         }
-        if (tiles <= a.dyn_single || n_active <= 1) {
-            n_active = 1;
-            run = tiles;
-            longer = 0;
-        }
-        if (split >= n_active) return;
     }
     const int cached_len = seq_len - (APPEND ? 1 : 0);  // positions streamed from the cache
     const int ntiles = run + (split < longer ? 1 : 0);
@@ -154,14 +240,16 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     u32x4 qb[4];                       // query group, MFMA B operand
     // Append variant: wave 0 of the last split (the one with the shortest run) takes the new token.
     const bool holds_new_row = APPEND && split == n_active - 1 && wave == 0;
-    // Append variant: the rows of this workgroup -- the query heads, in the last split's the new K and V rows too -- are dealt to the waves in
-    // pairs, the last wave first: the first pair of this one (the next is NW on). With two waves on a SIMD those that have rows go first
+    // Append variant: with two waves on a SIMD those that have rows go first
     // until the rows are done: their requests would else queue behind the tiles of the others (64 Q / 8 KV heads, a layer of a captured step at
     // 1000 positions, without : with 6.49 : 6.32 us).
     const int work_rows = a.group + (split == n_active - 1 ? 2 : 0);
-    const int first_pair = NW - 1 - wave;
     const bool has_rows = APPEND && 2 * first_pair < work_rows;
     if (NW > 4 && has_rows) __builtin_amdgcn_s_setprio(3);
+    if (kEarlyRows && has_rows && !has_queries) {
+        issue_rows();
+        issue_sincos(seq_len);
+    }
 
     // Wave-uniform 64-bit bases of this split; lanes add 32-bit byte offsets
     // (scalar-base + vector-offset addressing, no 64-bit multiplies per load).
@@ -200,43 +288,6 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         for (int j = 0; j < 8; ++j) ov[h][j] = 0.0f;
 #endif
 
-    // Each wave streams its tiles through a private ring of NSTAGE LDS slots
-    // (8 KiB each: 4 KiB of K rows, 4 KiB of V rows) filled by LDS-DMA loads,
-    // so the bytes in flight cost no VGPRs. A load lands at offset 16*lane of its
-    // 1 KiB block, i.e. as four whole rows; the operand reads pick their 16 bytes
-    // out of those rows (K through a row-dependent swizzle, V directly), both free
-    // of bank conflicts. Out-of-range rows of a ragged last
-    // tile read the last valid row and are masked out of the softmax.
-    constexpr int kStageBytes = 8192;
-    constexpr int kRingBytes = NW * NSTAGE * kStageBytes;
-    // Epilogue: a wave's G x 128 partial outputs go to the start of its own (drained) ring,
-    // so no wave has to wait for another one's ring. Behind the rings: per-wave and merged
-    // (max, sum) pairs, then the combine area (weights [G][kMaxSplits], denominators [G],
-    // per-wave arrival flags [NW], one 16-byte partial sum per thread).
-    constexpr int kWaveRingBytes = NSTAGE * kStageBytes;
-    static_assert(G * kHeadDim * (int)sizeof(float) <= kWaveRingBytes, "a wave's partial outputs must fit its ring");
-    constexpr int kMergeTail = (2 * NW * G + 2 * G) * (int)sizeof(float);
-    constexpr int kCombineBase = kRingBytes + ((kMergeTail + 15) & ~15);
-    constexpr int kCombineBytes = (G * kMaxSplits + G + NW) * (int)sizeof(float) + NW * 64 * 16;
-    // 1 KiB LDS-DMA slots for the small operands, one wavefront's rows of 256 bytes four to a slot. Plain variant: every wave fetches all
-    // query rows of the group for itself. Append variant, in front of them: a slot shared by the workgroup, q_norm | k_norm | sin row |
-    // cos row (every wave that works on rows fills it with the same bytes and waits only for its own loads). The query rows, and in the
-    // workgroup of the last split the new K and V rows behind them, are dealt to the waves two at a time, 32 lanes a row, the last wave
-    // first (it has the fewest tiles); a wave fetches its own, raw, and leaves them normalised and rotated (V: as it is) behind the
-    // slots, where all waves read them after a barrier. The slots
-    // lie over the combine area, which nobody touches before the barrier of the epilogue, so they
-    // cost no LDS: with more than 80 KiB per workgroup the compiler assumes one wave per SIMD, puts
-    // the MFMA accumulators into AGPRs and copies all 32 of them to VGPRs and back around the
-    // rescaling of every tile.
-    constexpr int kRowPasses = (G + 2 + 2 * NW - 1) / (2 * NW);  // append variant: rows per half wavefront
-    constexpr int kRowSlots = APPEND ? (2 * kRowPasses + 3) / 4 : (G * 16 + 63) / 64;
-    constexpr int kSharedSlots = APPEND ? 1 : 0;
-    constexpr int kReadyBytes = APPEND ? (G + 2) * 256 : 0;  // the finished rows: G query rows, the new K row, the new V row
-    constexpr int kStagingBase = (kCombineBase + 1023) & ~1023;
-    constexpr int kStagingBytes = (kSharedSlots + NW * kRowSlots) * 1024 + kReadyBytes;
-    constexpr int kSmemBytes =
-        kCombineBase + kCombineBytes > kStagingBase + kStagingBytes ? kCombineBase + kCombineBytes : kStagingBase + kStagingBytes;
-    __shared__ __attribute__((aligned(1024))) char smem[kSmemBytes];
     char* my_ring = smem + wave * (NSTAGE * kStageBytes);
     const uint32_t my_ring_lds = (uint32_t)(uintptr_t)my_ring;  // low 32 bits of a flat LDS address = LDS offset
 
@@ -358,10 +409,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         // the tiles, so that nothing near the end of the kernel has to wait for it.
         proj.gen_base = __hip_atomic_load(a.ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    char* shared_staging = smem + kStagingBase;                                       // append variant only
-    char* my_rows = smem + kStagingBase + (kSharedSlots + wave * kRowSlots) * 1024;  // this wave's rows
-    char* ready_rows = smem + kStagingBase + (kSharedSlots + NW * kRowSlots) * 1024;  // append variant only
-    {
+    char* my_rows = row_slots();
+    if constexpr (!kEarlyRows) {
         const uint32_t st = (uint32_t)(uintptr_t)shared_staging;
         const uint32_t st_rows = (uint32_t)(uintptr_t)my_rows;
         const int c16 = lane & 15, which = lane >> 4;
@@ -446,7 +495,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
         // (the accumulators are cleared here, in front of the wait, not behind it)
 #pragma unroll
         for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(o[j]));
-        wait_tiles_in_flight(first_tiles);
+        if constexpr (!APPEND) wait_tiles_in_flight(first_tiles);
         const int hq_local = min(n16, a.group - 1);
         if constexpr (APPEND) {
             const int half = lane >> 5, p32 = lane & 31;
@@ -456,6 +505,8 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
             // 5.47 at 1100, 7.38 : 7.21 at 4000; 64 Q heads 5.97 : 5.74 at 200, 6.52 : 6.32 at 1000, 8.25 : 8.06 at 5000.
             // (finished query rows: the 16-byte chunks swizzled by row & 7, so that the operand read below, one chunk of every row
             // at once, spreads over the LDS banks)
+            if constexpr (!kEarlyRows) wait_tiles_in_flight(first_tiles);
+            else if (has_rows) wait_loads_in_flight<1>(first_tiles);  // (all but the sin and cos rows and the tile)
 #pragma unroll
             for (int j = 0; j < kRowPasses; ++j) {
                 const int pair = first_pair + NW * j;
@@ -463,8 +514,11 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 const int row = 2 * pair + half;
                 const bool is_new = row >= a.group, is_v = row > a.group;
                 uint32_t xl, xh, lo, hi;
-                norm_rope_row32(my_rows + (2 * j + half) * 256, shared_staging + (is_new ? 256 : 0), shared_staging + 512, shared_staging + 768,
-                                p32, a.eps, xl, xh, lo, hi);
+                // (early: weights and rows are a wavefront's own, the tables the workgroup's)
+                const char* raw = my_rows + (kEarlyRows ? 512 : 0) + (2 * j + half) * 256;
+                const char* weights = (kEarlyRows ? my_rows : shared_staging) + (is_new ? 256 : 0);
+                const char* tables = shared_staging + (kEarlyRows ? 0 : 512);
+                norm_rope_row32<kEarlyRows>(raw, weights, tables, tables + 256, p32, a.eps, [&]() { wait_tiles_in_flight(first_tiles); }, xl, xh, lo, hi);
                 lo = is_v ? xl : lo;
                 hi = is_v ? xh : hi;
                 if (row < work_rows) {
@@ -480,6 +534,7 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
                 }
             }
             if (NW > 4 && has_rows) __builtin_amdgcn_s_setprio(0);
+            if constexpr (kEarlyRows) wait_tiles_in_flight(first_tiles);  // (whatever was asked for and is not used has landed too: its place is the combine area's)
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
             for (int s0 = 1; s0 < NSTAGE; ++s0)

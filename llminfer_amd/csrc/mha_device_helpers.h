@@ -199,6 +199,13 @@ __device__ __forceinline__ void wait_tiles_in_flight(int newer_tiles) {
     else asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
 }
 
+// The same with MORE single loads behind the oldest ones, tiles 0 or 1.
+template <int MORE>
+__device__ __forceinline__ void wait_loads_in_flight(int tiles) {
+    if (tiles <= 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MORE) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MORE + 8) : "memory");
+}
+
 struct TileRegs {
     u32x4 k[4];
     u32x4 v[4];
@@ -288,11 +295,14 @@ __device__ __forceinline__ float inverse_rms(float ss, float eps) {
     const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0);
     return __builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y);
 }
-__device__ __forceinline__ void rotate_pair(float a, float b, float wa, float wb, float r, float sn, float cs, float& lo, float& hi) {
-    const float av = a * wa * r, bv = b * wb * r;
+__device__ __forceinline__ float scaled(float x, float w, float r) { return x * w * r; }
+__device__ __forceinline__ void rotate_scaled(float av, float bv, float sn, float cs, float& lo, float& hi) {
     const float bs = bv * sn, bc = bv * cs;
     lo = __builtin_fmaf(av, cs, -bs);
     hi = __builtin_fmaf(av, sn, bc);
+}
+__device__ __forceinline__ void rotate_pair(float a, float b, float wa, float wb, float r, float sn, float cs, float& lo, float& hi) {
+    rotate_scaled(scaled(a, wa, r), scaled(b, wb, r), sn, cs, lo, hi);
 }
 
 // In place, by one wavefront: the 16 lanes of DPP row r take row `row` of `rows` (256 bytes each); lane p of them
@@ -335,13 +345,18 @@ __device__ __forceinline__ void norm_rope_rows_lds(char* rows, const char* w, co
 
 // A row on 32 lanes, half a wavefront, into registers: lane p of them takes the pairs 2p and 2p + 1, i.e. dword p of the row (lo) and
 // dword p + 32 (hi); xl, xh: the same two as they were. Half the instructions of the form above behind the root (a lane's share is half as
-// long); in front of it both lanes of a neighbouring two have the chain of their four pairs.
-__device__ __forceinline__ void norm_rope_row32(const char* row, const char* w, const char* sin16, const char* cos16, int p, float eps,
+// long); in front of it both lanes of a neighbouring two have the chain of their four pairs. `tables_in` waits for the sines and cosines, which
+// are not asked for before the position is known: everything but the rotation is done by then.
+template <bool LATE_TABLES, typename W>
+__device__ __forceinline__ void norm_rope_row32(const char* row, const char* w, const char* sin16, const char* cos16, int p, float eps, W&& tables_in,
                                                 uint32_t& xl, uint32_t& xh, uint32_t& lo, uint32_t& hi) {
     const u32x2 xl2 = *reinterpret_cast<const u32x2*>(row + (p >> 1) * 8), xh2 = *reinterpret_cast<const u32x2*>(row + 128 + (p >> 1) * 8);
     const uint32_t wl = *reinterpret_cast<const uint32_t*>(w + p * 4), wh = *reinterpret_cast<const uint32_t*>(w + 128 + p * 4);
-    const u32x2 sn = *reinterpret_cast<const u32x2*>(sin16 + p * 8), cs = *reinterpret_cast<const u32x2*>(cos16 + p * 8);
-    const uint32_t sn0 = sn[0], sn1 = sn[1], cs0 = cs[0], cs1 = cs[1];
+    u32x2 sn, cs;
+    if constexpr (!LATE_TABLES) {
+        sn = *reinterpret_cast<const u32x2*>(sin16 + p * 8);
+        cs = *reinterpret_cast<const u32x2*>(cos16 + p * 8);
+    }
     const uint32_t xl0 = xl2[0], xl1 = xl2[1], xh0 = xh2[0], xh1 = xh2[1];
     const float a[4] = {bf16_lo(xl0), bf16_hi(xl0), bf16_lo(xl1), bf16_hi(xl1)};
     const float b[4] = {bf16_lo(xh0), bf16_hi(xh0), bf16_lo(xh1), bf16_hi(xh1)};
@@ -358,9 +373,18 @@ __device__ __forceinline__ void norm_rope_row32(const char* row, const char* w, 
     const float r = inverse_rms(ss, eps);
     xl = (p & 1) ? xl1 : xl0;
     xh = (p & 1) ? xh1 : xh0;
+    float a0 = scaled(bf16_lo(xl), bf16_lo(wl), r), b0 = scaled(bf16_lo(xh), bf16_lo(wh), r);
+    float a1 = scaled(bf16_hi(xl), bf16_hi(wl), r), b1 = scaled(bf16_hi(xh), bf16_hi(wh), r);
+    if constexpr (LATE_TABLES) {
+        asm volatile("" : "+v"(a0), "+v"(b0), "+v"(a1), "+v"(b1));
+        tables_in();
+        sn = *reinterpret_cast<const u32x2*>(sin16 + p * 8);
+        cs = *reinterpret_cast<const u32x2*>(cos16 + p * 8);
+    }
+    const uint32_t sn0 = sn[0], sn1 = sn[1], cs0 = cs[0], cs1 = cs[1];
     float l0, l1, h0, h1;
-    rotate_pair(bf16_lo(xl), bf16_lo(xh), bf16_lo(wl), bf16_lo(wh), r, __builtin_bit_cast(float, sn0), __builtin_bit_cast(float, cs0), l0, h0);
-    rotate_pair(bf16_hi(xl), bf16_hi(xh), bf16_hi(wl), bf16_hi(wh), r, __builtin_bit_cast(float, sn1), __builtin_bit_cast(float, cs1), l1, h1);
+    rotate_scaled(a0, b0, __builtin_bit_cast(float, sn0), __builtin_bit_cast(float, cs0), l0, h0);
+    rotate_scaled(a1, b1, __builtin_bit_cast(float, sn1), __builtin_bit_cast(float, cs1), l1, h1);
     lo = pack_bf16(l0, l1);
     hi = pack_bf16(h0, h1);
 }
