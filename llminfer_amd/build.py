@@ -46,6 +46,87 @@ def kernels_using_scratch(compiler_output):
     return bad
 
 
+_REGISTERS = re.compile(r"\b(?:s(\d+)\b|s\[(\d+):(\d+)\]|(vcc_lo|vcc_hi|vcc|m0)\b)")
+_VMEM = ("global_", "buffer_", "flat_", "scratch_", "tbuffer_")
+_WAIT_STATES = 5  # between a vector instruction that writes a scalar register and a memory instruction that reads it
+
+
+def _scalar_registers(operands):
+    regs = set()
+    for one, lo, hi, name in _REGISTERS.findall(operands):
+        if name:
+            regs |= {"vcc_lo", "vcc_hi"} if name == "vcc" else {name}
+        else:
+            regs |= set(range(int(lo or one), int(hi or one) + 1))
+    return regs
+
+
+def scalar_reads_too_early(disassembly):
+    """Memory instructions that read a scalar register fewer than five wait states behind the vector instruction that
+    wrote it, as "kernel: writer -> reader", from llvm-objdump's output. The compiler keeps that distance for its own
+    instructions and does not look into asm statements, and the LDS-DMA loads are asm statements: with their base in
+    vector registers it puts the v_readfirstlane pair right in front of the load, which then goes to a wrong address."""
+    found = set()
+    for kernel, body in re.findall(r"^[0-9a-f]+ <(\S+)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)", disassembly, re.M | re.S):
+        code, index, jumps = [], {}, []
+        for line in body.splitlines():
+            text, _, where = line.partition("//")
+            if not where:
+                continue
+            name, _, operands = text.strip().partition(" ")
+            index[int(where.partition(":")[0], 16)] = len(code)
+            if "branch" in name:
+                jumps.append((len(code), int(where.rpartition("+0x")[2].rstrip(">") or "0", 16)))
+            code.append((name, operands.strip()))
+        ends = ("s_branch", "s_endpgm", "s_setpc_b64")
+        before = [[i - 1] if i and code[i - 1][0] not in ends else [] for i in range(len(code))]
+        first = min(index, default=0)
+        for i, target in jumps:
+            if first + target in index:
+                before[index[first + target]].append(i)
+
+        def look(i, watched, states, reader):
+            if states >= _WAIT_STATES or not watched:
+                return
+            for j in before[i]:
+                name, operands = code[j]
+                fields = operands.split(", ")
+                if name.startswith("v_"):
+                    # (the carry of an addition and the scale of a division come second)
+                    written = _scalar_registers(fields[0]) | (_scalar_registers(fields[1]) if "_co_" in name or "div_scale" in name else set())
+                    if written & watched:
+                        found.add("%s: %s %s -> %s %s" % ((kernel, name, operands) + reader))
+                        continue
+                    left = watched
+                elif name.startswith("s_") and not re.match(r"s_(cmp|bitcmp|cbranch|branch|waitcnt|nop|barrier|sleep|setprio)", name):
+                    left = watched - _scalar_registers(fields[0])  # (rewritten by the scalar unit: no distance to keep)
+                else:
+                    left = watched
+                look(j, left, states + (int(operands, 0) + 1 if name == "s_nop" else 1), reader)
+
+        for i, (name, operands) in enumerate(code):
+            if name.startswith(_VMEM):
+                look(i, _scalar_registers(operands) | ({"m0"} if "_lds_" in name or operands.endswith(" lds") else set()), 0, (name, operands))
+    return sorted(found)
+
+
+def _early_scalar_reads(obj):
+    """... in the gfx950 code of an object file that was just built, disassembled."""
+    import tempfile
+
+    def tool(name, *args):
+        return _run([_run([os.environ.get("HIPCC", "hipcc"), "--print-prog-name=" + name]).strip()] + list(args))
+
+    with tempfile.TemporaryDirectory() as tmp:
+        bundle, code = os.path.join(tmp, "bundle"), os.path.join(tmp, "code")
+        tool("llvm-objcopy", "--dump-section", ".hip_fatbin=" + bundle, obj, os.path.join(tmp, "rest"))
+        tool("clang-offload-bundler", "--type=o", "--unbundle", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", "--input=" + bundle, "--output=" + code)
+        listing = tool("llvm-objdump", "-d", code)
+    if "s_endpgm" not in listing:
+        raise RuntimeError("no gfx950 code found in " + obj)
+    return scalar_reads_too_early(listing)
+
+
 def _compile_objects(sources, defines, tag):
     """Each source to an object file (in parallel: the kernels' file takes minutes, the others seconds), the
     compiler's remarks of all of them joined."""
@@ -59,7 +140,12 @@ def _compile_objects(sources, defines, tag):
         obj = os.path.join(obj_dir, os.path.basename(src) + ".o")
         cmd = [hipcc] + flags + ["-c", "-Rpass-analysis=kernel-resource-usage"] + ["-D" + d for d in defines]
         cmd += ["-I" + os.path.join(ROOT, "include"), "-I" + CSRC, src, "-o", obj]
-        return obj, _run(cmd)
+        remarks = _run(cmd)
+        early = _early_scalar_reads(obj) if src.endswith(".hip") else []
+        if early:
+            raise RuntimeError("scalar registers read too early by a memory instruction (pin them, see scalar_bases in mha_device_helpers.h):\n"
+                               + "\n".join(early))
+        return obj, remarks
 
     with ThreadPoolExecutor(max_workers=min(8, len(sources))) as pool:
         results = list(pool.map(one, sources))

@@ -149,7 +149,8 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 // The bases of the dma16 loads that follow, in scalar registers and there for long enough: a scalar register that a vector instruction has
 // written (v_readfirstlane, which is how the compiler brings a value it has computed in vector registers, a clamp by v_med3 is enough, over to
 // dma16's operand) may be read by a memory instruction five wait states later at the earliest, and the compiler, which counts them
-// elsewhere, does not look into an asm statement. For callers whose bases are computed as they go.
+// elsewhere, does not look into an asm statement. For callers whose bases are computed as they go; where they are scalar throughout it is not needed,
+// and the build's look at the disassembly says so.
 __device__ __forceinline__ void scalar_bases(const char*& a, const char*& b) {
     asm volatile("s_nop 4" : "+s"(a), "+s"(b));
 }
@@ -158,10 +159,10 @@ __device__ __forceinline__ void scalar_bases(const char*& a, const char*& b) {
 // lane L's bytes land at lds_off + 16*L. `base` and `lds_off` are wave-uniform,
 // `voff` is the lane's byte offset from base. Counted by vmcnt like any load.
 __device__ __forceinline__ void dma16(const char* base, uint32_t voff, uint32_t lds_off) {
-    // (`base` in scalar registers already: see scalar_bases.)
     // The instruction takes its base and the LDS offset (through M0) from scalar
-    // registers; readfirstlane guarantees that whatever the surrounding code
-    // made of these wave-uniform values (it is free when they already are scalar).
+    // registers. Both are wave-uniform and meant to be scalar already, where readfirstlane is free: a base that the compiler
+    // keeps in vector registers it would fill right in front of the load (see scalar_bases). The build
+    // disassembles what it has made and refuses a pair that is too close.
     // M0 is an operand of the asm statement (constraint {m0}): the compiler writes it and
     // knows that it is live; the s_nop covers the wait state between that write and the load.
     const uint64_t b = reinterpret_cast<uint64_t>(base);

@@ -351,6 +351,37 @@ def test_build_rejects_kernels_with_a_private_segment():
     assert build.kernels_using_scratch("") == []
 
 
+_LOAD = "global_load_lds_dwordx4 v3, s[8:9] nt"
+
+
+@pytest.mark.parametrize("code,writer", [
+    (["v_readfirstlane_b32 s8, v1", "v_readfirstlane_b32 s9, v2", "s_nop 0", _LOAD], "v_readfirstlane_b32 s9, v2"),  # (the nearer of the two)
+    (["v_readfirstlane_b32 s9, v2", "s_nop 3", _LOAD], "v_readfirstlane_b32 s9, v2"),           # four wait states
+    (["v_readfirstlane_b32 s9, v2", "s_nop 4", _LOAD], None),                                   # five
+    (["v_readfirstlane_b32 s9, v2"] + ["v_mov_b32_e32 v0, v1"] * 5 + [_LOAD], None),
+    (["v_readfirstlane_b32 s9, v2", "s_mov_b32 s9, s20", "s_nop 0", _LOAD], None),              # rewritten by the scalar unit
+    (["v_readfirstlane_b32 s10, v2", "s_nop 0", _LOAD], None),                                  # another register
+    (["v_cmp_eq_u32_e64 s[8:9], 2, v1", "s_nop 0", _LOAD], "v_cmp_eq_u32_e64 s[8:9], 2, v1"),
+    (["v_add_co_u32_e64 v0, s[8:9], v1, v2", _LOAD], "v_add_co_u32_e64 v0, s[8:9], v1, v2"),
+    (["v_readlane_b32 s8, v1, 0", "global_load_dwordx4 v[0:3], v4, s[8:9]"], "v_readlane_b32 s8, v1, 0"),
+    (["v_readfirstlane_b32 m0, v1", "s_nop 0", "global_load_lds_dwordx4 v[0:1], off"], "v_readfirstlane_b32 m0, v1"),
+    # by way of a jump: instruction 0 goes on at the load, instruction 2 does not fall through to it
+    (["v_readfirstlane_b32 s8, v1", "s_cbranch_scc1 JUMP 5", "s_nop 7", "s_endpgm", "s_nop 7", _LOAD], "v_readfirstlane_b32 s8, v1"),
+    (["s_branch JUMP 3", "v_readfirstlane_b32 s8, v1", "s_endpgm", _LOAD], None),
+])
+def test_build_finds_scalar_registers_read_too_early(code, writer):
+    """The build reads the disassembly and refuses a memory instruction closer than five wait states behind the vector
+    instruction that wrote its scalar base: the compiler does not look into the asm statements the LDS-DMA loads are."""
+    from llminfer_amd import build
+    lines = ["0000000000001000 <kern>:"]
+    for i, text in enumerate(code):
+        name, jump, target = text.partition(" JUMP ")
+        where = " <kern+0x%x>" % (8 * int(target)) if jump else ""
+        lines.append("\t%s    // %012X: BF800000%s" % (name + (" 1" if jump else ""), 0x1000 + 8 * i, where))
+    load = [c for c in code if c.startswith("global_load")][0]
+    assert build.scalar_reads_too_early("\n".join(lines) + "\n") == (["kern: %s -> %s" % (writer, load)] if writer else [])
+
+
 @pytest.mark.parametrize("head_dim", [64, 128, 256, 4096, 2**31 - 1])
 def test_workspace_bytes_for_any_head_dim(head_dim):
     """The size query never divides by a block count of zero (a row wider than the 8 KiB blocks of the layout by side
