@@ -78,7 +78,7 @@ constexpr int kWavesPerEu = (G >= 16 && NW != 2) ? 1 : LLMI_MIN_WAVES_PER_EU;
 #endif
 constexpr int kWideMergeMin = LLMI_WIDE_MERGE_MIN;
 
-template <int G, int NW, int NSTAGE, bool APPEND, bool DYN, bool STAGGER, bool OPROJ, bool BYSIDE>
+template <int G, int NW, int NSTAGE, bool APPEND, bool DYN, bool STAGGER, bool OPROJ, bool BYSIDE, bool EARLY = false>
 __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState& proj) {
     constexpr bool kSpreadMerge = LLMI_SPREAD_MERGE && !OPROJ;
     const int lane = threadIdx.x & 63;
@@ -111,13 +111,17 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     constexpr int kMergeTail = (2 * NW * G + 2 * G) * (int)sizeof(float);
     constexpr int kCombineBase = kRingBytes + ((kMergeTail + 15) & ~15);
     constexpr int kCombineBytes = (G * kMaxSplits + G + NW) * (int)sizeof(float) + NW * 64 * 16;
-    // Position on the device, eight wavefronts: norm weights and raw query rows are asked for while the position travels and the sines and cosines as
-    // soon as it is in, ahead of the splits' rule, so that all of a row's work but the rotation is done when they land; and a long
-    // context branches past the rule's other lines. What bounds these launches is the instructions in front of the first score. Everything behind the
-    // position, the rule in selects : so, 36 layers of 64 Q / 8 KV heads, us: 197.6 : 196.8 at 200 positions, 210.8 : 206.8 at 1000, 240.8 : 236.1 at 2500,
-    // 280.3 : 277.2 at 5000; 8 layers' blocks at 3001 310.8 : 309.1. Not with four wavefronts, one to a SIMD, where those with rows have tiles too:
-    // 32 Q / 8 KV heads 177.8 : 185.8 at 300, 187.5 : 195.9 at 1100, 16 Q heads 143.4 : 151.4; the branch alone is as bad there.
-    constexpr bool kEarlyRows = APPEND && DYN && NW > 4;
+    // Position on the device, groups of exactly eight on eight wavefronts: norm weights and raw query rows are asked for while the position
+    // travels and the sines and cosines as soon as it is in, ahead of the splits' rule, so that all of a row's work but the rotation is done
+    // when they land; and a long context branches past the rule's other lines. Everything behind the position, the rule in selects : so, 36 captured
+    // layers of 64 Q / 8 KV heads, us: 195.1 : 195.9 at 200 positions, 203.8 : 206.4 at 300, 207.8 : 205.0 at 600, 211.4 : 208.0 at 1000, 229.6 :
+    // 221.9 at 1700, 240.2 : 234.3 at 2500, 252.6 : 249.9 at 3500, 277.7 : 275.2 at 5000, a window of 160 positions 155.5 : 153.3. It is the three
+    // together: at 1000, 2500 and 5000 positions without the branch 210.8, 242.2, 277.9, without the rows ahead 214.2, 232.3, 280.0, one wait for
+    // rows and tables 213.8, 240.7, 275.4, the branch alone 212.3, 231.3, 290.8. Nobody else gains: 40 Q heads, not so : so, 204.0 : 207.7 at 300, 209.2 : 215.3
+    // at 1000, 239.8 : 235.5 at 2500, 275.7 : 283.8 at 5000, 48 Q heads 211.0 : 217.0 at 1000; eight wavefronts for smaller groups, windows of 160
+    // positions, 32 Q heads 153.0 : 155.5, 8 Q heads 144.8 : 146.8; four wavefronts, 32 Q heads 177.8 : 185.8 at 300, 187.5 : 195.9 at 1100.
+    constexpr bool kEarlyRows = EARLY;
+    static_assert(!EARLY || (G == 8 && NW == 8 && APPEND && DYN), "");
     // 1 KiB LDS-DMA slots for the small operands, rows of 256 bytes four to a slot. Plain variant: every wave fetches all
     // query rows of the group for itself. Append variant: the query rows, and in the
     // workgroup of the last split the new K and V rows behind them, are dealt to the waves two at a time, 32 lanes a row, the last wave
@@ -146,19 +150,17 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     const int first_pair = NW - 1 - wave;
     const bool has_queries = APPEND && 2 * first_pair < a.group;
     // (early, wavefronts with nothing but the new K and V rows wait for the position all the same: they are the last split's business)
+    // (one pass and one slot: the weights in lanes 0 to 31, where `row` lies in front of the first one and is not used, the pair behind them)
+    static_assert(!kEarlyRows || (kRowPasses == 1 && kRowSlots == 1), "");
     auto issue_rows = [&]() {
         const int which = lane >> 4;
-#pragma unroll
-        for (int i = 0; i < kRowSlots; ++i) {
-            if (i > 0 && 2 * (first_pair + NW * (2 * i - 1)) >= a.group + 2) continue;
-            // pass j lies 512 * (j + 1) bytes into the slots
-            const int row = 2 * (first_pair + NW * (2 * i - 1 + (which >> 1))) + (which & 1);
-            const uint64_t q_row = reinterpret_cast<uint64_t>(a.q) + (uint64_t)(uint32_t)((kvh * a.group + min(row, a.group - 1)) * 256);
-            const uint64_t new_row = reinterpret_cast<uint64_t>(row == a.group ? a.k_new : a.v_new) + (uint64_t)(uint32_t)(kvh * 256);
-            uint64_t src = row >= a.group ? new_row : q_row;  // (rows behind the last one repeat a row that is there and are not used)
-            if (i == 0) src = which < 2 ? reinterpret_cast<uint64_t>(a.norm_w) + (uint64_t)which * 256u : src;
-            dma16_gather(reinterpret_cast<const void*>(src + (uint64_t)n16 * 16u), (uint32_t)(uintptr_t)row_slots() + i * 1024);
-        }
+        const int row = 2 * (first_pair + NW * ((which >> 1) - 1)) + (which & 1);
+        const uint64_t q_row = reinterpret_cast<uint64_t>(a.q) + (uint64_t)(uint32_t)((kvh * a.group + min(row, a.group - 1)) * 256);
+        const uint64_t new_row = reinterpret_cast<uint64_t>(row == a.group ? a.k_new : a.v_new) + (uint64_t)(uint32_t)(kvh * 256);
+        const uint64_t weights = reinterpret_cast<uint64_t>(a.norm_w) + (uint64_t)which * 256u;
+        uint64_t src = row >= a.group ? new_row : q_row;  // (rows behind the last one repeat a row that is there and are not used)
+        src = which < 2 ? weights : src;                  // (selects: with the weights' address in its arm this becomes a branch)
+        dma16_gather(reinterpret_cast<const void*>(src + (uint64_t)n16 * 16u), (uint32_t)(uintptr_t)row_slots());
     };
     auto issue_sincos = [&](int seq_len) {
         const uint64_t row = reinterpret_cast<uint64_t>((lane & 16) ? a.cos_cache : a.sin_cache) + (uint64_t)(uint32_t)(seq_len - 1) * 256u;
@@ -1140,10 +1142,10 @@ __device__ __forceinline__ void mha_decode_body(const KernelArgs& a, OprojState&
     }
 }
 
-template <int G, int NW, int NSTAGE, bool APPEND, bool DYN, bool STAGGER = false, bool BYSIDE = false>
+template <int G, int NW, int NSTAGE, bool APPEND, bool DYN, bool STAGGER = false, bool BYSIDE = false, bool EARLY = false>
 __global__ __launch_bounds__(NW * 64, (kWavesPerEu<G, NW>)) void mha_decode_kernel(KernelArgs a) {
     OprojState unused;
-    mha_decode_body<G, NW, NSTAGE, APPEND, DYN, STAGGER, false, BYSIDE>(a, unused);
+    mha_decode_body<G, NW, NSTAGE, APPEND, DYN, STAGGER, false, BYSIDE, EARLY>(a, unused);
 }
 
 // The attention launch with the layer's output projection and residual add behind it, in the same launch
@@ -1255,6 +1257,16 @@ void launch_decode(const KernelArgs& ka, int n_kv, bool append, hipStream_t stre
     constexpr int kStages = (NW * LLMI_STAGES * 8192 <= LLMI_RING_LIMIT) ? LLMI_STAGES : LLMI_RING_LIMIT / (NW * 8192);
     dim3 grid(n_kv, ka.num_splits);
     const bool dyn = ka.pos_dev != nullptr;  // position read at run time: its own instantiation, the static one pays nothing
+    if constexpr (G == 8 && NW == 8) {
+        if (append && dyn && ka.group == 8) {  // (kEarlyRows: only these)
+            const bool stagger = ka.stagger && ka.num_splits > 1;
+            if (ka.by_side && stagger) hipLaunchKernelGGL((mha_decode_kernel<8, 8, kStages, true, true, true, true, true>), grid, dim3(512), 0, stream, ka);
+            else if (ka.by_side) hipLaunchKernelGGL((mha_decode_kernel<8, 8, kStages, true, true, false, true, true>), grid, dim3(512), 0, stream, ka);
+            else if (stagger) hipLaunchKernelGGL((mha_decode_kernel<8, 8, kStages, true, true, true, false, true>), grid, dim3(512), 0, stream, ka);
+            else hipLaunchKernelGGL((mha_decode_kernel<8, 8, kStages, true, true, false, false, true>), grid, dim3(512), 0, stream, ka);
+            return;
+        }
+    }
     if constexpr (kHasBySide<G, NW>) {
         if (ka.by_side) {
             if (append) {

@@ -14,6 +14,8 @@ from helpers import assert_parity, assert_tap_parity, from_dev_bf16, to_dev
 
 pytestmark = pytest.mark.gpu
 
+HEAD, POS = B.KV_LAYOUT_HEAD_MAJOR, B.KV_LAYOUT_POS_MAJOR
+
 
 def _oracle_at(oracle, case, pos):
     return oracle.mha_cpu(case["q"], case["k"], case["v"], case["layer_id"], pos, case["kv_dim"], case["kv_mul"],
@@ -205,3 +207,68 @@ def test_plan_rejects_device_position_with_separate_combine(dev):
     a = ops.make_mha_args(t, kv, kv, t, ws, layer_id=0, pos=511, kv_dim=1024, kv_mul=4, head_num=32, head_dim=128,
                           max_seq_len=512, force_path=B.PATH_SPLIT, num_splits=4, pos_device=pos_t)
     assert ops.mha_decode_raw(a) == B.STATUS["INVALID_ARG"]
+
+
+@pytest.mark.parametrize("n_q,n_kv,msl,layout,kw", [
+    (64, 8, 4096, HEAD, {}), (64, 8, 4096, POS, dict(side=True)),      # groups of eight: rows ahead of the position
+    (56, 8, 4096, HEAD, {}), (40, 8, 4096, HEAD, dict(side=True)),     # of seven and five: not
+    (32, 8, 4096, HEAD, dict(waves_per_group=8)), (8, 8, 2048, POS, dict(waves_per_group=8)),
+    (64, 8, 230, HEAD, {}), (24, 8, 170, HEAD, {}),                    # a window of one pass on eight wavefronts
+    (64, 8, 4096, HEAD, dict(num_splits=12, force_path=B.PATH_SPLIT_FUSED)),  # no rule: twelve as far as there are tiles
+])
+def test_append_walks_over_the_split_rule(dev, n_q, n_kv, msl, layout, kw):
+    """One captured append launch planned for the whole window; the position walks over both sides of every length at which the rule changes
+    the split count. Outputs, the tap and the caches have the bits of a launch with the position on the host and as many splits."""
+    kw = dict(kw)
+    rng = np.random.RandomState(n_q + msl)
+    bits = lambda *shape: to_dev(synth.f32_to_bf16_bits(rng.standard_normal(shape).astype(np.float32)), dev)
+    kv_dim = n_kv * 128
+    k, v, w = bits(1, msl, kv_dim), bits(1, msl, kv_dim), to_dev(synth.f32_to_bf16_bits(1 + 0.1 * rng.standard_normal(256).astype(np.float32)), dev)
+    sin, cos = ops.sincos_table(128, msl, dev)
+    q, kn, vn = (torch.zeros(n, dtype=torch.int16, device=dev) for n in (n_q * 128, kv_dim, kv_dim))
+    ws = torch.full((ops.workspace_bytes(n_q, 128, msl) // 4,), float("nan"), dtype=torch.float32, device=dev)
+    side = ops.workspace_side(ws) or 0x55555555 if kw.pop("side", False) else 0
+    pos = torch.zeros(1, dtype=torch.int32, device=dev)
+    common = dict(layer_id=0, kv_dim=kv_dim, kv_mul=n_q // n_kv, head_num=n_q, head_dim=128, max_seq_len=msl, kv_layout=layout, workspace_side=side)
+    a, b = ({"k": k.clone(), "v": v.clone(), "out": torch.zeros(n_q * 128, dtype=torch.int16, device=dev),
+             "tap": torch.zeros(n_q * 128, dtype=torch.float32, device=dev)} for _ in "ab")
+
+    def append(s, **more):
+        ops.mha_decode_append(q, kn, vn, w, sin, cos, s["k"], s["v"], s["out"], ws, output_f32=s["tap"], **dict(common, **more))
+
+    args = ops.make_mha_args(q, a["k"], a["v"], a["out"], ws, pos=msl - 1, pos_device=pos, **common, **kw)
+    plan, rule = ops.mha_plan(args), (ctypes.c_int32 * 3)()
+    B.check(B.lib().llmi_hip_device_split_rule(ctypes.byref(args), 1, rule), "rule")
+    single, quarter, half = rule
+    assert plan.waves_per_group == 8
+
+    def splits(n):
+        tiles = (n - 1 + 15) // 16
+        count = quarter if tiles < half else half if tiles <= 4 * half else plan.num_splits
+        count = min(count, tiles)
+        return 1 if tiles <= single or plan.num_splits == 1 else max(count, 1)
+
+    stream, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(g, stream=stream):
+            append(a, pos=msl - 1, pos_device=pos, stream=stream, **kw)
+    full = max(4 * half, single, plan.num_splits)  # (more tiles than this: nothing but all splits)
+    edges = [t * 16 + 1 for t in (single, quarter, half, 4 * half, plan.num_splits, full)]
+    lengths = sorted({1, 2, 17, 18, 100, 1000, msl - 1, msl} | {e + d for e in edges for d in (-16, -1, 0, 1, 16)})
+    seen = set()
+    for n in [x for x in lengths if 0 < x <= msl]:
+        for t in (q, kn, vn):
+            t.copy_(bits(t.numel()))
+        pos.fill_(n - 1)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        count = splits(n)
+        seen.add(count)
+        forced = dict(force_path=B.PATH_SPLIT_FUSED, num_splits=count) if count > 1 else dict(force_path=B.PATH_SINGLE_PASS)
+        append(b, pos=n - 1, waves_per_group=8, **forced)
+        torch.cuda.synchronize()
+        what = "%d positions, %d splits" % (n, count)
+        assert torch.equal(a["out"], b["out"]) and torch.equal(a["tap"], b["tap"]), what
+        assert torch.equal(a["k"], b["k"]) and torch.equal(a["v"], b["v"]), what
+    assert plan.num_splits in seen and (msl < 4096 or kw or {1, half, plan.num_splits} <= seen)
