@@ -51,6 +51,12 @@ int32_t llmi_hip_spread_min_splits(int32_t kv_mul, int32_t waves, int32_t head_n
  * one split takes them all, splits below rule[2] tiles (a tile each if there are fewer), splits up to 4 * rule[2] tiles. */
 int32_t llmi_hip_device_split_rule(const llmi_mha_args* args, int32_t append, int32_t rule[3]);
 
+/* The form llmi_hip_mha_decode_append_stack takes for layers that are independent of each other, on a device of `compute_units`
+ * (0: the present one; otherwise none is needed): form[0] = workgroups of the launch that takes them a KV head at a time (0: another
+ * form is taken, and the rest is 0), [1] parts of a cut head (1: none is cut), [2] cut heads, [3] wavefronts that stream, [4] splits of a
+ * head, [5] splits a workgroup takes side by side. */
+int32_t llmi_hip_heads_form(const llmi_mha_stack_args* args, int32_t compute_units, int32_t form[6]);
+
 #ifdef __cplusplus
 }
 #endif

@@ -150,6 +150,7 @@ SYMBOLS = {
     "llmi_hip_stagger_mask": (c_i32, [c_i32, ctypes.c_int64, c_i32]),
     "llmi_hip_spread_min_splits": (c_i32, [c_i32, c_i32, c_i32]),
     "llmi_hip_device_split_rule": (c_i32, [ctypes.POINTER(MhaArgs), c_i32, ctypes.POINTER(c_i32)]),
+    "llmi_hip_heads_form": (c_i32, [ctypes.POINTER(MhaStackArgs), c_i32, ctypes.POINTER(c_i32)]),
     "llmi_hip_workspace_side_stats": (None, [ctypes.POINTER(ctypes.c_uint64)]),
 }
 

@@ -580,12 +580,11 @@ static bool layers_are_independent(const llmi_mha_stack_args& st) {
 }
 
 // Whether the resident launch that walks the layers (mha_stack.hip) takes this shape.
-static bool resident_form(const llmi_mha_args& m, const llmi_mha_plan& plan) {
+static bool resident_form(const llmi_mha_args& m, const llmi_mha_plan& plan, int cus) {
     if (plan.path != LLMI_PATH_SPLIT_FUSED || plan.num_splits < 2 || plan.num_splits > 64) return false;
     if (plan.group_pad > 4 || plan.waves_per_group != 4 || m.head_num > 64) return false;  // (one lane of the polling wavefront per head)
     if (m.workspace_bytes < plan.workspace_needed + stack_workspace_extra(m.head_num)) return false;
     // every workgroup must be resident at once: workgroups wait for each other
-    const int cus = compute_units();
     if (cus <= 0 || (int64_t)(m.kv_dim / m.head_dim) * plan.num_splits > cus) return false;
     // Lengths at which the per-layer launches stagger their walk stay with them: the resident kernel walks in step, so
     // it would neither be as fast there nor give the same bits (the order of a split's tiles is the order of its sums).
@@ -597,7 +596,7 @@ static bool resident_form(const llmi_mha_args& m, const llmi_mha_plan& plan) {
 constexpr int kFewestHeads = 32;
 
 // Whether a KV head of a layer at a time per workgroup (mha_heads.hip) takes this shape and is the faster form.
-static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan, bool resident, HeadsForm* form) {
+static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan, bool resident, int cus, HeadsForm* form) {
     *form = HeadsForm{};
     const llmi_mha_args& m = st.first.mha;
     if (plan.path != LLMI_PATH_SINGLE_PASS && plan.path != LLMI_PATH_SPLIT_FUSED) return false;
@@ -607,7 +606,6 @@ static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan,
     const int waves = plan.group_pad == 8 || plan.waves_per_group == 8 ? 8 : 4;
     if (plan.waves_per_group != waves && !(plan.num_splits == 1 && plan.waves_per_group < waves && tiles <= plan.waves_per_group)) return false;
     const int n_kv = m.kv_dim / m.head_dim;
-    const int cus = compute_units();
     const int64_t heads = (int64_t)st.layer_count * n_kv;
     if (cus <= 0 || heads > INT32_MAX / 64) return false;
     if (heads < kFewestHeads) return false;
@@ -647,8 +645,8 @@ static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan,
 }
 
 // Validates a multi-layer call and decides between the one-launch form (*one_launch = true, plan = layer 0's) and
-// one launch per layer.
-static int plan_stack(const llmi_mha_stack_args* args, llmi_mha_plan* plan, bool* one_launch, bool* heads, HeadsForm* form) {
+// one launch per layer. `cus`: compute units of the device (0: of the present one).
+static int plan_stack(const llmi_mha_stack_args* args, llmi_mha_plan* plan, bool* one_launch, bool* heads, HeadsForm* form, int cus = 0) {
     if (!args) return LLMI_ERR_NULL_POINTER;
     const llmi_mha_append_args& ap = args->first;
     if (!ap.key_new || !ap.value_new || !ap.norm_weight || !ap.sin_cache || !ap.cos_cache) return LLMI_ERR_NULL_POINTER;
@@ -666,8 +664,9 @@ static int plan_stack(const llmi_mha_stack_args* args, llmi_mha_plan* plan, bool
     *one_launch = *heads = false;
     const llmi_mha_args& m = ap.mha;
     if (m.pos_device) return LLMI_OK;
-    const bool resident = resident_form(m, *plan);
-    if (plan_heads(*args, *plan, resident, form) && layers_are_independent(*args)) {
+    if (cus <= 0) cus = compute_units();
+    const bool resident = resident_form(m, *plan, cus);
+    if (plan_heads(*args, *plan, resident, cus, form) && layers_are_independent(*args)) {
         *heads = true;
         return LLMI_OK;
     }
@@ -888,6 +887,20 @@ int32_t llmi_hip_device_split_rule(const llmi_mha_args* args, int32_t append, in
     if (!args || !rule) return LLMI_ERR_NULL_POINTER;
     if (int rc = make_plan(args, &plan, kMaxWaves, append ? 1 : 0)) return rc;
     dyn_split_rule(*args, plan, append != 0, &rule[0], &rule[1], &rule[2]);
+    return LLMI_OK;
+}
+
+int32_t llmi_hip_heads_form(const llmi_mha_stack_args* args, int32_t compute_units, int32_t form[6]) {
+    llmi_mha_plan plan;
+    bool one = false, heads = false;
+    HeadsForm f;
+    if (!form) return LLMI_ERR_NULL_POINTER;
+    for (int i = 0; i < 6; ++i) form[i] = 0;
+    if (int rc = plan_stack(args, &plan, &one, &heads, &f, compute_units)) return rc;
+    if (!heads) return LLMI_OK;
+    const int tiles = std::max(ceil_div(args->first.mha.pos, kTile), 1);
+    const int32_t out[6] = {f.grid, f.parts, f.cut_heads, f.waves, plan.num_splits, heads_splits_at_once(plan.num_splits, ceil_div(tiles, plan.num_splits), f.waves)};
+    std::copy(out, out + 6, form);
     return LLMI_OK;
 }
 

@@ -464,6 +464,38 @@ def test_split_counts_of_a_device_position(append, n_q, n_kv, single, quarter, h
     assert tuple(rule) == (0, 0, 0)
 
 
+def _stack_args(layers, ctx, n_q, n_kv, **over):
+    """Independent layers at made-up addresses, a workspace of the size that llmi_hip_mha_workspace_bytes asks for."""
+    dim, kv_dim, base = n_q * 128, n_kv * 128, 1 << 40
+    s = B.MhaStackArgs()
+    a = good_args(head_num=n_q, kv_mul=n_q // n_kv, kv_dim=kv_dim, pos=ctx, max_seq_len=ctx + 3, kv_layout=B.KV_LAYOUT_HEAD_MAJOR,
+                  workspace_bytes=B.lib().llmi_hip_mha_workspace_bytes(n_q, 128, ctx + 3), **over)
+    a.query, a.key_cache, a.value_cache, a.output, a.workspace = (base * i for i in range(1, 6))
+    s.first.mha = a
+    s.first.key_new, s.first.value_new, s.first.norm_weight, s.first.sin_cache, s.first.cos_cache = (base * i for i in range(6, 11))
+    s.first.eps = 1e-6
+    s.layer_count, s.query_stride, s.output_stride = layers, dim, dim
+    s.key_new_stride, s.value_new_stride, s.norm_weight_stride = kv_dim, kv_dim, 256
+    return s
+
+
+@pytest.mark.parametrize("layers,ctx,n_q,over,form", [  # on 256 compute units: workgroups, parts, cut heads, wavefronts, splits, splits at a time
+    (5, 250, 64, {}, (40, 1, 0, 8, 16, 8)),
+    (5, 257, 64, {}, (40, 1, 0, 8, 16, 4)),
+    (36, 300, 32, {}, (256, 2, 32, 4, 16, 2)),
+    (4, 513, 32, {}, (256, 8, 32, 4, 16, 1)),
+    (35, 432, 64, dict(num_splits=27, force_path=B.PATH_SPLIT_FUSED), (256, 2, 24, 8, 27, 8)),
+    (8, 100, 64, {}, (64, 1, 0, 8, 1, 1)),            # a single pass
+    (3, 250, 64, {}, (0,) * 6),                       # too few heads
+    (16, 2000, 32, {}, (0,) * 6),                     # the stream by layers is the faster one
+    (36, 300, 32, dict(pos_device=0x1000), (0,) * 6),
+])
+def test_layers_a_kv_head_at_a_time_by_size(layers, ctx, n_q, over, form):
+    got = (ctypes.c_int32 * 6)(*[7] * 6)
+    assert B.lib().llmi_hip_heads_form(ctypes.byref(_stack_args(layers, ctx, n_q, 8, **over)), 256, got) == 0
+    assert tuple(got) == form
+
+
 @pytest.mark.parametrize("pos", [100, 200, 250, 700, 2999, 40000])
 def test_workgroups_that_wait_for_each_other_leave_room(pos):
     """A spread merge has a workgroup per query head wait for the other splits of its KV head; a compute unit may hold one of
