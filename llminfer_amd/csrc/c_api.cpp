@@ -609,12 +609,17 @@ static bool plan_heads(const llmi_mha_stack_args& st, const llmi_mha_plan& plan,
     const int64_t heads = (int64_t)st.layer_count * n_kv;
     if (cus <= 0 || heads > INT32_MAX / 64) return false;
     if (heads < kFewestHeads) return false;
-    // What either side takes, in us (fitted to sweeps of 4 to 64 layers, 32 to 20000 positions, groups of 1 to 8; within a tenth
-    // mostly). Here a split, or a round of splits side by side (short ones: within a quarter), costs a workgroup a fixed part (folding, the barrier) and its wavefronts' tiles, all of them share the
-    // memory's rate, and cut heads are handed over at the end: 8 layers at 2048 positions, 2 : 4 : 8 : 16 : 32 splits, 26.9 : 28.8 : 31.8 :
-    // 38.0 : 48.8 (four wavefronts), 27.3 : 28.4 : 31.3 : 38.2 : 62.9 (eight). Both sides near the line, this form : the other one: 36 layers
+    // What either side takes, in us (fitted to sweeps of 4 to 64 layers, 32 to 20000 positions, groups of 1 to 8). Here a split, or a
+    // round of splits side by side, costs a workgroup a fixed part (folding, the barrier) and its wavefronts' tiles, all of them share the
+    // memory's rate, and cut heads are handed over at the end: 8 layers at 2048 positions, none cut, 2 : 4 : 8 : 16 : 32 splits, 26.6 : 27.6 : 30.6 :
+    // 36.1 : 46.4 (four wavefronts), 27.1 : 28.2 : 30.4 : 35.8 : 43.4 (eight, the last two at a time). Over 4 to 36 layers of 16, 32 and 64 Q heads at
+    // 40 to 4000 positions the estimate is 0.90 to 1.31 times what is measured with four wavefronts, the most for few layers of two splits at a time, and 0.73 to
+    // 1.01 with eight, the least with splits side by side, whose folds it leaves out. The form it takes was the faster one everywhere; where it
+    // says no with four wavefronts this form can be ahead by a third: 10 layers of 32 Q heads at 700 16.5 : 24.1, 6 at 1000 12.4 : 16.4, 36
+    // at 1500 56 : 75. Both sides near the line, this form : the other one: 36 layers
     // of 32 Q heads at 4096 96 : 107, 30 at 3000 69 : 75, 24 at 4000 75 : 74, 28 at 2000 50 : 55, 16 at 2000 50 : 33, 10 of 16 Q heads at
-    // 600 16 : 17, 6 of 32 Q heads at 20000 89 : 81; groups of 8 (one launch per layer) 8 at 300 33 : 50, 4 at 6000 26 : 34.
+    // 600 16 : 17, 6 of 32 Q heads at 20000 89 : 81; groups of 8 (one launch per layer) 8 at 300 11 : 44 (16 in a workspace too small for cut heads), 4 at
+    // 6000 26 : 33.
     const double head_bytes = 4.0 * m.pos * m.head_dim, rate = 6.4e6;
     const int most = std::max(ceil_div(tiles, plan.num_splits), 1), at_once = heads_splits_at_once(plan.num_splits, most, waves);
     const int tiles_per_wave = ceil_div(most, waves);

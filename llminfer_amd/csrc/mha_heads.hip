@@ -2,8 +2,8 @@
 // llmi_hip_mha_decode_append_stack's one launch (the first, and how the layers are told to be independent, is in mha_stack.hip).
 //
 // The work is layers x KV heads, and with a dozen layers and more there are about as many of those as compute units: a workgroup
-// takes a KV head of a layer whole. It walks the head's splits one after the other, the tiles of all of them (and of its next
-// head) as one sequence through the LDS rings, and keeps a split's folded row in registers, so that nothing has to be handed
+// takes a KV head of a layer whole. It walks the head's splits in rounds, one after the other or a few short ones side by side, the tiles of all
+// of them (and of its next head) as one sequence through the LDS rings, and keeps a split's folded row in registers, so that nothing has to be handed
 // over: no partial rows in memory, no records, no waits for anybody. The splits, the tiles of a split's wavefronts, the folds and
 // the merge are those of one launch per layer, in the same order: same bits. What bounds it is the K/V stream.
 //
@@ -12,11 +12,12 @@
 // brings them into its registers and merges. Parts are handed out ahead of the whole heads, consecutive workgroups taking the
 // parts of a head, the last part the highest: the only wait (bounded) is for workgroups that were started earlier and wait for nobody.
 //
-// us, this form : the stream by layers (mha_layers_kernel), 32 Q / 8 KV heads: 36 layers at 4096 + 1 positions 96-102 : 108 (6.1 TB/s), at
-// 300 22 : 54, 64 layers at 1000 55 : 109; 28 layers of 16 Q heads at 1000 27 : 45. Against one launch per layer, 64 Q / 8 KV heads:
-// 64 layers at 3000 144 : 476, 36 at 1100 52 : 234, 8 at 300 11 : 50; single passes, 12 layers of 32 Q heads at 150 9 : 55. With one tile
-// per wavefront and round it is the work between tiles that bounds it, 0.75 us per round (0.57 per tile): instructions, one or two
-// wavefronts to a SIMD.
+// us, this form : the stream by layers (mha_layers_kernel), 32 Q / 8 KV heads: 36 layers at 4096 + 1 positions 95 : 107 (6.4 TB/s), at
+// 300 22 : 55, 64 layers at 1000 51 : 105; 28 layers of 16 Q heads at 1000 25 : 43. Against one launch per layer, 64 Q / 8 KV heads:
+// 64 layers at 3000 135 : 413, 36 at 1000 36 : 199, at 1100 52 : 203, 8 at 300 11 : 44; single passes, 12 layers of 32 Q heads at 150 8 : 51.
+// Short lengths are bound by instructions, one or two wavefronts to a SIMD, not by the tiles' way: four wavefronts 0.75 us per round and 0.57 per
+// tile; eight, by the clock in the kernel (23 layers at 384, 64 at 250, 36 at 1000 and at 1100 positions), 0.02 - 0.2 us waiting for a tile, 0.5 - 0.9
+// folding it, 0.5 - 0.8 from there to the barrier, 0.4 - 1.3 at it, 0.5, 0.8 or 1.7 folding two, four or eight splits.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
